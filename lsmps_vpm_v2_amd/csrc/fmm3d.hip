@@ -32,13 +32,12 @@
 //     excluded.
 //
 // Mapping: cells are emitted in depth-first pre-order with a skip pointer
-// (the next cell after the subtree), so a traversal is a loop over one index.
-// One wavefront takes 64 consecutive sorted targets and walks the tree once
-// for all of them: a cell is visited when some lane has to test it, and each
-// lane keeps one bit per level saying whether it opened the cell of that
-// level on the current path (a lane tests a cell only when its bit of the
-// parent's level is set).  Cell records, moments and source particles are
-// wave-uniform loads (scalar cache).
+// (the next cell after the subtree); every non-leaf cell also has a row of its
+// active children, so a wavefront can test many cells at once.  One wavefront
+// takes kGrp consecutive sorted targets (wave-uniform coordinates) and puts
+// the tree in its lanes: a lane tests one cell against every target, holds one
+// far cell's coefficients or one near source, and keeps the kGrp partial
+// velocities, which are summed over the lanes once at the end.
 //
 // This file is compiled without FMA contraction: cell centres and the
 // opening test round as the reference's; the arithmetic of the sums opts
@@ -52,9 +51,9 @@ namespace vpm {
 namespace {
 
 constexpr int kHalf = kFmm3Depth / 2;  // levels per key word
-constexpr unsigned kF3NonFinite = 1u, kF3Deeper = 2u, kF3Depth = 4u, kF3Degenerate = 8u;
+constexpr unsigned kF3NonFinite = 1u, kF3Deeper = 2u, kF3Depth = 4u, kF3Degenerate = 8u,
+                   kF3OddStrength = 16u;  // a strength that is not finite
 constexpr int kMomStride = 32;
-constexpr int kEvalBlock = 256;
 
 struct __align__(16) Par3 {
     double x, y, z, ax, ay, az, act, pad;
@@ -297,7 +296,7 @@ __global__ void __launch_bounds__(256)
               const double *__restrict__ s, const double *__restrict__ wx,
               const double *__restrict__ wy, const double *__restrict__ wz,
               const uint8_t *__restrict__ active, int n, Par3 *__restrict__ P,
-              uint64_t *__restrict__ key, uint8_t *__restrict__ act8) {
+              uint64_t *__restrict__ key, uint8_t *__restrict__ act8, Fmm3Hdr *__restrict__ h) {
     const int j = blockIdx.x * 256 + threadIdx.x;
     if (j >= n) return;
     const uint32_t i = perm[j];
@@ -320,6 +319,9 @@ __global__ void __launch_bounds__(256)
     }
     r.act = a ? 1.0 : 0.0;
     r.pad = 0.0;
+    const uint64_t odd = __ballot(!(isfinite(r.ax) && isfinite(r.ay) && isfinite(r.az)));
+    if (odd && (threadIdx.x & (kWave - 1)) == (uint32_t)(__ffsll((unsigned long long)odd) - 1))
+        atomicOr(&h->flags, kF3OddStrength);
     P[j] = r;
     act8[j] = a ? 1 : 0;
 }
@@ -579,15 +581,88 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// One thread per leaf of level >= 2 (the level-1 cells are never tested):
-// P2M of its active particles.
+// A far cell's term as the evaluation uses it.  With phi = 1 / r the M2P
+// multipliers of M2P_mul_calc are -(derivatives of phi), and phi is harmonic:
+// phi_xx + phi_yy + phi_zz = 0 and likewise for its derivatives.  So the six
+// second-order multipliers of each velocity component need only the seven
+// mixed third derivatives T_xxy, T_xxz, T_xyy, T_yyz, T_xzz, T_yzz, T_xyz, and
+// the cross product of the 30 moments with the 30 multipliers (60 FMAs)
+// becomes 42 FMAs with 27 combinations of the moments, formed once per cell.
+// f[0..2] order 0, f[3..11] order 1, f[12..26] order 2, f[27..29] the centre;
+// m: component-major moments (x: m[0..9], y: m[10..19], z: m[20..29]).
+constexpr int kFarStride = 32;
+__device__ __forceinline__ void far_row(const double *m, double cx, double cy, double cz,
+                                        double *f) {
+    const double *X = m, *Y = m + 10, *Z = m + 20;
+    f[0] = X[0];
+    f[1] = Y[0];
+    f[2] = Z[0];
+    f[3] = X[2];
+    f[4] = X[3];
+    f[5] = Y[1];
+    f[6] = Y[3];
+    f[7] = Z[1];
+    f[8] = Z[2];
+    f[9] = Y[2] - Z[3];
+    f[10] = Z[3] - X[1];
+    f[11] = X[1] - Y[2];
+    f[12] = Y[4] - Y[6];
+    f[13] = Y[5] - Y[6] - Z[8];
+    f[14] = Y[7] - Z[9];
+    f[15] = Y[8] - Z[6] + Z[5];
+    f[16] = Y[9];
+    f[17] = Z[5] - Z[4];
+    f[18] = Z[7];
+    f[19] = Z[6] - Z[4] - X[9];
+    f[20] = Z[8] - X[7];
+    f[21] = Z[9] - X[4] + X[6];
+    f[22] = X[6] - X[5];
+    f[23] = X[8];
+    f[24] = X[4] - X[5] - Y[7];
+    f[25] = X[7] + Y[4] - Y[5];
+    f[26] = X[9] - Y[8];
+    f[27] = cx;
+    f[28] = cy;
+    f[29] = cz;
+}
+
+// One thread per cell.  A leaf of level >= 2 (the level-1 cells are never
+// tested): P2M of its active particles, as moments (for the shifts of its
+// ancestors) and as its far row.  A non-leaf: the row of its active children
+// (-1 beyond the last); thread ncell writes the root's row, the non-leaf
+// level-1 cells, which the walk opens untested.
+constexpr int kKids = 8;
 __global__ void __launch_bounds__(256)
     k3_p2m(const Cell3 *__restrict__ cells, int ncell, const Src3 *__restrict__ S,
-           double *__restrict__ mom) {
+           double *__restrict__ mom, double *__restrict__ far, int *__restrict__ kids) {
 #pragma clang fp contract(fast)
     const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= ncell) return;
-    const Cell3 C = cells[c];
+    if (c > ncell) return;
+    const bool root = c == ncell;
+    Cell3 C;
+    if (!root) C = cells[c];
+    if (root || !(C.meta & 0x100u)) {
+        int4 *row = reinterpret_cast<int4 *>(kids + (size_t)c * kKids);
+        int k[kKids], m = 0;
+#pragma unroll
+        for (int q = 0; q < kKids; ++q) k[q] = -1;
+        int d = root ? 0 : c + 1;
+        const int end = root ? ncell : (int)C.skip;
+#pragma unroll
+        for (int q = 0; q < kKids; ++q) {  // at most eight children
+            if (d >= end) break;
+            const uint32_t meta = cells[d].meta, skip = cells[d].skip;
+            const bool keep = root ? !(meta & 0x100u) : (meta & 0x200u) != 0;
+#pragma unroll
+            for (int z = 0; z < kKids; ++z)
+                if (keep && z == m) k[z] = d;
+            m += keep ? 1 : 0;
+            d = (int)skip;
+        }
+        row[0] = make_int4(k[0], k[1], k[2], k[3]);
+        row[1] = make_int4(k[4], k[5], k[6], k[7]);
+        return;
+    }
     const int L = (int)(C.meta & 0xffu);
     if (L < 2 || (C.meta & 0x300u) != 0x300u) return;
     double m[30];
@@ -608,12 +683,18 @@ __global__ void __launch_bounds__(256)
     double *o = mom + (size_t)c * kMomStride;
 #pragma unroll
     for (int k = 0; k < 30; k += 2) *reinterpret_cast<double2 *>(o + k) = make_double2(m[k], m[k + 1]);
+    double f[30];
+    far_row(m, C.cx, C.cy, C.cz, f);
+    o = far + (size_t)c * kFarStride;
+#pragma unroll
+    for (int k = 0; k < 30; k += 2) *reinterpret_cast<double2 *>(o + k) = make_double2(f[k], f[k + 1]);
 }
 
 // One wavefront per non-leaf cell of level >= 2: its leaves' moments shifted
 // to its centre (the order-2 shift of M2M_calc, applied from each leaf).
 __global__ void __launch_bounds__(256)
-    k3_m2m(const Cell3 *__restrict__ cells, int ncell, double *__restrict__ mom) {
+    k3_m2m(const Cell3 *__restrict__ cells, int ncell, const double *__restrict__ mom,
+           double *__restrict__ far) {
 #pragma clang fp contract(fast)
     const int lane = threadIdx.x & (kWave - 1);
     const int c = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + threadIdx.x / kWave));
@@ -648,19 +729,19 @@ __global__ void __launch_bounds__(256)
     }
 #pragma unroll
     for (int k = 0; k < 30; ++k) m[k] = wave_sum(m[k]);
+    double f[30];
+    far_row(m, C.cx, C.cy, C.cz, f);
     if (lane < 30) {
-        double v = m[0];
+        double v = f[0];
 #pragma unroll
-        for (int k = 1; k < 30; ++k) v = lane == k ? m[k] : v;
-        mom[(size_t)c * kMomStride + lane] = v;
+        for (int k = 1; k < 30; ++k) v = lane == k ? f[k] : v;
+        far[(size_t)c * kFarStride + lane] = v;
     }
 }
 
 // -------------------------------------------------------------------------
 // evaluation
 // -------------------------------------------------------------------------
-constexpr int kEvalWaves = kEvalBlock / kWave;
-
 // Lanes of one wavefront read what other lanes of it wrote to LDS.
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -682,44 +763,72 @@ __device__ __forceinline__ double rsqrt_pos(double x) {
     return fma(y0 * t, fma(t, 0.375, 0.5), y0);
 }
 
-// The far-cell term: the moments against the Taylor coefficients of
-// r / |r|^3 at the target (M2P_mul_calc), crossed into the velocity.
-__device__ __forceinline__ void m2p_term(const double *__restrict__ M, double dx, double dy,
-                                         double dz, double R2, double &vu, double &vv,
+// x where bit t of m is set, else +0 (whatever x): a bit mask, not a select,
+// which the compiler would turn into a branch around what forms x.
+__device__ __forceinline__ double masked(double x, uint32_t m, int t) {
+    const uint32_t k = (uint32_t)((int32_t)(m << (31 - t)) >> 31);
+    return __hiloint2double((int)((uint32_t)__double2hiint(x) & k),
+                            (int)((uint32_t)__double2loint(x) & k));
+}
+
+// The far-cell term (far_row) at a target displaced by (dx, dy, dz) from the
+// centre, added to the velocity where bit t of m is set: about 90 instructions.
+__device__ __forceinline__ void far_term(const double (&f)[27], double dx, double dy, double dz,
+                                         uint32_t m, int t, double &vu, double &vv,
                                          double &vw) {
 #pragma clang fp contract(fast)
-    const double ir = rsqrt_pos(R2);
-    const double i2 = ir * ir, i3 = i2 * ir, i5 = i3 * i2, i7 = i5 * i2;
-    const double a = 3.0 * i5, b = 15.0 * i7;
-    const double xx = dx * dx, yy = dy * dy, zz = dz * dz;
-    const double xy = dx * dy, yz = dy * dz, xz = dx * dz, bxyz = b * xy * dz;
-    const double mx[10] = {dx * i3,          i3 - a * xx,          -a * xy,
-                           -a * xz,          (b * xx - 3.0 * a) * dx, (b * yy - a) * dx,
-                           (b * zz - a) * dx, (b * xx - a) * dy,   bxyz,
-                           (b * xx - a) * dz};
-    const double my[10] = {dy * i3,          -a * xy,           i3 - a * yy,
-                           -a * yz,          (b * xx - a) * dy, (b * yy - 3.0 * a) * dy,
-                           (b * zz - a) * dy, (b * yy - a) * dx, (b * yy - a) * dz,
-                           bxyz};
-    const double mz[10] = {dz * i3,           -a * xz,           -a * yz,
-                           i3 - a * zz,       (b * xx - a) * dz, (b * yy - a) * dz,
-                           (b * zz - 3.0 * a) * dz, bxyz,        (b * zz - a) * dy,
-                           (b * zz - a) * dx};
-    // each cross term accumulated on its own (two FMAs per term)
-    double su = 0.0, sv = 0.0, sw = 0.0;
-#pragma unroll
-    for (int k = 0; k < 10; ++k) {
-        const double Vx = M[k], Vy = M[10 + k], Vz = M[20 + k];
-        su = fma(Vy, mz[k], su);
-        su = fma(-Vz, my[k], su);
-        sv = fma(Vz, mx[k], sv);
-        sv = fma(-Vx, mz[k], sv);
-        sw = fma(Vx, my[k], sw);
-        sw = fma(-Vy, mx[k], sw);
-    }
-    vu += su;
-    vv += sv;
-    vw += sw;
+    const double ir = masked(rsqrt_pos(dx * dx + dy * dy + dz * dz), m, t);
+    const double i2 = ir * ir, i3 = i2 * ir, a = (3.0 * i2) * i3, c = 5.0 * i2;
+    const double gx = dx * i3, gy = dy * i3, gz = dz * i3;
+    const double ax = a * dx, ay = a * dy, az = a * dz;
+    const double uxy = ax * dy, uxz = ax * dz, uyz = ay * dz;
+    const double pxx = ax * dx, pyy = ay * dy, pzz = az * dz;
+    const double sx = i3 - pxx, sy = i3 - pyy, sz = i3 - pzz;
+    const double qx = fma(c, pxx, -a), qy = fma(c, pyy, -a), qz = fma(c, pzz, -a);
+    const double txxy = qx * dy, txxz = qx * dz, txyy = qy * dx, tyyz = qy * dz, txzz = qz * dx,
+                 tyzz = qz * dy, txyz = c * uxy * dz;
+    vu = fma(f[1], gz, vu);
+    vu = fma(-f[2], gy, vu);
+    vu = fma(f[6], sz, vu);
+    vu = fma(-f[8], sy, vu);
+    vu = fma(-f[5], uxz, vu);
+    vu = fma(-f[9], uyz, vu);
+    vu = fma(f[7], uxy, vu);
+    vu = fma(f[12], txxz, vu);
+    vu = fma(f[13], tyyz, vu);
+    vu = fma(f[14], txyz, vu);
+    vu = fma(f[15], tyzz, vu);
+    vu = fma(f[16], txzz, vu);
+    vu = fma(f[17], txxy, vu);
+    vu = fma(-f[18], txyy, vu);
+    vv = fma(f[2], gx, vv);
+    vv = fma(-f[0], gz, vv);
+    vv = fma(f[7], sx, vv);
+    vv = fma(-f[4], sz, vv);
+    vv = fma(-f[10], uxz, vv);
+    vv = fma(-f[8], uxy, vv);
+    vv = fma(f[3], uyz, vv);
+    vv = fma(f[17], txyy, vv);
+    vv = fma(f[19], txzz, vv);
+    vv = fma(f[18], txxy, vv);
+    vv = fma(f[20], txyz, vv);
+    vv = fma(f[21], txxz, vv);
+    vv = fma(f[22], tyyz, vv);
+    vv = fma(-f[23], tyzz, vv);
+    vw = fma(f[0], gy, vw);
+    vw = fma(-f[1], gx, vw);
+    vw = fma(f[3], sy, vw);
+    vw = fma(-f[5], sx, vw);
+    vw = fma(-f[11], uxy, vw);
+    vw = fma(-f[4], uyz, vw);
+    vw = fma(f[6], uxz, vw);
+    vw = fma(f[24], txxy, vw);
+    vw = fma(f[22], tyzz, vw);
+    vw = fma(f[25], txyy, vw);
+    vw = fma(f[12], txzz, vw);
+    vw = fma(f[23], tyyz, vw);
+    vw = fma(f[26], txyz, vw);
+    vw = fma(-f[16], txxz, vw);
 }
 
 // Workgroups are dispatched to the 8 XCDs in turn (workgroup b to XCD
@@ -734,128 +843,357 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
     return (b % kXcds) * per + b / kXcds;
 }
 
-// The direct sum of a near leaf's sources [ab, ae) for the lanes with near
-// set, the sources read as wave-uniform loads (scalar cache), four per
-// batch; SELF drops the pair of a target with itself.
-template <bool SELF>
-__device__ __forceinline__ void direct_pairs(const Src3 *__restrict__ S, uint32_t ab, uint32_t ae,
-                                             double xp, double yp, double zp, double di,
-                                             bool near, double &vu, double &vv, double &vw) {
-#pragma clang fp contract(fast)
-    if (!near) return;
-#pragma unroll 4
-    for (uint32_t j = ab; j < ae; ++j) {
-        const Src3 q = S[j];
-        const double ex = xp - q.x, ey = yp - q.y, ez = zp - q.z;
-        const double r2 = ex * ex + ey * ey + ez * ez;
-        const double ir = rsqrt_pos(r2);
-        const double i3 = (!SELF || q.idx != di) ? ir * ir * ir : 0.0;
-        vu += (q.ay * ez - q.az * ey) * i3;
-        vv += (q.az * ex - q.ax * ez) * i3;
-        vw += (q.ax * ey - q.ay * ex) * i3;
+// The evaluation: one wavefront per kGrp consecutive sorted targets.
+//
+// The walk keeps a stack of opened cells, each with the mask of the targets
+// that opened it; a step pops up to 8 of them and gives each lane one child to
+// test against every target of the mask.  Far cells and near leaves go to
+// queues in LDS (with their target masks); 64 queued far cells, or the sources
+// of 64 queued leaves, are then evaluated with a cell or a source per lane and
+// the targets in turn.  A lane's far cell or source is loaded once for kGrp
+// terms (the cells' rows through LDS: coalesced 256-byte rows in, a row per
+// lane out), and every wavefront step is 64 terms, of which the mask keeps
+// those whose target takes this cell.
+//
+// The kernel is bound by vector-ALU issue in FP64 (0.7 of the cycles), so what
+// counts is the share of a step's 64 lane slots that hold a wanted term.  One
+// lane per target, one cell or source at a time for 64 targets, used 0.53
+// (far) and 0.30 (near) of them: the far cells and near leaves of 64
+// consecutive targets are 1.9 and 3.3 times those of one.  With 8 targets it
+// is 0.74 and 0.58, and the far term takes 93 instructions instead of 150
+// (far_row): 5.91 -> 3.6 ms on the 780k-particle vortex ring, 0.92 -> 0.22 ms
+// at 60k, where 64 targets per wavefront also left most of the chip idle.
+// kGrp 8 holds the 24 partial velocities, a cell's 27 coefficients and the
+// term's temporaries in 168 registers (3 wavefronts per SIMD); one wavefront
+// per workgroup lets LDS hold as many (2 and 4 per workgroup: 1 % and 7 %
+// slower at 780k).
+//
+// The stack holds at most 64 cells of a level: a step pops from the deepest
+// level down, so whatever stays is no deeper than what was popped, and the
+// entries of a level all come from one step.
+constexpr int kGrp = 8;
+constexpr int kEvalWaves = 1;
+constexpr int kFarRow = 18;     // LDS stride of a staged half row, in doubles (conflict-free)
+constexpr int kQueue = 128;     // far cells / near leaves queued (64 evaluated at a time)
+constexpr int kTakeMax = 16;    // sources a lane emits per round from its leaf
+constexpr int kSrcQueue = kWave * kTakeMax + kWave;
+
+struct EvalLds {
+    union {
+        double row[kWave * kFarRow];
+        struct {
+            uint32_t idx[kSrcQueue];
+            uint8_t m[kSrcQueue];
+        } s;
+    };
+    uint32_t fq[kQueue];
+    uint32_t nb[kQueue], ne[kQueue];
+    uint32_t left[kWave];  // sources carried to the next leaf batch
+    uint8_t fm[kQueue], nm[kQueue], leftm[kWave];
+};
+
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+struct Acc3 {
+    double u[kGrp], v[kGrp], w[kGrp];
+};
+
+// The far cells fq[base .. base + cnt) (cnt <= 64).
+__device__ __forceinline__ void eval_far(EvalLds &l, int base, int cnt, int lane,
+                                         const double *__restrict__ far, const double (&xt)[kGrp],
+                                         const double (&yt)[kGrp], const double (&zt)[kGrp],
+                                         Acc3 &acc) {
+    const uint32_t m = lane < cnt ? (uint32_t)l.fm[base + lane] : 0u;
+    // rows of 32 doubles: 8 lanes load half a row (every load in flight before
+    // the first is stored), and the halves pass through LDS in turn
+    v2d ta[8], tb[8], fa[8], fb[7];
+#pragma unroll
+    for (int it = 0; it < 8; ++it) {
+        const size_t c = l.fq[base + min(it * 8 + (lane >> 3), cnt - 1)];
+        const v2d *row = reinterpret_cast<const v2d *>(far + c * kFarStride) + (lane & 7);
+        ta[it] = row[0];
+        tb[it] = row[8];
+    }
+    v2d *in = reinterpret_cast<v2d *>(&l.row[(lane >> 3) * kFarRow]) + (lane & 7);
+    const v2d *out = reinterpret_cast<const v2d *>(&l.row[lane * kFarRow]);
+#pragma unroll
+    for (int it = 0; it < 8; ++it) in[it * 4 * kFarRow] = ta[it];
+    wave_sync();
+#pragma unroll
+    for (int k = 0; k < 8; ++k) fa[k] = out[k];
+    wave_sync();
+#pragma unroll
+    for (int it = 0; it < 8; ++it) in[it * 4 * kFarRow] = tb[it];
+    wave_sync();
+#pragma unroll
+    for (int k = 0; k < 7; ++k) fb[k] = out[k];
+    wave_sync();
+    const double fc[27] = {fa[0].x, fa[0].y, fa[1].x, fa[1].y, fa[2].x, fa[2].y, fa[3].x,
+                           fa[3].y, fa[4].x, fa[4].y, fa[5].x, fa[5].y, fa[6].x, fa[6].y,
+                           fa[7].x, fa[7].y, fb[0].x, fb[0].y, fb[1].x, fb[1].y, fb[2].x,
+                           fb[2].y, fb[3].x, fb[3].y, fb[4].x, fb[4].y, fb[5].x};
+    const double cx = fb[5].y, cy = fb[6].x, cz = fb[6].y;
+#pragma unroll
+    for (int t = 0; t < kGrp; ++t) {
+        far_term(fc, xt[t] - cx, yt[t] - cy, zt[t] - cz, m, t, acc.u[t], acc.v[t], acc.w[t]);
+        __builtin_amdgcn_sched_barrier(0);  // one target's temporaries at a time
     }
 }
 
-// A near leaf's active sources are read as wave-uniform loads (scalar
-// cache), four per batch.
-__global__ void __launch_bounds__(kEvalBlock)
-    k3_eval(const Cell3 *__restrict__ cells, int ncell, const double *__restrict__ mom,
-            const Par3 *__restrict__ P, const Src3 *__restrict__ S,
-            const uint32_t *__restrict__ perm, int n, double u_inf, double v_inf, double w_inf,
-            double *__restrict__ u, double *__restrict__ v, double *__restrict__ w,
-            int src_all, unsigned long long *__restrict__ wstat) {
+// The pairs of the lane's source q with the targets of m.  A masked pair is
+// multiplied by zero; with STRICT its strength is masked too, for fields with
+// a strength that is not finite.
+template <bool STRICT>
+__device__ __forceinline__ void near_terms(const Src3 &q, uint32_t m, const double (&xt)[kGrp],
+                                           const double (&yt)[kGrp], const double (&zt)[kGrp],
+                                           Acc3 &acc) {
+#pragma clang fp contract(fast)
+#pragma unroll
+    for (int t = 0; t < kGrp; ++t) {
+        const double ex = xt[t] - q.x, ey = yt[t] - q.y, ez = zt[t] - q.z;
+        const double ir = masked(rsqrt_pos(ex * ex + ey * ey + ez * ez), m, t);
+        const double i3 = ir * ir * ir;
+        const double ax = STRICT ? masked(q.ax, m, t) : q.ax, ay = STRICT ? masked(q.ay, m, t) : q.ay,
+                     az = STRICT ? masked(q.az, m, t) : q.az;
+        acc.u[t] += (ay * ez - az * ey) * i3;
+        acc.v[t] += (az * ex - ax * ez) * i3;
+        acc.w[t] += (ax * ey - ay * ex) * i3;
+        if (t & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// The sources s.idx[base .. base + cnt) (cnt <= 64); i0: the first target's
+// tree index (a target is not its own source).
+template <bool STRICT>
+__device__ __forceinline__ void eval_near(EvalLds &l, int base, int cnt, int lane, int i0,
+                                          const Src3 *__restrict__ S, const double (&xt)[kGrp],
+                                          const double (&yt)[kGrp], const double (&zt)[kGrp],
+                                          Acc3 &acc) {
+#pragma clang fp contract(fast)
+    uint32_t m = lane < cnt ? (uint32_t)l.s.m[base + lane] : 0u;
+    const Src3 q = S[l.s.idx[base + min(lane, cnt - 1)]];
+    const double self = q.idx - (double)i0;
+    if (self >= 0.0 && self < (double)kGrp) m &= ~(1u << (int)self);
+    near_terms<STRICT>(q, m, xt, yt, zt, acc);
+}
+
+// The sources of the leaves [nb, ne)[base .. base + cnt): each lane lists its
+// leaf's sources, kTakeMax a round, at the offsets of a wave scan; whole
+// batches of 64 are evaluated, the rest is carried in left / leftm (with last,
+// evaluated too).
+template <bool STRICT>
+__device__ __forceinline__ void eval_leaves(EvalLds &l, int base, int cnt, int lane, int i0,
+                                            const Src3 *__restrict__ S,
+                                            const double (&xt)[kGrp], const double (&yt)[kGrp],
+                                            const double (&zt)[kGrp], Acc3 &acc, bool last,
+                                            int &nleft, uint32_t &wpair) {
+    uint32_t b = 0, rem = 0;
+    uint8_t m = 0;
+    if (lane < cnt) {
+        b = l.nb[base + lane];
+        rem = l.ne[base + lane] - b;
+        m = l.nm[base + lane];
+    }
+    bool more;
+    do {
+        const uint32_t take = min(rem, (uint32_t)kTakeMax);
+        uint32_t inc = take, most = take;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const uint32_t y = __shfl_up(inc, o, kWave);
+            if (lane >= o) inc += y;
+            most = max(most, (uint32_t)__shfl_xor((int)most, o, kWave));
+        }
+        int total = __builtin_amdgcn_readlane((int)inc, kWave - 1) + nleft;
+        most = (uint32_t)__builtin_amdgcn_readfirstlane((int)most);
+        const uint32_t pos = (uint32_t)nleft + inc - take;
+        if (lane < nleft) {
+            l.s.idx[lane] = l.left[lane];
+            l.s.m[lane] = l.leftm[lane];
+        }
+        for (uint32_t k = 0; k < most; ++k)
+            if (k < take) {
+                l.s.idx[pos + k] = b + k;
+                l.s.m[pos + k] = m;
+            }
+        b += take;
+        rem -= take;
+        wave_sync();
+        more = __ballot(rem > 0) != 0;
+        while (total >= kWave || (last && !more && total > 0)) {
+            const int nb = min(total, kWave);
+            total -= nb;
+            eval_near<STRICT>(l, total, nb, lane, i0, S, xt, yt, zt, acc);
+            wpair += kGrp;
+        }
+        if (lane < total) {
+            l.left[lane] = l.s.idx[lane];
+            l.leftm[lane] = l.s.m[lane];
+        }
+        nleft = total;
+        wave_sync();
+    } while (more);
+}
+
+// STRICT for fields with a strength that is not finite: such a source may reach
+// only the targets that take it (inactive particles of type 2 are summed by
+// near targets alone).
+template <bool STRICT>
+__global__ void __launch_bounds__(kEvalWaves *kWave) __attribute__((amdgpu_waves_per_eu(3, 3)))
+    k3_eval(const Cell3 *__restrict__ cells, int ncell, const int *__restrict__ kids,
+            const double *__restrict__ far, const Par3 *__restrict__ P,
+            const Src3 *__restrict__ S, const uint32_t *__restrict__ perm, int n, int stk_cap,
+            double u_inf, double v_inf, double w_inf, double *__restrict__ u,
+            double *__restrict__ v, double *__restrict__ w, int src_all,
+            unsigned long long *__restrict__ wstat) {
+    __shared__ EvalLds lds[kEvalWaves];
+    extern __shared__ uint32_t stk_mem[];  // per wavefront: stk_cap cells, then stk_cap masks
     const int lane = threadIdx.x & (kWave - 1);
-    const int wv = threadIdx.x / kWave;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
     const int wave = __builtin_amdgcn_readfirstlane(blk * kEvalWaves + wv);
-    const int i = wave * kWave + lane;
-    if (wave * kWave >= n) return;
-    const bool valid = i < n;
-    double xp = 0.0, yp = 0.0, zp = 0.0;
-    bool my_act = false;
-    if (valid) {
-        xp = P[i].x;
-        yp = P[i].y;
-        zp = P[i].z;
-        my_act = P[i].act != 0.0;
+    const int i0 = wave * kGrp;
+    if (i0 >= n) return;
+    EvalLds &l = lds[wv];
+    uint32_t *stk = stk_mem + (size_t)wv * (stk_cap + stk_cap / 4);
+    uint8_t *stkm = reinterpret_cast<uint8_t *>(stk + stk_cap);
+    const int nt = min(kGrp, n - i0);
+    const uint32_t all = (1u << nt) - 1u;
+    double xt[kGrp], yt[kGrp], zt[kGrp];
+    uint32_t act = 0;  // targets that are sources too
+#pragma unroll
+    for (int t = 0; t < kGrp; ++t) {
+        const Par3 &q = P[i0 + min(t, nt - 1)];
+        xt[t] = q.x;
+        yt[t] = q.y;
+        zt[t] = q.z;
+        act |= (src_all || q.act != 0.0) ? 1u << t : 0u;
     }
-    const double di = (double)i;
-    double vu = 0.0, vv = 0.0, vw = 0.0;
+    Acc3 acc;
+#pragma unroll
+    for (int t = 0; t < kGrp; ++t) acc.u[t] = acc.v[t] = acc.w[t] = 0.0;
     uint32_t npair = 0, nfar = 0;
-    uint32_t wfar = 0, wpair = 0;  // wave-level steps (uniform)
-    uint32_t open = 0;  // bit L: this lane opened the level-L cell of the current path
-    int c = 0;
-    while (c < ncell) {
-        const Cell3 C = cells[c];
-        const int L = (int)(C.meta & 0xffu);
-        if (L == 1) {
-            // level-1 cells are always opened and never tested; a level-1
-            // leaf is passed over
-            if (C.meta & 0x100u) {
-                c = (int)C.skip;
-            } else {
-                open = valid ? 2u : 0u;
-                c = c + 1;
-            }
-            continue;
+    uint32_t wfar = 0, wpair = 0;  // wavefront steps (uniform)
+    const uint64_t below = lane ? ~0ull >> (kWave - lane) : 0ull;
+    // the non-leaf level-1 cells are opened untested
+    int sp, nf = 0, nn = 0, nleft = 0;
+    {
+        const int c = lane < kKids ? kids[(size_t)ncell * kKids + lane] : -1;
+        const uint64_t b = __ballot(c >= 0);
+        if (c >= 0) {
+            stk[__popcll(b & below)] = (uint32_t)c;
+            stkm[__popcll(b & below)] = (uint8_t)all;
         }
-        if (!(C.meta & 0x200u)) {
-            c = (int)C.skip;
-            continue;
-        }
-        const bool test = (open >> (L - 1)) & 1u;
-        const double dx = xp - C.cx, dy = yp - C.cy, dz = zp - C.cz;
-        const double R2 = r2_exact(dx, dy, dz);
-        const bool far = test && R2 > C.rc2;
-        const bool near = test && !(R2 > C.rc2);
-        if (__ballot(far)) {
-            ++wfar;
-            if (far) {
-                m2p_term(mom + (size_t)c * kMomStride, dx, dy, dz, R2, vu, vv, vw);
-                ++nfar;
-            }
-        }
-        const bool any_near = __ballot(near) != 0;
-        if (C.meta & 0x100u) {
-            if (any_near) {
-                const uint32_t ab = C.abegin, ae = C.aend;
-                wpair += ae - ab;
-                // the target itself is a source of its own leaf (when active,
-                // unless every particle is a source); only a leaf holding some
-                // lane's own particle needs the self test
-                const bool mine = (uint32_t)i >= C.begin && (uint32_t)i < C.end;
-                if (__ballot(near && mine))
-                    direct_pairs<true>(S, ab, ae, xp, yp, zp, di, near, vu, vv, vw);
-                else
-                    direct_pairs<false>(S, ab, ae, xp, yp, zp, di, near, vu, vv, vw);
-                if (near) npair += ae - ab - ((src_all || my_act) && mine ? 1u : 0u);
-            }
-            c = (int)C.skip;
-        } else {
-            open = near ? (open | (1u << L)) : (open & ~(1u << L));
-            c = any_near ? c + 1 : (int)C.skip;
-        }
+        sp = __popcll(b);
+        wave_sync();
     }
-    if (valid) {
-        const uint32_t o = perm[i];
-        u[o] = vu + u_inf;
-        v[o] = vv + v_inf;
-        w[o] = vw + w_inf;
+    for (bool done = false; !done;) {
+        if (sp > 0) {
+            const int np = min(sp, kWave / kKids);
+            sp -= np;
+            int c = -1;
+            uint32_t pm = 0;
+            if ((lane >> 3) < np) {
+                pm = stkm[sp + (lane >> 3)];
+                c = kids[(size_t)stk[sp + (lane >> 3)] * kKids + (lane & 7)];
+            }
+            const bool live = c >= 0;
+            Cell3 C{};
+            if (live) C = cells[c];
+            uint32_t fb = 0;
+#pragma unroll
+            for (int t = 0; t < kGrp; ++t)
+                fb |= r2_exact(xt[t] - C.cx, yt[t] - C.cy, zt[t] - C.cz) > C.rc2 ? 1u << t : 0u;
+            const uint32_t fm = live ? fb & pm : 0u, nm = live ? ~fb & pm : 0u;
+            const bool leaf = (C.meta & 0x100u) != 0;
+            const uint64_t bf = __ballot(fm != 0), bl = __ballot(nm != 0 && leaf),
+                           bo = __ballot(nm != 0 && !leaf);
+            wave_sync();  // the popped entries have been read
+            if (fm) {
+                const int p = nf + __popcll(bf & below);
+                l.fq[p] = (uint32_t)c;
+                l.fm[p] = (uint8_t)fm;
+                nfar += __popc(fm);
+            }
+            if (nm && leaf) {
+                const int p = nn + __popcll(bl & below);
+                l.nb[p] = C.abegin;
+                l.ne[p] = C.aend;
+                l.nm[p] = (uint8_t)nm;
+                // targets in this leaf that are sources: their own pair is left out
+                const int lo = max((int)C.begin - i0, 0), hi = min((int)C.end - i0, kGrp);
+                const uint32_t own = hi > lo ? ((1u << hi) - 1u) & ~((1u << lo) - 1u) : 0u;
+                npair += (uint32_t)__popc(nm) * (C.aend - C.abegin) - (uint32_t)__popc(nm & own & act);
+            }
+            if (nm && !leaf) {
+                const int p = sp + __popcll(bo & below);
+                stk[p] = (uint32_t)c;
+                stkm[p] = (uint8_t)nm;
+            }
+            nf += __popcll(bf);
+            nn += __popcll(bl);
+            sp += __popcll(bo);
+            wave_sync();
+        }
+        done = sp == 0;
+        if (nf >= kWave || (done && nf > 0)) {
+            const int cnt = min(nf, kWave);
+            nf -= cnt;
+            eval_far(l, nf, cnt, lane, far, xt, yt, zt, acc);
+            wfar += kGrp;
+        }
+        done = done && nf == 0;
+        if (nn >= kWave || (done && nn + nleft > 0)) {
+            const int cnt = min(nn, kWave);
+            nn -= cnt;
+            eval_leaves<STRICT>(l, nn, cnt, lane, i0, S, xt, yt, zt, acc, done && nn == 0, nleft,
+                                wpair);
+        }
+        done = done && nn == 0;
+    }
+    // sums over the lanes: three halving exchanges leave one target per lane
+    // (bit k of its index = bit 5 - k of the lane), then the remaining bits
+    static_assert(kGrp == 8, "three halving exchanges");
+    double r[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        double a[kGrp];
+#pragma unroll
+        for (int t = 0; t < kGrp; ++t) a[t] = q == 0 ? acc.u[t] : q == 1 ? acc.v[t] : acc.w[t];
+#pragma unroll
+        for (int h = kGrp / 2, x = kWave / 2; h >= 1; h /= 2, x /= 2) {
+            const bool up = (lane & x) != 0;
+#pragma unroll
+            for (int t = 0; t < h; ++t) {
+                const double keep = up ? a[t + h] : a[t], send = up ? a[t] : a[t + h];
+                a[t] = keep + __shfl_xor(send, x, kWave);
+            }
+        }
+        r[q] = a[0];
+#pragma unroll
+        for (int x = kWave / (2 * kGrp); x >= 1; x /= 2) r[q] += __shfl_xor(r[q], x, kWave);
+    }
+    const int t = lane / kGrp;
+    if (lane % kGrp == 0 && t < nt) {
+        const uint32_t o = perm[i0 + t];
+        u[o] = r[0] + u_inf;
+        v[o] = r[1] + v_inf;
+        w[o] = r[2] + w_inf;
     }
     // work counts per wavefront (summed by k3_eval_stats; same-address
     // atomics from every wavefront would serialise)
-    unsigned long long sp = npair, sf = nfar;
+    unsigned long long sn = npair, sf = nfar;
     for (int m = 1; m < kWave; m <<= 1) {
-        sp += __shfl_xor(sp, m, kWave);
+        sn += __shfl_xor(sn, m, kWave);
         sf += __shfl_xor(sf, m, kWave);
     }
     if (lane == 0) {
-        ulonglong4 r;
-        r.x = sp;
-        r.y = sf;
-        r.z = wpair;
-        r.w = wfar;
-        reinterpret_cast<ulonglong4 *>(wstat)[wave] = r;
+        ulonglong4 q;
+        q.x = sn;
+        q.y = sf;
+        q.z = wpair;
+        q.w = wfar;
+        reinterpret_cast<ulonglong4 *>(wstat)[wave] = q;
     }
 }
 
@@ -957,7 +1295,7 @@ void fmm3d_velocity(Ctx3 &c, hipStream_t s, int n, const double *x, const double
         }
         c.perm = perm;
         k3_gather<<<nb, 256, 0, s>>>(perm, khi, klo, x, y, z, sz, wx, wy, wz, active, n, P, key,
-                                     act8);
+                                     act8, hd);
         scan_exclusive_u8(act8, A, n, &hd->n_active, true, tmp, s);
         uint4 *bstat = c.bstat.as<uint4>(nb);
         if (t2) {
@@ -1012,22 +1350,24 @@ void fmm3d_velocity(Ctx3 &c, hipStream_t s, int n, const double *x, const double
 
     Cell3 *cells = c.cells.as<Cell3>(ncell);
     double *mom = c.mom.as<double>((size_t)ncell * kMomStride);
+    double *far = c.far.as<double>((size_t)ncell * kFarStride);
+    int *kids = c.kids.as<int>(((size_t)ncell + 1) * kKids);
     Src3 *S = c.src.as<Src3>((size_t)std::max(1u, t2 ? (uint32_t)n : hh.n_active));
     k3_emit<<<nb, 256, 0, s>>>(key, settle, mprev, pos, A, n, ncell, hd, p.support, p.type,
                                cells);
     k3_compact<<<nb, 256, 0, s>>>(P, A, n, t2 ? 1 : 0, S);
     if (ev) VPM_HIP(hipEventRecord(ev[1], s));
-    const int cb = div_up(ncell, 4);
-    if (ncell > 0) {
-        k3_p2m<<<div_up(ncell, 256), 256, 0, s>>>(cells, (int)ncell, S, mom);
-        k3_m2m<<<cb, 256, 0, s>>>(cells, (int)ncell, mom);
-    }
+    k3_p2m<<<div_up((long long)ncell + 1, 256), 256, 0, s>>>(cells, (int)ncell, S, mom, far, kids);
+    if (ncell > 0) k3_m2m<<<div_up(ncell, 4), 256, 0, s>>>(cells, (int)ncell, mom, far);
     if (ev) VPM_HIP(hipEventRecord(ev[2], s));
-    const int waves = div_up(n, kWave);
+    const int waves = div_up(n, kGrp);
     unsigned long long *wstat = c.wstat.as<unsigned long long>(4 * (size_t)waves);
-    k3_eval<<<div_up(waves, kEvalWaves), kEvalBlock, 0, s>>>(
-        cells, (int)ncell, mom, P, S, c.perm, n, p.u_inf, p.v_inf, p.w_inf, u, v, w, t2 ? 1 : 0,
-        wstat);
+    // the walk's stack holds at most 64 cells per non-leaf level
+    const int stk_cap = kWave * std::max(1, (int)hh.depth);
+    ((hh.flags & kF3OddStrength) ? k3_eval<true> : k3_eval<false>)<<<
+        div_up(waves, kEvalWaves), kEvalWaves * kWave, kEvalWaves * 5 * (size_t)stk_cap, s>>>(
+        cells, (int)ncell, kids, far, P, S, c.perm, n, stk_cap, p.u_inf, p.v_inf, p.w_inf, u, v, w,
+        t2 ? 1 : 0, wstat);
     if (ev) VPM_HIP(hipEventRecord(ev[3], s));
     k3_eval_stats<<<1, 1024, 0, s>>>(wstat, waves, hd);
     VPM_LAUNCH_CHECK();

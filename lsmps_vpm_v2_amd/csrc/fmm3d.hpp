@@ -10,8 +10,12 @@
 //                                  Cell3 {centre, (support size)^2, particle
 //                                  range, skip = next cell after the subtree,
 //                                  level | leaf | active} (48 B)
-//   moments: 30 FP64 per cell (the 10 order-2 Cartesian moments of each
+//   moments: 30 FP64 per leaf (the 10 order-2 Cartesian moments of each
 //            vorticity component), stride 32
+//   far rows: 30 FP64 per cell (27 combinations of its moments, its centre),
+//            stride 32 (far_row in fmm3d.hip)
+//   children: 8 indices per non-leaf cell (active children), the root's row
+//            (its non-leaf level-1 cells) last
 #pragma once
 
 #include "ctx.hpp"
@@ -44,7 +48,7 @@ struct Fmm3Hdr {
     uint32_t min_settle;  // shallowest leaf level
     double pivot[3];      // type 2: the root box's lower corner
     unsigned long long pairs, m2p;  // evaluation work: direct pairs, far-cell terms
-    // wavefront steps: sources staged for near lanes, far cells with a far lane
+    // wavefront steps: up to 64 direct pairs, up to 64 far-cell terms
     unsigned long long wave_pairs, wave_m2p;
 };
 
@@ -62,7 +66,7 @@ struct Ctx3 {
     Fmm3Hdr *hdr_d = nullptr;
     Fmm3Hdr *hdr_h = nullptr;  // pinned mirror
     DBuf hdr_buf, bbox, khi, klo, key_a, key_b, val_a, val_b, tmp;
-    DBuf par, src, key64, act8, act_scan, lcpw, settle, mprev, starts, pos, cells, mom;
+    DBuf par, src, key64, act8, act_scan, lcpw, settle, mprev, starts, pos, cells, mom, far, kids;
     DBuf bstat, wstat;
     uint32_t *perm = nullptr;  // sorted slot -> caller index (val_a or val_b)
     int levels_guess = 10;     // the previous build's sort depth
