@@ -677,26 +677,12 @@ __global__ void __launch_bounds__(kWave *kTopWaves64)
     }
 }
 
-// Evaluation: one wavefront per leaf.  Lanes are split into G groups of
-// 64/G lanes; a group owns the targets, the G groups split the sources and are
-// reduced with cross-lane shuffles.  List-1 sources are staged in LDS (x, y, q,
-// index) by the whole wavefront, then read by every lane.
-constexpr int kEvalWaves = 4;
-// Sources staged per wavefront per round: 128 (4 KB of LDS per wavefront)
-// leaves room for 7 wavefronts per SIMD where 256 allowed 5; the FP64 pair
-// loop is latency bound, and the larger count of resident wavefronts cut the
-// 780k evaluation by about 50 us.  A target's sum does not depend on it.
-constexpr int kStage64 = 128;
-
-
-
-// 1/x to full double precision: hardware estimate and two Newton steps.
+// 1/x to full double precision: the hardware estimate y (error under 2^-22)
+// corrected by y (e + e^2), e = 1 - x y, which leaves e^3.
 __device__ __forceinline__ double rcp64(double x) {
-    double y = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, y, 1.0);
-    y = fma(y, e, y);
-    e = fma(-x, y, 1.0);
-    return fma(y, e, y);
+    const double y = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, y, 1.0);
+    return fma(y, fma(e, e, e), y);
 }
 
 // Regularization factor of a near-field pair, 2 pi q of regul_func_2d
@@ -710,251 +696,402 @@ __device__ __forceinline__ double regul64(double rho2) {
     return 1.0 - (1.0 - qt) * exp(qt);
 }
 
-// ICUT 0: the singular P2P of fmm2D (fmm2D.cpp:164-173); a pair at r = 0
-// raises DUPLICATE_POINTS.  ICUT 1..3: the type-1 near field of direct_sum
+// Evaluation: W wavefronts per leaf (1, or 4 when the leaves alone would leave
+// most of the chip idle).  Lanes split into G groups of 64 / G; a lane owns two
+// targets, a group all of the leaf's (G by leaf size), and the groups and
+// wavefronts split the sources and list-3 cells and are reduced at the end.
+//
+// The kernel is bound by vector-ALU issue where leaves abound (0.74 of the
+// cycles on the 780k flat plate, half of them outside the pair loop, whose
+// leaves hold 16 targets) and by the latency of one leaf's chain where they
+// do not.  Two targets per lane halve the LDS reads per pair (24 B a source,
+// no index: only the leaf's own particles need the self test); the list-1
+// cells' ranges are read 64 at a time, so a leaf waits for three dependent
+// loads, not for three per cell.  780k flat plate 162 -> 115 us; 2,000
+// particles 55 -> 13 us; 100k clusters with the Gaussian kernel 146 -> 88 us.
+//
+// MODE 0: the singular P2P of fmm2D (fmm2D.cpp:164-173); a pair at r = 0
+// raises DUPLICATE_POINTS.  1..3: the type-1 near field of direct_sum
 // (subroutine_all_fmm_2d.cpp:594-627): each pair term times regul64 at
-// sij^2 = (si^2 + sj^2) / 4 (ss: the sorted sizes); pairs at r = 0 add
-// nothing.
+// sij^2 = (si^2 + sj^2) / 4 (ss: the sorted sizes); pairs at r = 0 add nothing.
+// kPot: the potential (fmm2D::calcPotential, fmm2D.cpp:681-896): P2P
+// q log(r^2) / 2 (potDirSum, :77-122), M2P Re[a_0 log(z - zc) -
+// sum_p a_p (z - zc)^-p / p] (:817-834), L2P Re[b_0 + sum_p b_p (z - z0)^p]
+// (:854-866); a pair at r = 0 raises DUPLICATE_POINTS (log 0).
 // T1: the type-1 FMM (biotsavart_fmm_2d.cpp:321-419): pairs at r = 0 add
 // nothing whatever the kernel; the multipoles hold orders 0..P-1 (stride P)
 // and the local expansions orders 0..P (stride P + 1) in the Cauchy form
 // F = sum_l b_l (z - z0)^l.
-// One leaf's targets in groups of 64 / G lanes, G a compile-time constant so
-// that the source stride and the group reduction are fixed and the pair loop
-// unrolls (four pairs in flight per lane); stage / stage_s are the
-// wavefront's LDS rows.  Returns whether a pair at r = 0 was seen.
-template <int ICUT, bool T1, int G>
-__device__ __forceinline__ bool eval64_leaf(int t, int j, int lane, double4 *stage,
-                                            double *stage_s, int P, const uint32_t *c_begin,
-                                            const uint32_t *c_end, const double *c_cx,
-                                            const double *c_cy, const uint32_t *off1,
-                                            const int *l1, const uint32_t *off3, const int *l3,
-                                            const double *xs, const double *ys, const double *qs,
-                                            const double *ss, const uint32_t *perm,
-                                            const double2 *ak, const double2 *bk, int velocity,
-                                            double u_inf, double v_inf, int mask, double *out_a,
-                                            double *out_b) {
-    const uint32_t b = c_begin[j], e = c_end[j];
-    constexpr int LG = kWave / G;
-    const int g = lane / LG, tl = lane % LG;
-    const int P1 = P + 1;
-    const double lcx = c_cx[j], lcy = c_cy[j];
-    const uint32_t a1 = off1[t], z1 = off1[t + 1], a3 = off3[t], z3 = off3[t + 1];
-    bool dup = false;
-    for (uint32_t tb = b; tb < e; tb += LG) {
-        const uint32_t i = tb + tl;
-        const bool valid = i < e;
-        const double xi = valid ? xs[i] : 0.0, yi = valid ? ys[i] : 0.0;
-        const double si2 = (ICUT && valid) ? ss[i] * ss[i] : 0.0;
-        double ex = 0.0, ey = 0.0;
-        // P2P over every particle of the list-1 cells, j != i (fmm2D.cpp:135-179)
-        uint32_t u = a1, pos = a1 < z1 ? c_begin[l1[a1]] : 0u;
-        while ((mask & 1) && u < z1) {
-            int fill = 0;
-            while (u < z1 && fill < kStage64) {
-                const uint32_t se = c_end[l1[u]];
-                const int take = (int)min<uint32_t>(se - pos, (uint32_t)(kStage64 - fill));
-                for (int r = lane; r < take; r += kWave) {
-                    const uint32_t src = pos + r;
-                    stage[fill + r] = make_double4(xs[src], ys[src], qs[src], (double)src);
-                    if (ICUT) stage_s[fill + r] = ss[src] * ss[src];
-                }
-                fill += take;
-                pos += take;
-                if (pos >= se && ++u < z1) pos = c_begin[l1[u]];
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll 4
-            for (int r = g; r < fill; r += G) {
-                const double4 sv = stage[r];
-                const double dx = xi - sv.x, dy = yi - sv.y;
-                const double r2 = dx * dx + dy * dy;
-                if (ICUT == 0 && !T1 && valid && (uint32_t)sv.w != i) {
-                    dup |= r2 == 0.0;
-                    const double qr = sv.z * rcp64(r2);
-                    ex += qr * dx;
-                    ey += qr * dy;
-                }
-                if (ICUT == 0 && T1 && valid && r2 > 0.0) {
-                    const double qr = sv.z * rcp64(r2);
-                    ex += qr * dx;
-                    ey += qr * dy;
-                }
-                if (ICUT != 0 && valid && r2 > 0.0) {
-                    const double sij2 = 0.25 * (si2 + stage_s[r]);
-                    const double qr = sv.z * regul64<ICUT>(r2 / sij2) * rcp64(r2);
-                    ex += qr * dx;
-                    ey += qr * dy;
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+constexpr int kEvalWaves = 4;
+constexpr int kStage64 = 128;   // sources staged per wavefront per round
+constexpr int kPot = 4;
+constexpr int kEvalP1 = 41;     // coefficients of a leaf's local expansion (orders up to 40)
+
+struct Eval64Args {
+    const uint32_t *leaf_idx;
+    int nl, P;
+    const uint8_t *c_flags;
+    const uint32_t *c_begin, *c_end;
+    const double *c_cx, *c_cy;
+    const uint32_t *off1;
+    const int *l1;
+    const uint32_t *off3;
+    const int *l3;
+    const double *xs, *ys, *qs, *ss;
+    const uint32_t *perm;
+    const double2 *ak, *bk;
+    int velocity, mask;
+    double u_inf, v_inf;
+    double *out_a, *out_b;
+    const DevHdr *hdr;
+    unsigned *flags;
+};
+
+// LDS of one wavefront: staged sources (the list-3 rows and the partial sums
+// pass through the same space), the list-1 cells' offsets, the leaf's local
+// coefficients.
+template <int MODE>
+struct Eval64Lds {
+    double2 xy[kStage64];
+    double q[kStage64];
+    double s2[MODE >= 1 && MODE <= 3 ? kStage64 : 1];
+    uint32_t off[kWave], beg[kWave];
+    double2 b[kEvalP1];
+};
+
+// One pair's contribution to a target at (xi, yi): the field in (ex, ey), or
+// the potential in ex.  skip: the target itself (own leaf only); tame: every
+// size of the round is well inside the range of rcp64 (a size of zero, say, is
+// not: the division's limits then hold).
+template <int MODE, bool T1, bool OWN>
+__device__ __forceinline__ void pair64(double xi, double yi, double si2, double2 s, double q,
+                                       double sj2, bool skip, bool tame, double &ex,
+                                       double &ey) {
+    const double dx = xi - s.x, dy = yi - s.y;
+    const double r2 = dx * dx + dy * dy;
+    if (MODE == kPot) {
+        const double t = q * log(r2) / 2.0;
+        ex += OWN && skip ? 0.0 : t;
+        return;
+    }
+    double qr = q * rcp64(r2);
+    if (MODE == 0) {
+        if (T1) qr = r2 > 0.0 ? qr : 0.0;
+        else if (OWN) qr = skip ? 0.0 : qr;
+    } else {
+        const double sij2 = 0.25 * (si2 + sj2);
+        const double rho2 = tame ? r2 * rcp64(sij2) : r2 / sij2;
+        // the factor is 1 to the last bit beyond rho^2 = 90 (1 - (1 + h) e^-h,
+        // h = 45); a wavefront with no closer pair skips the exponential
+        if (MODE == 1 || __ballot(!(rho2 > 90.0 && rho2 < 1e300))) qr *= regul64<MODE>(rho2);
+        qr = r2 > 0.0 ? qr : 0.0;
+    }
+    ex += qr * dx;
+    ey += qr * dy;
+}
+
+// The staged sources g, g + G, ... (nu of them per group, padded) against the
+// lane's two targets; r0: the sorted index of stage slot 0 (own leaf).
+template <int MODE, bool T1, bool OWN, int G>
+__device__ __forceinline__ void pairs64g(const Eval64Lds<MODE> &l, int g, int nu,
+                                         const double (&xi)[2], const double (&yi)[2],
+                                         const double (&si2)[2], uint32_t r0, uint32_t i0,
+                                         uint32_t i1, bool tame, double (&ex)[2],
+                                         double (&ey)[2]) {
+    constexpr int kUnroll = MODE == 0 ? 2 : 1;
+#pragma unroll kUnroll
+    for (int u = 0; u < nu; ++u) {
+        const int r = g + u * G;
+        const double2 s = l.xy[r];
+        const double q = l.q[r], sj2 = MODE >= 1 && MODE <= 3 ? l.s2[r] : 0.0;
+        const uint32_t src = r0 + (uint32_t)r;
+        pair64<MODE, T1, OWN>(xi[0], yi[0], si2[0], s, q, sj2, OWN && src == i0, tame, ex[0],
+                              ey[0]);
+        pair64<MODE, T1, OWN>(xi[1], yi[1], si2[1], s, q, sj2, OWN && src == i1, tame, ex[1],
+                              ey[1]);
+    }
+}
+
+// The same with the group count G a compile-time constant (LDS offsets and
+// unrolling), chosen per call.
+template <int MODE, bool T1, bool OWN>
+__device__ __forceinline__ void pairs64(const Eval64Lds<MODE> &l, int G, int g, int nu,
+                                        const double (&xi)[2], const double (&yi)[2],
+                                        const double (&si2)[2], uint32_t r0, uint32_t i0,
+                                        uint32_t i1, bool tame, double (&ex)[2],
+                                        double (&ey)[2]) {
+    switch (G) {
+        case 16: pairs64g<MODE, T1, OWN, 16>(l, g, nu, xi, yi, si2, r0, i0, i1, tame, ex, ey); break;
+        case 8: pairs64g<MODE, T1, OWN, 8>(l, g, nu, xi, yi, si2, r0, i0, i1, tame, ex, ey); break;
+        case 4: pairs64g<MODE, T1, OWN, 4>(l, g, nu, xi, yi, si2, r0, i0, i1, tame, ex, ey); break;
+        case 2: pairs64g<MODE, T1, OWN, 2>(l, g, nu, xi, yi, si2, r0, i0, i1, tame, ex, ey); break;
+        default: pairs64g<MODE, T1, OWN, 1>(l, g, nu, xi, yi, si2, r0, i0, i1, tame, ex, ey); break;
+    }
+}
+
+// Returns whether a sum of this lane's targets is not finite.
+template <int MODE, bool T1, int W>
+__device__ __forceinline__ bool eval64_leaf(const Eval64Args &A, int t, int j, int wi, int lane,
+                                            int G, Eval64Lds<MODE> *lds) {
+    const int LG = kWave / G;   // lanes of a group
+    constexpr bool kSized = MODE >= 1 && MODE <= 3;
+    Eval64Lds<MODE> &l = lds[wi];
+    const int tl = lane & (LG - 1), g = lane / LG;
+    const int P = A.P, P1 = P + 1;
+    const uint32_t b = (uint32_t)__builtin_amdgcn_readfirstlane((int)A.c_begin[j]);
+    const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)A.c_end[j]);
+    const bool own = (A.c_flags[j] & kActive) != 0;  // the leaf is in its own list 1
+    const double lcx = A.c_cx[j], lcy = A.c_cy[j];
+    const uint32_t a1 = A.off1[t], z1 = A.off1[t + 1], a3 = A.off3[t], z3 = A.off3[t + 1];
+    // padding source: zero strength, outside the root box
+    const double padx = lcx + 4.0 * A.hdr->root_len;
+    if (wi == 0)
+        for (int k = lane; k < P1; k += kWave) l.b[k] = A.bk[(size_t)j * P1 + k];
+    bool odd = false;
+    for (uint32_t tb = b; tb < e; tb += 2 * LG) {
+        const uint32_t i0 = tb + tl, i1 = i0 + LG;
+        const bool valid[2] = {i0 < e, i1 < e};
+        const uint32_t ic[2] = {valid[0] ? i0 : b, valid[1] ? i1 : b};
+        double xi[2], yi[2], si2[2] = {0.0, 0.0}, ex[2] = {0.0, 0.0}, ey[2] = {0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            xi[k] = A.xs[ic[k]];
+            yi[k] = A.ys[ic[k]];
+            if (kSized) si2[k] = A.ss[ic[k]] * A.ss[ic[k]];
         }
-        // M2P over list 3, split across groups
+        auto wild = [](double v) { return !(v > 1e-280 && v < 1e280); };
+        const bool tame_t = !kSized || __ballot(wild(si2[0]) || wild(si2[1])) == 0;
+        const bool two = tb + LG < e;  // (uniform) some lane has a second target
+        // P2P from the leaf's own particles, the wavefronts taking a share each
+        if ((A.mask & 1) && own) {
+            const uint32_t n = e - b, per = (n + W - 1) / W;
+            const uint32_t lo = min(n, wi * per), hi = min(n, lo + per);
+            for (uint32_t base = lo; base < hi; base += kStage64) {
+                const int fill = (int)min<uint32_t>(kStage64, hi - base);
+                const int nu = (fill + G - 1) / G;
+                bool odd_s = false;
+                for (int r = lane; r < nu * G; r += kWave) {
+                    const uint32_t src = b + base + min(r, fill - 1);
+                    l.xy[r] = r < fill ? make_double2(A.xs[src], A.ys[src])
+                                       : make_double2(padx, lcy);
+                    l.q[r] = r < fill ? A.qs[src] : 0.0;
+                    if (kSized) {
+                        const double s2 = A.ss[src] * A.ss[src];
+                        l.s2[r] = s2;
+                        odd_s |= wild(s2);
+                    }
+                }
+                const bool tame = tame_t && (!kSized || __ballot(odd_s) == 0);
+                wave_sync();
+                pairs64<MODE, T1, true>(l, G, g, nu, xi, yi, si2, b + base, ic[0],
+                                           two ? ic[1] : ic[0], tame, ex, ey);
+                wave_sync();
+            }
+        }
+        // P2P from the other list-1 cells, 64 cells at a time: lane k fetches
+        // cell k's range, a wave scan gives its offset in the concatenated
+        // source list, of which each wavefront stages a share
+        for (uint32_t c0 = a1; (A.mask & 1) && c0 < z1; c0 += kWave) {
+            const int ncell = (int)min<uint32_t>(kWave, z1 - c0);
+            uint32_t cnt = 0, beg = 0;
+            if (lane < ncell) {
+                const int sc = A.l1[c0 + lane];
+                if (sc != j) {  // the own leaf was done above
+                    beg = A.c_begin[sc];
+                    cnt = A.c_end[sc] - beg;
+                }
+            }
+            uint32_t inc = cnt;
+            for (int o = 1; o < kWave; o <<= 1) {
+                const uint32_t y = __shfl_up(inc, o, kWave);
+                if (lane >= o) inc += y;
+            }
+            const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)inc, kWave - 1);
+            l.off[lane] = inc - cnt;
+            l.beg[lane] = beg;
+            wave_sync();
+            const uint32_t per = (n + W - 1) / W, lo = min(n, wi * per), hi = min(n, lo + per);
+            for (uint32_t base = lo; base < hi; base += kStage64) {
+                const int fill = (int)min<uint32_t>(kStage64, hi - base);
+                const int nu = (fill + G - 1) / G;
+                bool odd_s = false;
+                for (int r = lane; r < nu * G; r += kWave) {
+                    const uint32_t gi = base + (uint32_t)min(r, fill - 1);
+                    // last cell whose offset is <= gi (empty cells share the
+                    // offset of the next one and are never the last)
+                    int cl = 0, ch = ncell - 1;
+                    while (cl < ch) {
+                        const int mid = (cl + ch + 1) >> 1;
+                        if (l.off[mid] <= gi) cl = mid;
+                        else ch = mid - 1;
+                    }
+                    const uint32_t src = l.beg[cl] + (gi - l.off[cl]);
+                    l.xy[r] = r < fill ? make_double2(A.xs[src], A.ys[src])
+                                       : make_double2(padx, lcy);
+                    l.q[r] = r < fill ? A.qs[src] : 0.0;
+                    if (kSized) {
+                        const double s2 = A.ss[src] * A.ss[src];
+                        l.s2[r] = s2;
+                        odd_s |= wild(s2);
+                    }
+                }
+                const bool tame = tame_t && (!kSized || __ballot(odd_s) == 0);
+                wave_sync();
+                pairs64<MODE, T1, false>(l, G, g, nu, xi, yi, si2, 0u, 0u, 0u, tame, ex, ey);
+                wave_sync();
+            }
+        }
+        if ((MODE == 0 && !T1) || MODE == kPot)
+#pragma unroll
+            for (int k = 0; k < 2; ++k) odd |= valid[k] && !isfinite(ex[k] + ey[k]);
+        // M2P over list 3: this wavefront's cells a3 + wi, a3 + wi + W, ...,
+        // their coefficients staged as many at a time as fit
         const int PM = T1 ? P - 1 : P;  // highest multipole order
-        for (uint32_t v = a3 + g; (mask & 2) && v < z3; v += G) {
-            const int sc = l3[v];
-            const cd wv = cinv(cd{xi - c_cx[sc], yi - c_cy[sc]});
-            const size_t sbk = (size_t)sc * (PM + 1);
-            cd f = ld(ak, sbk + PM);
-            for (int p = PM - 1; p >= 0; --p) f = cadd(cmul(f, wv), ld(ak, sbk + p));
-            f = cmul(f, wv);
-            if (valid) {
-                ex += f.x;
-                ey -= f.y;
+        const int per3 = min(kWave, kStage64 / (PM + 1));
+        for (uint32_t v0 = a3 + wi; (A.mask & 2) && v0 < z3; v0 += W * per3) {
+            const int nc = min(per3, (int)((z3 - v0 + W - 1) / W));
+            double2 *zc = reinterpret_cast<double2 *>(l.q);
+            for (int r = lane; r < nc * (PM + 1); r += kWave)
+                l.xy[r] = A.ak[(size_t)A.l3[v0 + W * (r / (PM + 1))] * (PM + 1) + r % (PM + 1)];
+            for (int r = lane; r < nc; r += kWave) {
+                const int sc = A.l3[v0 + W * r];
+                zc[r] = make_double2(A.c_cx[sc], A.c_cy[sc]);
             }
+            wave_sync();
+            for (int c = g; c < nc; c += G) {
+                const double2 z0 = zc[c];
+                const double2 *a = &l.xy[c * (PM + 1)];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const cd zr = {xi[k] - z0.x, yi[k] - z0.y};
+                    const cd wv = cinv(zr);
+                    if (MODE == kPot) {
+                        // sum_{p>=1} a_p w^p / p by Horner, then a_0 log(z - zc) minus it
+                        cd f = {0.0, 0.0};
+                        for (int p = PM; p >= 1; --p)
+                            f = cmul(cadd(f, cscale(ld(a, p), 1.0 / p)), wv);
+                        ex[k] += cmul(ld(a, 0), clog(zr)).x - f.x;
+                    } else {
+                        cd f = ld(a, PM);
+                        for (int p = PM - 1; p >= 0; --p) f = cadd(cmul(f, wv), ld(a, p));
+                        f = cmul(f, wv);
+                        ex[k] += f.x;
+                        ey[k] -= f.y;
+                    }
+                }
+            }
+            wave_sync();
         }
-        for (int m = LG; m < kWave; m <<= 1) {
-            ex += shfl_xor_d(ex, m);
-            ey += shfl_xor_d(ey, m);
+        for (int m = LG; m < kWave; m <<= 1)
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                ex[k] += shfl_xor_d(ex[k], m);
+                if (MODE != kPot) ey[k] += shfl_xor_d(ey[k], m);
+            }
+        if (W > 1) {
+            // the wavefronts' sums, added in wavefront order (two rows of 64)
+            __syncthreads();
+            if (g == 0) {
+                l.xy[tl] = make_double2(ex[0], ey[0]);
+                l.xy[kWave + tl] = make_double2(ex[1], ey[1]);
+            }
+            __syncthreads();
+            if (wi == 0)
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    for (int u = 1; u < W; ++u) {
+                        const double2 o = lds[u].xy[k * kWave + tl];
+                        ex[k] += o.x;
+                        ey[k] += o.y;
+                    }
+            __syncthreads();
+        } else {
+            wave_sync();  // (the local coefficients)
         }
-        if (valid && g == 0) {
-            if (mask & 4) {
-                // L2P
-                const cd z = {xi - lcx, yi - lcy};
-                const size_t lb = (size_t)j * P1;
-                cd f;
-                if (T1) {
-                    f = ld(bk, lb + P);
-                    for (int p = P - 1; p >= 0; --p) f = cadd(cmul(f, z), ld(bk, lb + p));
+        // every group holds the sums: groups 0 and 1 finish the lanes' first
+        // and second targets (the only group both in turn when G is 1)
+        if (wi == 0) {
+            for (int pass = 0; pass < (G == 1 ? 2 : 1); ++pass) {
+                const bool second = G == 1 ? pass == 1 : g == 1;
+                if (g > 1 || !(second ? valid[1] : valid[0])) continue;
+                double fx = second ? ex[1] : ex[0], fy = second ? ey[1] : ey[0];
+                if (A.mask & 4) {  // L2P
+                    const cd z = {(second ? xi[1] : xi[0]) - lcx, (second ? yi[1] : yi[0]) - lcy};
+                    cd f;
+                    if (T1 || MODE == kPot) {
+                        f = ld(l.b, P);
+                        for (int p = P - 1; p >= 0; --p) f = cadd(cmul(f, z), ld(l.b, p));
+                    } else {
+                        f = cscale(ld(l.b, P), (double)P);
+                        for (int p = P - 1; p >= 1; --p)
+                            f = cadd(cmul(f, z), cscale(ld(l.b, p), (double)p));
+                    }
+                    fx += f.x;
+                    fy -= f.y;
+                }
+                const uint32_t o = A.perm[second ? ic[1] : ic[0]];
+                if (MODE == kPot) {
+                    A.out_a[o] = fx;
+                } else if (A.velocity) {
+                    A.out_a[o] = fy + A.u_inf;
+                    A.out_b[o] = -fx + A.v_inf;
                 } else {
-                    f = cscale(ld(bk, lb + P), (double)P);
-                    for (int p = P - 1; p >= 1; --p)
-                        f = cadd(cmul(f, z), cscale(ld(bk, lb + p), (double)p));
+                    A.out_a[o] = fx;
+                    A.out_b[o] = fy;
                 }
-                ex += f.x;
-                ey -= f.y;
-            }
-            const uint32_t o = perm[i];
-            if (velocity) {
-                out_a[o] = ey + u_inf;
-                out_b[o] = -ex + v_inf;
-            } else {
-                out_a[o] = ex;
-                out_b[o] = ey;
             }
         }
     }
-    return dup;
+    return odd;
 }
 
-// The singular kernel is held to 64 registers per lane so that 8 wavefronts
-// per SIMD reside (7 otherwise; 27 us of 188 at 780k); the regularized ones
-// would spill under that limit and keep the compiler's choice.
-template <int ICUT, bool T1 = false>
+// The singular kernel is held to 80 registers (6 wavefronts per SIMD; 5 equal,
+// 8 spills, 1 % slower); the others keep what they need.
+template <int MODE, bool T1, int W>
 __global__ void __launch_bounds__(kWave *kEvalWaves)
-    __attribute__((amdgpu_waves_per_eu(ICUT == 0 ? 8 : 1, 8)))
-    k_eval64(const uint32_t *leaf_idx, int nl, int P, const uint32_t *c_begin, const uint32_t *c_end,
-             const double *c_cx, const double *c_cy, const uint32_t *off1, const int *l1,
-             const uint32_t *off3, const int *l3, const double *xs, const double *ys,
-             const double *qs, const double *ss, const uint32_t *perm, const double2 *ak,
-             const double2 *bk, int velocity, double u_inf, double v_inf, int mask,
-             double *out_a, double *out_b, unsigned *flags) {
-    __shared__ double4 stage[kEvalWaves][kStage64];
-    __shared__ double stage_s[ICUT ? kEvalWaves : 1][ICUT ? kStage64 : 1];
-    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const int t = blockIdx.x * kEvalWaves + w;
-    if (t >= nl) return;
-    const int j = (int)leaf_idx[t];
-    const int nt = (int)(c_end[j] - c_begin[j]);
-    double *sst = stage_s[ICUT ? w : 0];
-    bool dup;
-#define EVAL64_G(GG)                                                                          \
-    eval64_leaf<ICUT, T1, GG>(t, j, lane, stage[w], sst, P, c_begin, c_end, c_cx, c_cy, off1, \
-                              l1, off3, l3, xs, ys, qs, ss, perm, ak, bk, velocity, u_inf,   \
-                              v_inf, mask, out_a, out_b)
-    if (nt <= 8) dup = EVAL64_G(8);
-    else if (nt <= 16) dup = EVAL64_G(4);
-    else if (nt <= 32) dup = EVAL64_G(2);
-    else dup = EVAL64_G(1);
-#undef EVAL64_G
-    if (dup) atomicOr(flags, kFlagDuplicate);
+    __attribute__((amdgpu_waves_per_eu(MODE == 0 ? 6 : 4, 8))) k_eval64(Eval64Args A) {
+    __shared__ Eval64Lds<MODE> lds[kEvalWaves];
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int lane = threadIdx.x & (kWave - 1);
+    const int t = W == 1 ? (int)blockIdx.x * kEvalWaves + w : (int)blockIdx.x;
+    if (t >= A.nl) return;  // (W > 1: uniform over the workgroup)
+    const int j = __builtin_amdgcn_readfirstlane((int)A.leaf_idx[t]);
+    const int nt = (int)(A.c_end[j] - A.c_begin[j]);
+    Eval64Lds<MODE> *l = W == 1 ? lds + w : lds;
+    const int wi = W == 1 ? 0 : w;
+    const int G = nt <= 8 ? 16 : nt <= 16 ? 8 : nt <= 32 ? 4 : nt <= 64 ? 2 : 1;
+    const bool odd = eval64_leaf<MODE, T1, W>(A, t, j, wi, lane, G, l);
+    if ((MODE == 0 && !T1) || MODE == kPot)
+        // a pair at r = 0 leaves a sum that is not finite; so does a strength
+        // that is not, so the positions decide
+        if (__ballot(odd)) {
+            bool dup = false;
+            const uint32_t b = A.c_begin[j], e = A.c_end[j];
+            for (uint32_t i = b + lane; i < e; i += kWave)
+                for (uint32_t u = A.off1[t]; u < A.off1[t + 1]; ++u) {
+                    const int c = A.l1[u];
+                    for (uint32_t r = A.c_begin[c]; r < A.c_end[c]; ++r) {
+                        const double dx = A.xs[i] - A.xs[r], dy = A.ys[i] - A.ys[r];
+                        dup |= r != i && dx * dx + dy * dy == 0.0;
+                    }
+                }
+            if (dup) atomicOr(A.flags, kFlagDuplicate);
+        }
 }
 
-// Potential evaluation (fmm2D::calcPotential, fmm2D.cpp:681-896), one
-// wavefront per leaf as k_eval64: P2P phi += q log(r^2) / 2 over every
-// particle of the list-1 cells, j != i (potDirSum, :77-122); M2P over list 3,
-// Re[a_0 log(z - zc) - sum_p a_p (z - zc)^-p / p] (:817-834); L2P
-// Re[b_0 + sum_p b_p (z - z0)^p] (:854-866).  A pair at r = 0 raises
-// DUPLICATE_POINTS (log 0).
-__global__ void __launch_bounds__(kWave *kEvalWaves)
-    k_pot64(const uint32_t *leaf_idx, int nl, int P, const uint32_t *c_begin, const uint32_t *c_end,
-            const double *c_cx, const double *c_cy, const uint32_t *off1, const int *l1,
-            const uint32_t *off3, const int *l3, const double *xs, const double *ys,
-            const double *qs, const uint32_t *perm, const double2 *ak, const double2 *bk,
-            int mask, double *phi, unsigned *flags) {
-    __shared__ double4 stage[kEvalWaves][kStage64];
-    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const int t = blockIdx.x * kEvalWaves + w;
-    if (t >= nl) return;
-    const int j = (int)leaf_idx[t];
-    const uint32_t b = c_begin[j], e = c_end[j];
-    const int nt = (int)(e - b);
-    const int G = nt <= 8 ? 8 : nt <= 16 ? 4 : nt <= 32 ? 2 : 1;
-    const int LG = kWave / G;
-    const int g = lane / LG, tl = lane % LG;
-    const int P1 = P + 1;
-    const double lcx = c_cx[j], lcy = c_cy[j];
-    const uint32_t a1 = off1[t], z1 = off1[t + 1], a3 = off3[t], z3 = off3[t + 1];
-    bool dup = false;
-    for (uint32_t tb = b; tb < e; tb += LG) {
-        const uint32_t i = tb + tl;
-        const bool valid = i < e;
-        const double xi = valid ? xs[i] : 0.0, yi = valid ? ys[i] : 0.0;
-        double ph = 0.0;
-        uint32_t u = a1, pos = a1 < z1 ? c_begin[l1[a1]] : 0u;
-        while ((mask & 1) && u < z1) {
-            int fill = 0;
-            while (u < z1 && fill < kStage64) {
-                const uint32_t se = c_end[l1[u]];
-                const int take = (int)min<uint32_t>(se - pos, (uint32_t)(kStage64 - fill));
-                for (int r = lane; r < take; r += kWave) {
-                    const uint32_t src = pos + r;
-                    stage[w][fill + r] = make_double4(xs[src], ys[src], qs[src], (double)src);
-                }
-                fill += take;
-                pos += take;
-                if (pos >= se && ++u < z1) pos = c_begin[l1[u]];
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            for (int r = g; r < fill; r += G) {
-                const double4 sv = stage[w][r];
-                const double dx = xi - sv.x, dy = yi - sv.y;
-                const double r2 = dx * dx + dy * dy;
-                if (valid && (uint32_t)sv.w != i) {
-                    dup |= r2 == 0.0;
-                    ph += sv.z * log(r2) / 2.0;
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-        }
-        for (uint32_t v = a3 + g; (mask & 2) && v < z3; v += G) {
-            const int sc = l3[v];
-            const cd zr = {xi - c_cx[sc], yi - c_cy[sc]};
-            const cd wv = cinv(zr);
-            const size_t sbk = (size_t)sc * P1;
-            // sum_{p>=1} a_p w^p / p by Horner, then a_0 log(z - zc) minus it
-            cd f = {0.0, 0.0};
-            for (int p = P; p >= 1; --p) f = cmul(cadd(f, cscale(ld(ak, sbk + p), 1.0 / p)), wv);
-            const cd a0l = cmul(ld(ak, sbk), clog(zr));
-            if (valid) ph += a0l.x - f.x;
-        }
-        for (int m = LG; m < kWave; m <<= 1) ph += shfl_xor_d(ph, m);
-        if (valid && g == 0) {
-            if (mask & 4) {
-                const cd z = {xi - lcx, yi - lcy};
-                const size_t lb = (size_t)j * P1;
-                cd f = ld(bk, lb + P);
-                for (int p = P - 1; p >= 0; --p) f = cadd(cmul(f, z), ld(bk, lb + p));
-                ph += f.x;
-            }
-            phi[perm[i]] = ph;
-        }
-    }
-    if (dup) atomicOr(flags, kFlagDuplicate);
+// Leaves up to which a leaf is shared by four wavefronts: the chip holds 6,144
+// wavefronts at 6 per SIMD, and below about that many leaves the longest
+// leaf's chain is what the launch waits for (about 5,000 leaves of 100k
+// clusters, Gaussian kernel: 426 us a solve with one wavefront per leaf, 397
+// with four; about 13,000 of a 200k plate: 531 and 570).
+constexpr int kSplitLeaves = 8192;
+
+template <int MODE, bool T1>
+void eval64_launch(const Eval64Args &A, hipStream_t s) {
+    if (A.nl <= kSplitLeaves)
+        k_eval64<MODE, T1, 4><<<A.nl, kWave * kEvalWaves, 0, s>>>(A);
+    else
+        k_eval64<MODE, T1, 1><<<div_up(A.nl, kEvalWaves), kWave * kEvalWaves, 0, s>>>(A);
 }
 
 // Type-1 M2L and P2L (biotsavart_fmm_2d.cpp:199-271) for every cell of level
@@ -1064,6 +1201,39 @@ __global__ void __launch_bounds__(256)
 }
 
 }  // namespace
+
+static Eval64Args eval64_args(const Ctx &c, int P, bool velocity, double u_inf, double v_inf,
+                              int mask, double *out_a, double *out_b) {
+    Eval64Args A{};
+    A.leaf_idx = (const uint32_t *)c.leaf_idx.p;
+    A.nl = c.info.n_leaves;
+    A.P = P;
+    A.c_flags = (const uint8_t *)c.c_flags.p;
+    A.c_begin = (const uint32_t *)c.c_begin.p;
+    A.c_end = (const uint32_t *)c.c_end.p;
+    A.c_cx = (const double *)c.c_cx.p;
+    A.c_cy = (const double *)c.c_cy.p;
+    A.off1 = (const uint32_t *)c.off1.p;
+    A.l1 = (const int *)c.l1.p;
+    A.off3 = (const uint32_t *)c.off3.p;
+    A.l3 = (const int *)c.l3.p;
+    A.xs = (const double *)c.xs.p;
+    A.ys = (const double *)c.ys.p;
+    A.qs = (const double *)c.qs.p;
+    A.ss = (const double *)c.ss.p;
+    A.perm = c.perm_sorted;
+    A.ak = (const double2 *)c.ak.p;
+    A.bk = (const double2 *)c.bk.p;
+    A.velocity = velocity ? 1 : 0;
+    A.mask = mask;
+    A.u_inf = u_inf;
+    A.v_inf = v_inf;
+    A.out_a = out_a;
+    A.out_b = out_b;
+    A.hdr = c.hdr_d;
+    A.flags = &c.hdr_d->flags;
+    return A;
+}
 
 void fmm64_run(Ctx &c, int P, int list4_mode, int stage_mask, double *out_a, double *out_b,
                bool velocity, double u_inf, double v_inf, const FmmMarks &mk, bool potential) {
@@ -1175,28 +1345,13 @@ void fmm64_run(Ctx &c, int P, int list4_mode, int stage_mask, double *out_a, dou
                                                                          c_cx, c_cy, bk);
     }
     mk.mark(5, s);
-    if (potential) {
-        k_pot64<<<div_up(nl, kEvalWaves), kWave * kEvalWaves, 0, s>>>(
-            leaf_idx, nl, P, c_begin, c_end, c_cx, c_cy, (const uint32_t *)c.off1.p,
-            (const int *)c.l1.p, (const uint32_t *)c.off3.p, (const int *)c.l3.p, xs, ys, qs,
-            c.perm_sorted, ak, bk, stage_mask, out_a, &c.hdr_d->flags);
-        mk.mark(6, s);
-        VPM_LAUNCH_CHECK();
-        return;
-    }
-    const double *ss = (const double *)c.ss.p;
-    auto eval = [&](auto kern) {
-        kern<<<div_up(nl, kEvalWaves), kWave * kEvalWaves, 0, s>>>(
-            leaf_idx, nl, P, c_begin, c_end, c_cx, c_cy, (const uint32_t *)c.off1.p,
-            (const int *)c.l1.p, (const uint32_t *)c.off3.p, (const int *)c.l3.p, xs, ys, qs, ss,
-            c.perm_sorted, ak, bk, velocity ? 1 : 0, u_inf, v_inf, stage_mask, out_a, out_b,
-            &c.hdr_d->flags);
-    };
-    switch (c.icut) {
-        case 1: eval(k_eval64<1>); break;
-        case 2: eval(k_eval64<2>); break;
-        case 3: eval(k_eval64<3>); break;
-        default: eval(k_eval64<0>); break;
+    const Eval64Args ea = eval64_args(c, P, velocity, u_inf, v_inf, stage_mask, out_a, out_b);
+    switch (potential ? kPot : c.icut) {
+        case 1: eval64_launch<1, false>(ea, s); break;
+        case 2: eval64_launch<2, false>(ea, s); break;
+        case 3: eval64_launch<3, false>(ea, s); break;
+        case kPot: eval64_launch<kPot, false>(ea, s); break;
+        default: eval64_launch<0, false>(ea, s); break;
     }
     mk.mark(6, s);
     VPM_LAUNCH_CHECK();
@@ -1245,18 +1400,12 @@ void fmm_t1_run(Ctx &c, int ND, double *u, double *v, double u_inf, double v_inf
             c_cy, bk);
     }
     mk.mark(5, s);
-    const double *ss = (const double *)c.ss.p;
-    auto eval = [&](auto kern) {
-        kern<<<div_up(nl, kEvalWaves), kWave * kEvalWaves, 0, s>>>(
-            leaf_idx, nl, ND, c_begin, c_end, c_cx, c_cy, (const uint32_t *)c.off1.p,
-            (const int *)c.l1.p, (const uint32_t *)c.off3.p, (const int *)c.l3.p, xs, ys, qs, ss,
-            c.perm_sorted, ak, bk, 1, u_inf, v_inf, 7, u, v, &c.hdr_d->flags);
-    };
+    const Eval64Args ea = eval64_args(c, ND, true, u_inf, v_inf, 7, u, v);
     switch (c.icut) {
-        case 1: eval(k_eval64<1, true>); break;
-        case 2: eval(k_eval64<2, true>); break;
-        case 3: eval(k_eval64<3, true>); break;
-        default: eval(k_eval64<0, true>); break;
+        case 1: eval64_launch<1, true>(ea, s); break;
+        case 2: eval64_launch<2, true>(ea, s); break;
+        case 3: eval64_launch<3, true>(ea, s); break;
+        default: eval64_launch<0, true>(ea, s); break;
     }
     mk.mark(6, s);
     VPM_LAUNCH_CHECK();

@@ -1,0 +1,61 @@
+"""The FP64 evaluation at the edges of its groups (leaves of up to 8, 16, 32,
+64 and more particles), of its 128-source rounds, and on both sides of the
+number of leaves up to which four wavefronts share a leaf: velocity, regularized
+velocity and potential against the oracle, 1e-10 relative as the other FP64
+parity tests (the same FP64 sums in another order; measured under 1e-14)."""
+import numpy as np
+import pytest
+
+from lsmps_vpm_v2_amd import FmmSolver, workloads as W
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-10
+
+
+def _rel(a, b):
+    return float(np.linalg.norm(np.asarray(a) - np.asarray(b)) / np.linalg.norm(b))
+
+
+CASES = [(7, 4), (700, 7), (700, 8), (700, 9), (900, 16), (900, 17), (1500, 32), (1500, 33),
+         (3000, 64), (3000, 65), (3000, 130), (4000, 300), (60001, 8)]
+
+
+@pytest.mark.parametrize("n,cap", CASES, ids=[f"{n}-{c}" for n, c in CASES])
+def test_groups_match_oracle(gpu, oracle, n, cap):
+    f = W.random_clusters(n, seed=n + cap, active_frac=0.9)
+    print(f"eval64 n={n} max_par={cap}", flush=True)
+    kw = dict(max_par=cap, max_src=cap)
+    a = [f[k] for k in ("x", "y", "s", "omega", "active")]
+    for icut in (0, 1, 2, 3):
+        u, v = FmmSolver(icutoff=icut, u_inf=0.0, **kw).velocity(*a)
+        u0, v0 = oracle.velocity(*a, oracle.opts(icutoff=icut, **kw), 0.0, 0.0)
+        assert _rel(np.hypot(u - u0, v - v0) + np.hypot(u0, v0), np.hypot(u0, v0)) <= TOL
+    b = [f[k] for k in ("x", "y", "q", "active")]
+    phi = FmmSolver(**kw).potential(*b)
+    assert _rel(phi, oracle.fmm_potential(*b, oracle.opts(**kw))) <= TOL
+
+
+@pytest.mark.parametrize("n", [3000, 60001])
+def test_strength_that_is_not_finite_is_no_duplicate(gpu, n):
+    """A NaN strength is not a DUPLICATE_POINTS error, and does not reach the
+    particle that carries it through its own pair."""
+    f = W.random_clusters(n, seed=3)
+    w = f["omega"].copy()
+    w[n // 3] = np.nan
+    # one tree level, so that everything is near field
+    for icut in (0, 2):
+        s = FmmSolver(max_par=4096, max_src=4096, icutoff=icut) if n < 4096 else FmmSolver(icutoff=icut)
+        u, v = s.velocity(f["x"], f["y"], f["s"], w, f["active"])
+        bad = np.isnan(u)
+        assert bad.any() and not bad[n // 3]
+
+
+def test_sizes_of_zero(gpu, oracle):
+    """Gaussian near field of point particles: the factor is 1."""
+    f = W.random_clusters(2000, seed=9)
+    z = np.zeros_like(f["s"])
+    z[::2] = f["s"][::2]
+    a = [f["x"], f["y"], z, f["omega"], f["active"]]
+    u, v = FmmSolver(icutoff=2).velocity(*a)
+    u0, v0 = oracle.velocity(*a, oracle.opts(icutoff=2), 1.0, 0.0)
+    assert np.isfinite(u).all() and _rel(u, u0) <= TOL and _rel(v, v0) <= TOL
