@@ -64,12 +64,16 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 // P2M (fmm2D.cpp:237-284, with the sign and 1/p folded into the translation
-// tables): four leaves per wavefront, 16 lanes each.  A leaf's lanes stage 16
-// of its particles at a time in LDS as (z - zc, q), zero strength for
-// inactive particles and leaves; lane r then adds q (z - zc)^p for its own
-// order p = k0 + r over the staged particles, in particle order (the
-// reference's loop order), with no cross-lane reduction.  Orders beyond 15
-// take further chunks of 16.
+// tables): four leaves per wavefront, 16 lanes each.  A leaf's lanes take 16
+// of its particles at a time, and lane i stages q z^b (b = 0..3) and z^(4a)
+// (a = 0..3) of its particle, z from the leaf's centre, zero strength for
+// inactive particles and leaves; lane r then adds its own order p = 4a + b as
+// one complex product per particle, four FMAs from two LDS reads, with no
+// cross-lane reduction.  Orders beyond 15 take further chunks of 16.  (Forming
+// z^p afresh per particle and order took about 40 operations: 37 -> 13 us at
+// 780k particles, order 10; 21 -> 5 us at 2,000.)
+// Block 0 also clears the rows no later stage writes: the root's multipole,
+// and the local expansions of levels 0 and 1 (nz rows of bk, stride bs).
 constexpr int kP2m64Waves = 4;
 constexpr int kP2mLanes = 16;                    // lanes per leaf
 constexpr int kP2mLeaves = kWave / kP2mLanes;    // leaves per wavefront
@@ -78,13 +82,20 @@ __global__ void __launch_bounds__(kWave *kP2m64Waves)
     k_p2m64(const uint32_t *leaf_idx, int nl, int P, const uint8_t *c_flags,
             const uint32_t *c_begin, const uint32_t *c_end, const double *c_cx,
             const double *c_cy, const double *xs, const double *ys, const double *qs,
-            const uint8_t *as, double2 *ak) {
-    __shared__ double4 stg[kP2m64Waves][kWave];
+            const uint8_t *as, double2 *ak, double2 *bk, int nz, int bs) {
+    // row b of leaf g from b 68 + g 17: the 16 rows a wavefront reads at a time
+    // lie on different banks
+    constexpr int kB = 68, kG = kP2mLanes + 1;
+    __shared__ double2 lo[kP2m64Waves][4 * kB], hi[kP2m64Waves][4 * kB];
     const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
     const int g = lane / kP2mLanes, r = lane % kP2mLanes;
     const long long t = ((long long)blockIdx.x * kP2m64Waves + w) * kP2mLeaves + g;
-    const bool has = t < nl;
     const int P1 = P + 1;
+    if (blockIdx.x == 0) {
+        for (int k = threadIdx.x; k < P1; k += blockDim.x) ak[k] = make_double2(0.0, 0.0);
+        for (int k = threadIdx.x; k < nz * bs; k += blockDim.x) bk[k] = make_double2(0.0, 0.0);
+    }
+    const bool has = t < nl;
     const int j = has ? (int)leaf_idx[t] : 0;
     const bool act = has && (c_flags[j] & kActive) != 0;
     const uint32_t b = has ? c_begin[j] : 0u, cnt = has ? c_end[j] - b : 0u;
@@ -97,17 +108,33 @@ __global__ void __launch_bounds__(kWave *kP2m64Waves)
         const int p = k0 + r;
         cd acc = {0.0, 0.0};
         for (uint32_t base = 0; base < mx; base += kP2mLanes) {
-            double4 v = make_double4(0.0, 0.0, 0.0, 0.0);
-            const uint32_t i = b + base + (uint32_t)r;
-            if (act && base + (uint32_t)r < cnt && as[i])
-                v = make_double4(xs[i] - cx, ys[i] - cy, qs[i], 0.0);
-            stg[w][lane] = v;
+            const bool in = act && base + (uint32_t)r < cnt;
+            const uint32_t i = in ? b + base + (uint32_t)r : 0u;
+            const uint8_t ai = as[i];  // (the four loads in one round)
+            const double xi = xs[i], yi = ys[i], qi = qs[i];
+            const bool src = in && ai != 0;
+            const cd z = {src ? xi - cx : 0.0, src ? yi - cy : 0.0};
+            const double q = src ? qi : 0.0;
+            const cd z2 = cmul(z, z), z4 = cmul(z2, z2), z8 = cmul(z4, z4);
+            cd f = {q, 0.0};
+            if (k0 > 0) f = cscale(cpowi(z, k0), q);
+            const cd f1 = cmul(f, z), f2 = cmul(f, z2);
+            const int me = g * kG + r;
+            st(lo[w], me, f);
+            st(lo[w], kB + me, f1);
+            st(lo[w], 2 * kB + me, f2);
+            st(lo[w], 3 * kB + me, cmul(f1, z2));
+            st(hi[w], me, cd{1.0, 0.0});
+            st(hi[w], kB + me, z4);
+            st(hi[w], 2 * kB + me, z8);
+            st(hi[w], 3 * kB + me, cmul(z8, z4));
             wave_sync();
-            if (p < P1) {
-                for (int u = 0; u < kP2mLanes; ++u) {
-                    const double4 sv = stg[w][g * kP2mLanes + u];
-                    if (sv.z != 0.0) acc = cadd(acc, cscale(cpowi(cd{sv.x, sv.y}, p), sv.z));
-                }
+            const double2 *fl = lo[w] + (r & 3) * kB + g * kG, *fh = hi[w] + (r >> 2) * kB + g * kG;
+#pragma unroll 4
+            for (int u = 0; u < kP2mLanes; ++u) {
+                const double2 x = fl[u], y = fh[u];
+                acc.x += x.x * y.x - x.y * y.y;
+                acc.y += x.x * y.y + x.y * y.x;
             }
             wave_sync();
         }
@@ -141,107 +168,130 @@ __global__ void __launch_bounds__(256)
     st(ak, (size_t)j * P1 + p, acc);
 }
 
-// The same M2M with G parent cells per wavefront, 64 / G lanes each (G = 4
-// for orders P <= 15, 1 up to 16): a cell's four children's coefficients and
-// the table are staged in LDS in one round of loads, then lane p of the cell
-// runs k_m2m64's Horner sums from LDS (the same operations in the same
-// order), so a level costs one dependent load, not one per order.
-constexpr int kTrWaves = 4;    // wavefronts per block of the per-cell translations
+// M2M and L2L in spans of three levels (orders P <= 16): one workgroup per cell
+// of a span's top level walks that cell's subtree through the span, 16 lanes
+// per cell and 16 cells at a time.  A subtree of three levels holds at most 4 +
+// 16 + 64 cells however the tree is shaped, so the workgroups stay balanced,
+// and a pass over ten levels is three launches instead of seven or nine, each
+// of which cost 5 to 9 us whatever it held.  What bounds a launch is its chain
+// of dependent loads (about 0.8 us each): the child slots of the three levels,
+// then every row and centre of the subtree at once, into LDS, where the levels
+// follow each other.
 constexpr int kTrP1 = 17;      // orders up to 16
+constexpr int kSpan = 3;
+constexpr int kSpanBlock = 256;
+constexpr int kSpanLanes = 16;                          // lanes per cell
+constexpr int kSpanCells = kSpanBlock / kSpanLanes;     // cells at a time
 
-template <int G>
-__global__ void __launch_bounds__(kWave *kTrWaves)
-    k_m2m64w(int j0, int j1, int P, const double *tab, const uint8_t *c_flags, const double *c_cx,
-             const double *c_cy, const int *c_child, double2 *ak) {
-    constexpr int LN = kWave / G;
-    __shared__ double s_tab[kTrP1 * kTrP1];
-    __shared__ double2 sa[kTrWaves][G][4 * kTrP1];
-    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const int g = lane / LN, r = lane % LN;
-    const int P1 = P + 1;
-    for (int t = threadIdx.x; t < P1 * P1; t += blockDim.x) s_tab[t] = tab[t];
-    const int j = j0 + ((int)blockIdx.x * kTrWaves + w) * G + g;
-    const bool live = j < j1 && !(c_flags[j] & kLeaf);  // uniform over the cell's lanes
-    int4 c4 = make_int4(-1, -1, -1, -1);
-    if (live) {
-        c4 = reinterpret_cast<const int4 *>(c_child)[j];
-        for (int idx = r; idx < 4 * P1; idx += LN) {
-            const int q = idx / P1, k = idx - q * P1;
-            const int ch = q == 0 ? c4.x : q == 1 ? c4.y : q == 2 ? c4.z : c4.w;
-            sa[w][g][q * kTrP1 + k] = ch >= 0 ? ak[(size_t)ch * P1 + k] : make_double2(0.0, 0.0);
+// The subtree of a cell, n <= 3 levels deep: the cells of each level are
+// consecutive (the children of consecutive cells, in level-major Morton
+// order).  Slot of cell i of level l: span_base(l) + i (0; 1..4; 5..20); link
+// (slot, q) = 4 slot + q stands for child q of a slot.
+struct SpanTree {
+    int child[4 * 21];           // cell index per link, -1: none
+    int up[4 + 16 + 64];         // link of cell i of level l at span_up(l) + i
+    int lo[kSpan + 1], hi[kSpan + 1];
+};
+__device__ __forceinline__ int span_base(int l) { return l == 0 ? 0 : l == 1 ? 1 : 5; }
+__device__ __forceinline__ int span_up(int l) { return l == 1 ? 0 : l == 2 ? 4 : 20; }
+
+// Fills t (every thread calls it; the first wavefront walks).
+__device__ __forceinline__ void span_walk(SpanTree &t, int j, int n, const int *c_child) {
+    if (threadIdx.x >= kWave && threadIdx.x < kWave + 4 * 21) t.child[threadIdx.x - kWave] = -1;
+    __syncthreads();
+    if (threadIdx.x < kWave) {
+        const int i = (int)threadIdx.x;
+        int a = j, b = j + 1;
+        if (i == 0) {
+            t.lo[0] = a;
+            t.hi[0] = b;
+        }
+        for (int l = 1; l <= n; ++l) {
+            const int c = i < 4 * (b - a) ? c_child[4 * a + i] : -1;  // at most 16 cells
+            if (c >= 0) t.child[4 * span_base(l - 1) + i] = c;
+            int mn = c >= 0 ? c : 0x7fffffff, mx = c >= 0 ? c + 1 : 0;
+#pragma unroll
+            for (int m = 1; m < kWave; m <<= 1) {
+                mn = min(mn, __shfl_xor(mn, m, kWave));
+                mx = max(mx, __shfl_xor(mx, m, kWave));
+            }
+            a = mx > 0 ? mn : 0;
+            b = mx;
+            if (c >= 0) t.up[span_up(l) + c - a] = 4 * span_base(l - 1) + i;
+            if (i == 0) {
+                t.lo[l] = a;
+                t.hi[l] = b;
+            }
         }
     }
     __syncthreads();
-    if (!live || r > P) return;
-    const int p = r;
-    const double cx = c_cx[j], cy = c_cy[j];
-    cd acc = {0.0, 0.0};
-    for (int q = 0; q < 4; ++q) {
-        const int ch = q == 0 ? c4.x : q == 1 ? c4.y : q == 2 ? c4.z : c4.w;
-        if (ch < 0) continue;
-        const cd d = {c_cx[ch] - cx, c_cy[ch] - cy};
-        const double2 *a = &sa[w][g][q * kTrP1];
-        cd sacc = ld(a, 0);
-        for (int k = 1; k <= p; ++k) sacc = cadd(cmul(sacc, d), cscale(ld(a, k), s_tab[p * P1 + k]));
-        acc = cadd(acc, sacc);
-    }
-    st(ak, (size_t)j * P1 + p, acc);
+}
+__device__ __forceinline__ bool span_leaf(const SpanTree &t, int slot) {
+    const int *c = t.child + 4 * slot;
+    return (c[0] & c[1] & c[2] & c[3]) < 0;  // every slot -1
 }
 
-// M2M for the parents of levels Lhi .. 1 (each holding at most kTopCells64
-// cells, orders P <= 15) in one workgroup: k_m2m64w's four-cells-per-wavefront
-// body, a level at a time with a barrier between levels, in place of a launch
-// per level.
-constexpr int kTopWaves64 = 8;
-constexpr int kTopCells64 = 64;
-
-__global__ void __launch_bounds__(kWave *kTopWaves64)
-    k_m2m64_top(int Lhi, const DevHdr *hdr, int P, const double *tab, const uint8_t *c_flags,
-                const double *c_cx, const double *c_cy, const int *c_child, double2 *ak) {
-    constexpr int G = 4, LN = kWave / G, S = kTrP1 - 1;
+// M2M for the cells of the `levels` levels from each level-L0 cell (j0 + block)
+// down, from the multipoles of the level below them (formed before) and of the
+// leaves: lane p of a cell runs k_m2m64's Horner sums over the children's rows
+// and its result is both stored and left as its parent's operand.
+__global__ void __launch_bounds__(kSpanBlock)
+    k_m2m64_span(int j0, int levels, int P, const double *tab, const double *c_cx,
+                 const double *c_cy, const int *c_child, double2 *ak) {
+    __shared__ SpanTree t;
     __shared__ double s_tab[kTrP1 * kTrP1];
-    __shared__ double2 sa[kTopWaves64][G][4 * S];
-    __shared__ int s_off[kMaxDepth + 2];
-    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const int g = lane / LN, r = lane % LN;
-    const int P1 = P + 1;
-    for (int t = threadIdx.x; t < P1 * P1; t += blockDim.x) s_tab[t] = tab[t];
-    if (threadIdx.x < kMaxDepth + 2) s_off[threadIdx.x] = (int)hdr->lev_off[threadIdx.x];
+    __shared__ double2 op[4 * 21][kTrP1];  // a child's row per link
+    __shared__ double2 ctr[1 + 4 * 21];    // centres: the top cell's, then per link
+    const int P1 = P + 1, g = threadIdx.x / kSpanLanes, r = threadIdx.x % kSpanLanes;
+    const int top = j0 + (int)blockIdx.x;
+    for (int u = threadIdx.x; u < P1 * P1; u += blockDim.x) s_tab[u] = tab[u];
+    span_walk(t, top, levels, c_child);
+    const int links = 4 * (levels == 1 ? 1 : levels == 2 ? 5 : 21);
+    for (int e = threadIdx.x; e < links * P1; e += blockDim.x) {
+        const int k = e / P1, ch = t.child[k], s = k >> 2;
+        const int l = s == 0 ? 0 : s < 5 ? 1 : 2;
+        if (ch >= 0 && (l + 1 == levels || span_leaf(t, span_base(l + 1) + ch - t.lo[l + 1])))
+            op[k][e - k * P1] = ak[(size_t)ch * P1 + (e - k * P1)];
+    }
+    for (int k = threadIdx.x; k <= links; k += blockDim.x) {
+        const int ch = k == 0 ? top : t.child[k - 1];
+        if (ch >= 0) ctr[k] = make_double2(c_cx[ch], c_cy[ch]);
+    }
     __syncthreads();
-    for (int L = Lhi; L >= 1; --L) {
-        const int j0 = s_off[L], nj = s_off[L + 1] - j0;
-        for (int u0 = 0; u0 < nj; u0 += kTopWaves64 * G) {
-            const int u = u0 + w * G + g, j = j0 + u;
-            const bool live = u < nj && !(c_flags[j] & kLeaf);
-            int4 c4 = make_int4(-1, -1, -1, -1);
-            if (live) {
-                c4 = reinterpret_cast<const int4 *>(c_child)[j];
-                for (int idx = r; idx < 4 * P1; idx += LN) {
-                    const int q = idx / P1, k = idx - q * P1;
-                    const int ch = q == 0 ? c4.x : q == 1 ? c4.y : q == 2 ? c4.z : c4.w;
-                    sa[w][g][q * S + k] = ch >= 0 ? ak[(size_t)ch * P1 + k] : make_double2(0.0, 0.0);
+    for (int l = levels - 1; l >= 0; --l) {
+        const int j = t.lo[l] + g, slot = span_base(l) + g;
+        if (j < t.hi[l] && !span_leaf(t, slot)) {
+            const int up = l == 0 ? -1 : t.up[span_up(l) + g];
+            const double2 c0 = ctr[up + 1];
+            const double2 (*a)[kTrP1] = op + 4 * slot;
+            cd d[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                d[q] = {ctr[4 * slot + q + 1].x - c0.x, ctr[4 * slot + q + 1].y - c0.y};
+            for (int p = r; p < P1; p += kSpanLanes) {
+                // the four children's sums side by side, every order's lane
+                // over all k (its own end by a select)
+                cd sacc[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sacc[q] = ld(a[q], 0);
+#pragma unroll 2
+                for (int k = 1; k <= P; ++k) {
+                    const double tk = s_tab[p * P1 + k];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const cd n = cadd(cmul(sacc[q], d[q]), cscale(ld(a[q], k), tk));
+                        sacc[q] = {k <= p ? n.x : sacc[q].x, k <= p ? n.y : sacc[q].y};
+                    }
                 }
-            }
-            wave_sync();
-            if (live && r <= P) {
-                const int p = r;
-                const double cx = c_cx[j], cy = c_cy[j];
                 cd acc = {0.0, 0.0};
-                for (int q = 0; q < 4; ++q) {
-                    const int ch = q == 0 ? c4.x : q == 1 ? c4.y : q == 2 ? c4.z : c4.w;
-                    if (ch < 0) continue;
-                    const cd d = {c_cx[ch] - cx, c_cy[ch] - cy};
-                    const double2 *a = &sa[w][g][q * S];
-                    cd sacc = ld(a, 0);
-                    for (int k = 1; k <= p; ++k)
-                        sacc = cadd(cmul(sacc, d), cscale(ld(a, k), s_tab[p * P1 + k]));
-                    acc = cadd(acc, sacc);
-                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (t.child[4 * slot + q] >= 0) acc = cadd(acc, sacc[q]);
                 st(ak, (size_t)j * P1 + p, acc);
+                if (l > 0) st(op[up], p, acc);
             }
-            wave_sync();
         }
-        __syncthreads();  // the next level up reads these multipoles
+        __syncthreads();  // the next level up reads these rows
     }
 }
 
@@ -551,6 +601,7 @@ __global__ void __launch_bounds__(kWave *kM2l64Waves) __attribute__((amdgpu_wave
     if (LEFT) red[w][4][lane] = acc4;
     __syncthreads();
     if (w != 0) return;
+    if (lane < cnt) bk[(size_t)(j0 + lane) * P1] = make_double2(0.0, 0.0);  // b_0 is not formed
     double *bo = reinterpret_cast<double *>(bk);
     if (LEFT) {
         double sum = 0.0;
@@ -599,81 +650,99 @@ __global__ void __launch_bounds__(256)
     st(bk, o, cadd(ld(bk, o), s));
 }
 
-// The same L2L with G child cells per wavefront, 64 / G lanes each (as
-// k_m2m64w): the parent's coefficients and the table are staged in LDS in
-// one round of loads, then lane i of the cell runs k_l2l64's Horner sum for
-// order p from LDS (the same operations in the same order).
-template <bool POT, int G>
-__global__ void __launch_bounds__(kWave *kTrWaves)
-    k_l2l64w(int j0, int j1, int P, const double *tab, const int *c_parent, const double *c_cx,
-             const double *c_cy, double2 *bk) {
-    constexpr int LN = kWave / G;
-    __shared__ double s_tab[kTrP1 * kTrP1];
-    __shared__ double2 sb[kTrWaves][G][kTrP1];
-    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const int g = lane / LN, r = lane % LN;
-    const int P1 = P + 1, NP = POT ? P1 : P;
-    for (int t = threadIdx.x; t < P1 * P1; t += blockDim.x) s_tab[t] = tab[t];
-    const int j = j0 + ((int)blockIdx.x * kTrWaves + w) * G + g;
-    const bool live = j < j1;  // uniform over the cell's lanes
-    int par = 0;
-    if (live) {
-        par = c_parent[j];
-        for (int k = r; k < P1; k += LN) sb[w][g][k] = bk[(size_t)par * P1 + k];
+// L2L for the cells up to `levels` below each level-L0 cell (j0 + block), whose
+// own expansion is complete (k_m2m64_span's walk, downward): a cell's parent's
+// row is read from LDS, lane p of the cell forms its order's sum, and the row
+// stays in LDS for the next level.
+enum L2lKind { kL2lField, kL2lPot, kL2lT1 };
+
+// Type-1 L2L (biotsavart_fmm_2d.cpp:283-312), order l of a child displaced by d
+// from its parent (local coefficients b, orders 0..ND):
+//   sum_{k = l..ND} coef[l][k] d^expo[l][k] b_k,
+// with the table of the shift as the reference runs it (or the exact one).
+// Along a row the exponent rises by one per term except at most once, where
+// it is formed afresh.
+__device__ __forceinline__ cd l2l_t1_sum(int l, int ND, const double *coef, const int *expo, cd d,
+                                         const double2 *b) {
+    const int NL = ND + 1;
+    cd s = {0.0, 0.0}, pw = {1.0, 0.0};
+    int e_prev = 0;
+    for (int k = l; k <= ND; ++k) {
+        const int e = expo[l * NL + k];
+        if (e == e_prev + 1) pw = cmul(pw, d);
+        else if (e != e_prev) pw = cpowi(d, e);
+        e_prev = e;
+        s = cadd(s, cscale(cmul(pw, ld(b, k)), coef[l * NL + k]));
     }
-    __syncthreads();
-    if (!live || r >= NP) return;
-    const int p = (POT ? 0 : 1) + r;
-    const cd d = {c_cx[j] - c_cx[par], c_cy[j] - c_cy[par]};
-    const double *row = s_tab + p * P1;
-    const double2 *b = sb[w][g];
-    cd s = cscale(ld(b, P), row[P]);
-    for (int k = P - 1; k >= p; --k) s = cadd(cmul(s, d), cscale(ld(b, k), row[k]));
-    const size_t o = (size_t)j * P1 + p;
-    st(bk, o, cadd(ld(bk, o), s));
+    return s;
 }
 
-// L2L into the cells of levels 3 .. Lhi (each holding at most kTopCells64
-// cells, orders P <= 15) in one workgroup: k_l2l64w's body, a level at a
-// time with a barrier between levels, in place of a launch per level.
-template <bool POT>
-__global__ void __launch_bounds__(kWave *kTopWaves64)
-    k_l2l64_top(int Lhi, const DevHdr *hdr, int P, const double *tab, const int *c_parent,
-                const double *c_cx, const double *c_cy, double2 *bk) {
-    constexpr int G = 4, LN = kWave / G;
+template <int KIND>
+__global__ void __launch_bounds__(kSpanBlock)
+    k_l2l64_span(int j0, int levels, int P, const double *tab, const int *expo,
+                 const int *c_child, const double *c_cx, const double *c_cy, double2 *bk) {
+    __shared__ SpanTree t;
     __shared__ double s_tab[kTrP1 * kTrP1];
-    __shared__ double2 sb[kTopWaves64][G][kTrP1];
-    __shared__ int s_off[kMaxDepth + 2];
-    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const int g = lane / LN, r = lane % LN;
-    const int P1 = P + 1, NP = POT ? P1 : P;
-    for (int t = threadIdx.x; t < P1 * P1; t += blockDim.x) s_tab[t] = tab[t];
-    if (threadIdx.x < kMaxDepth + 2) s_off[threadIdx.x] = (int)hdr->lev_off[threadIdx.x];
+    __shared__ int s_exp[KIND == kL2lT1 ? kTrP1 * kTrP1 : 1];
+    __shared__ double2 row[1 + 4 * 21][kTrP1];  // the top cell's, then per link
+    __shared__ double2 ctr[1 + 4 * 21];
+    __shared__ double2 pw[KIND == kL2lT1 ? kSpanCells : 1][kTrP1];  // powers of d
+    const int P1 = P + 1, g = threadIdx.x / kSpanLanes, r = threadIdx.x % kSpanLanes;
+    const int top = j0 + (int)blockIdx.x;
+    for (int u = threadIdx.x; u < P1 * P1; u += blockDim.x) {
+        s_tab[u] = tab[u];
+        if (KIND == kL2lT1) s_exp[u] = expo[u];
+    }
+    span_walk(t, top, levels, c_child);
+    const int links = 4 * (levels == 1 ? 1 : levels == 2 ? 5 : 21);
+    for (int e = threadIdx.x; e < (links + 1) * P1; e += blockDim.x) {
+        const int k = e / P1, j = k == 0 ? top : t.child[k - 1];
+        if (j >= 0) row[k][e - k * P1] = bk[(size_t)j * P1 + (e - k * P1)];
+    }
+    for (int k = threadIdx.x; k <= links; k += blockDim.x) {
+        const int j = k == 0 ? top : t.child[k - 1];
+        if (j >= 0) ctr[k] = make_double2(c_cx[j], c_cy[j]);
+    }
     __syncthreads();
-    for (int L = 3; L <= Lhi; ++L) {
-        const int j0 = s_off[L], nj = s_off[L + 1] - j0;
-        for (int u0 = 0; u0 < nj; u0 += kTopWaves64 * G) {
-            const int u = u0 + w * G + g, j = j0 + u;
-            const bool live = u < nj;
-            int par = 0;
-            if (live) {
-                par = c_parent[j];
-                for (int k = r; k < P1; k += LN) sb[w][g][k] = bk[(size_t)par * P1 + k];
+    for (int l = 1; l <= levels; ++l) {
+        for (int i = g; i < t.hi[l] - t.lo[l]; i += kSpanCells) {
+            const int link = t.up[span_up(l) + i], slot = link >> 2;
+            // the parent's own link, or the top cell
+            const int par = slot == 0 ? 0 : t.up[span_up(l - 1) + slot - span_base(l - 1)] + 1;
+            const double2 *b = row[par];
+            const cd d = {ctr[link + 1].x - ctr[par].x, ctr[link + 1].y - ctr[par].y};
+            if (KIND == kL2lT1) {
+                for (int p = r; p < P1; p += kSpanLanes) st(pw[g], p, cpowi(d, p));
+                wave_sync();
             }
-            wave_sync();
-            if (live && r < NP) {
-                const int p = (POT ? 0 : 1) + r;
-                const cd d = {c_cx[j] - c_cx[par], c_cy[j] - c_cy[par]};
-                const double *row = s_tab + p * P1;
-                const double2 *b = sb[w][g];
-                cd sv = cscale(ld(b, P), row[P]);
-                for (int k = P - 1; k >= p; --k) sv = cadd(cmul(sv, d), cscale(ld(b, k), row[k]));
-                const size_t o = (size_t)j * P1 + p;
-                st(bk, o, cadd(ld(bk, o), sv));
+            for (int p = r; p < P1; p += kSpanLanes) {
+                cd v = ld(row[link + 1], p);
+                if (KIND == kL2lT1) {
+                    // l2l_t1_sum with the powers at hand
+                    cd s = {0.0, 0.0};
+#pragma unroll 4
+                    for (int k = 0; k < P1; ++k) {
+                        const cd n = cscale(cmul(ld(pw[g], s_exp[p * P1 + k]), ld(b, k)),
+                                            s_tab[p * P1 + k]);
+                        s = {k >= p ? s.x + n.x : s.x, k >= p ? s.y + n.y : s.y};
+                    }
+                    v = cadd(v, s);
+                } else if (KIND == kL2lPot || p > 0) {
+                    const double *tr = s_tab + p * P1;
+                    cd s = cscale(ld(b, P), tr[P]);
+#pragma unroll 4
+                    for (int k = P - 1; k >= (KIND == kL2lPot ? 0 : 1); --k) {
+                        const cd n = cadd(cmul(s, d), cscale(ld(b, k), tr[k]));
+                        s = {k >= p ? n.x : s.x, k >= p ? n.y : s.y};
+                    }
+                    v = cadd(v, s);
+                }
+                if (KIND != kL2lField || p > 0) st(bk, (size_t)(t.lo[l] + i) * P1 + p, v);
+                st(row[link + 1], p, v);
             }
-            wave_sync();
+            if (KIND == kL2lT1) wave_sync();
         }
-        __syncthreads();  // the next level down reads these coefficients
+        __syncthreads();  // the next level down reads these rows
     }
 }
 
@@ -1135,12 +1204,8 @@ __global__ void __launch_bounds__(256)
     st(bk, (size_t)j * NL + l, acc);
 }
 
-// Type-1 L2L (biotsavart_fmm_2d.cpp:283-312) for the cells of one level
-// (>= 3; level-1 locals are zero): thread per (cell, l),
-//   b_l += sum_{k = l..ND} coef[l][k] d^expo[l][k] b_k(parent),  d = zc - zp,
-// with the table of the shift as the reference runs it (or the exact one).
-// Along a row the exponent rises by one per term except at most once, where
-// it is formed afresh.
+// Type-1 L2L for the cells of one level (>= 3; level-1 locals are zero), thread
+// per (cell, l): orders ND above 15.
 __global__ void __launch_bounds__(256)
     k_l2l_t1(int j0, int j1, int ND, const double *coef, const int *expo, const int *c_parent,
              const double *c_cx, const double *c_cy, double2 *bk) {
@@ -1150,18 +1215,8 @@ __global__ void __launch_bounds__(256)
     const int j = j0 + (int)(idx / NL), l = (int)(idx % NL);
     const int par = c_parent[j];
     const cd d = {c_cx[j] - c_cx[par], c_cy[j] - c_cy[par]};
-    const size_t b = (size_t)par * NL;
-    cd s = {0.0, 0.0}, pw = {1.0, 0.0};
-    int e_prev = 0;
-    for (int k = l; k <= ND; ++k) {
-        const int e = expo[l * NL + k];
-        if (e == e_prev + 1) pw = cmul(pw, d);
-        else if (e != e_prev) pw = cpowi(d, e);
-        e_prev = e;
-        s = cadd(s, cscale(cmul(pw, ld(bk, b + k)), coef[l * NL + k]));
-    }
     const size_t o = (size_t)j * NL + l;
-    st(bk, o, cadd(ld(bk, o), s));
+    st(bk, o, cadd(ld(bk, o), l2l_t1_sum(l, ND, coef, expo, d, bk + (size_t)par * NL)));
 }
 
 // FP64 direct sum with LDS source tiles (accuracy reference only).
@@ -1235,14 +1290,34 @@ static Eval64Args eval64_args(const Ctx &c, int P, bool velocity, double u_inf, 
     return A;
 }
 
+// M2M from the leaves' multipoles up to level 1.
+static void m2m64_run(const TreeInfo &ti, int P, const double *tab, const uint8_t *c_flags,
+                      const double *c_cx, const double *c_cy, const int *c_child, double2 *ak,
+                      hipStream_t s) {
+    if (P < kTrP1) {
+        for (int S = ti.max_level; S > 1; S -= kSpan) {
+            const int L0 = std::max(1, S - kSpan);
+            k_m2m64_span<<<(int)(ti.lev_off[L0 + 1] - ti.lev_off[L0]), kSpanBlock, 0, s>>>(
+                (int)ti.lev_off[L0], S - L0, P, tab, c_cx, c_cy, c_child, ak);
+        }
+        return;
+    }
+    for (int L = ti.max_level - 1; L >= 1; --L) {
+        const int j0 = (int)ti.lev_off[L], j1 = (int)ti.lev_off[L + 1];
+        k_m2m64<<<div_up((long long)(j1 - j0) * (P + 1), 256), 256, 0, s>>>(
+            j0, j1, P, tab, c_flags, c_cx, c_cy, c_child, ak);
+    }
+}
+
 void fmm64_run(Ctx &c, int P, int list4_mode, int stage_mask, double *out_a, double *out_b,
                bool velocity, double u_inf, double v_inf, const FmmMarks &mk, bool potential) {
     hipStream_t s = c.stream;
     const TreeInfo &ti = c.info;
     const int nc = ti.n_cells, nl = ti.n_leaves, P1 = P + 1;
     double2 *ak = c.ak.as<double2>((size_t)nc * P1), *bk = c.bk.as<double2>((size_t)nc * P1);
-    VPM_HIP(hipMemsetAsync(ak, 0, sizeof(double2) * (size_t)nc * P1, s));
-    VPM_HIP(hipMemsetAsync(bk, 0, sizeof(double2) * (size_t)nc * P1, s));
+    // every row a later stage reads is written by the stage that forms it, the
+    // exceptions by P2M; above order 16 order 0 of the local rows is not
+    if (P >= kTrP1) VPM_HIP(hipMemsetAsync(bk, 0, sizeof(double2) * (size_t)nc * P1, s));
     const uint8_t *c_flags = (const uint8_t *)c.c_flags.p;
     const uint32_t *c_begin = (const uint32_t *)c.c_begin.p, *c_end = (const uint32_t *)c.c_end.p;
     const double *c_cx = (const double *)c.c_cx.p, *c_cy = (const double *)c.c_cy.p;
@@ -1255,29 +1330,9 @@ void fmm64_run(Ctx &c, int P, int list4_mode, int stage_mask, double *out_a, dou
                  *t_l2l = (const double *)c.tab_l2l.p;
 
     k_p2m64<<<div_up(nl, kP2m64Waves * kP2mLeaves), kWave * kP2m64Waves, 0, s>>>(
-        leaf_idx, nl, P, c_flags, c_begin, c_end, c_cx, c_cy, xs, ys, qs, as, ak);
-    // the top levels (parents 1 .. Lt, each of at most kTopCells64 cells) go to
-    // one workgroup after the per-level launches below them
-    auto lev_cnt = [&](int L) { return (int)(ti.lev_off[L + 1] - ti.lev_off[L]); };
-    int Lt = 0;
-    if (P1 <= kTrP1 - 1)
-        while (Lt + 1 <= ti.max_level - 1 && lev_cnt(Lt + 1) <= kTopCells64) ++Lt;
-    for (int L = ti.max_level - 1; L > Lt; --L) {
-        const int j0 = (int)ti.lev_off[L], j1 = (int)ti.lev_off[L + 1];
-        if (j1 <= j0) continue;
-        if (P1 <= kTrP1 - 1)
-            k_m2m64w<4><<<div_up(j1 - j0, kTrWaves * 4), kWave * kTrWaves, 0, s>>>(
-                j0, j1, P, t_m2m, c_flags, c_cx, c_cy, c_child, ak);
-        else if (P1 == kTrP1)
-            k_m2m64w<1><<<div_up(j1 - j0, kTrWaves), kWave * kTrWaves, 0, s>>>(
-                j0, j1, P, t_m2m, c_flags, c_cx, c_cy, c_child, ak);
-        else
-            k_m2m64<<<div_up((long long)(j1 - j0) * P1, 256), 256, 0, s>>>(
-                j0, j1, P, t_m2m, c_flags, c_cx, c_cy, c_child, ak);
-    }
-    if (Lt >= 1)
-        k_m2m64_top<<<1, kWave * kTopWaves64, 0, s>>>(Lt, c.hdr_d, P, t_m2m, c_flags, c_cx, c_cy,
-                                                     c_child, ak);
+        leaf_idx, nl, P, c_flags, c_begin, c_end, c_cx, c_cy, xs, ys, qs, as, ak, bk,
+        (int)ti.lev_off[2], P1);
+    m2m64_run(ti, P, t_m2m, c_flags, c_cx, c_cy, c_child, ak, s);
     mk.mark(3, s);
     // M2L: every cell of level >= 2
     const int j2 = (int)ti.lev_off[2];
@@ -1319,30 +1374,20 @@ void fmm64_run(Ctx &c, int P, int list4_mode, int stage_mask, double *out_a, dou
             (const int *)c.l4.p, (const uint8_t *)c.n4.p, c_cx, c_cy, c_begin, c_end, xs, ys, qs,
             as, ak, bk);
     mk.mark(4, s);
-    // L2L: children at levels 3 .. maxL (parents 2 .. maxL-1, fmm2D.cpp:587);
-    // the top children levels (3 .. Lc, each of at most kTopCells64 cells) in
-    // one workgroup first
-    int Lc = 2;
-    if (P1 <= kTrP1 - 1)
-        while (Lc + 1 <= ti.max_level && lev_cnt(Lc + 1) <= kTopCells64) ++Lc;
-    if (Lc >= 3)
-        (potential ? k_l2l64_top<true> : k_l2l64_top<false>)<<<1, kWave * kTopWaves64, 0, s>>>(
-            Lc, c.hdr_d, P, t_l2l, c_parent, c_cx, c_cy, bk);
-    for (int L = std::max(3, Lc + 1); L <= ti.max_level; ++L) {
-        const int j0 = (int)ti.lev_off[L], j1 = (int)ti.lev_off[L + 1];
-        if (j1 <= j0) continue;
-        if (P1 <= kTrP1 - 1)
-            (potential ? k_l2l64w<true, 4> : k_l2l64w<false, 4>)<<<div_up(j1 - j0, kTrWaves * 4),
-                                                                  kWave * kTrWaves, 0, s>>>(
-                j0, j1, P, t_l2l, c_parent, c_cx, c_cy, bk);
-        else if (P1 == kTrP1)
-            (potential ? k_l2l64w<true, 1> : k_l2l64w<false, 1>)<<<div_up(j1 - j0, kTrWaves),
-                                                                  kWave * kTrWaves, 0, s>>>(
-                j0, j1, P, t_l2l, c_parent, c_cx, c_cy, bk);
-        else
+    // L2L: children at levels 3 .. maxL (parents 2 .. maxL-1, fmm2D.cpp:587)
+    if (P < kTrP1) {
+        for (int L = 2; L < ti.max_level; L += kSpan)
+            (potential ? k_l2l64_span<kL2lPot> : k_l2l64_span<kL2lField>)<<<
+                (int)(ti.lev_off[L + 1] - ti.lev_off[L]), kSpanBlock, 0, s>>>(
+                (int)ti.lev_off[L], std::min(kSpan, ti.max_level - L), P, t_l2l, nullptr, c_child,
+                c_cx, c_cy, bk);
+    } else {
+        for (int L = 3; L <= ti.max_level; ++L) {
+            const int j0 = (int)ti.lev_off[L], j1 = (int)ti.lev_off[L + 1];
             (potential ? k_l2l64<true> : k_l2l64<false>)<<<div_up((long long)(j1 - j0) * NP, 256),
                                                             256, 0, s>>>(j0, j1, P, t_l2l, c_parent,
                                                                          c_cx, c_cy, bk);
+        }
     }
     mk.mark(5, s);
     const Eval64Args ea = eval64_args(c, P, velocity, u_inf, v_inf, stage_mask, out_a, out_b);
@@ -1363,7 +1408,6 @@ void fmm_t1_run(Ctx &c, int ND, double *u, double *v, double u_inf, double v_inf
     const TreeInfo &ti = c.info;
     const int nc = ti.n_cells, nl = ti.n_leaves, NL = ND + 1, PM = ND - 1;
     double2 *ak = c.ak.as<double2>((size_t)nc * ND), *bk = c.bk.as<double2>((size_t)nc * NL);
-    VPM_HIP(hipMemsetAsync(ak, 0, sizeof(double2) * (size_t)nc * ND, s));
     const uint8_t *c_flags = (const uint8_t *)c.c_flags.p, *c_level = (const uint8_t *)c.c_level.p;
     const uint32_t *c_begin = (const uint32_t *)c.c_begin.p, *c_end = (const uint32_t *)c.c_end.p;
     const double *c_cx = (const double *)c.c_cx.p, *c_cy = (const double *)c.c_cy.p;
@@ -1375,14 +1419,10 @@ void fmm_t1_run(Ctx &c, int ND, double *u, double *v, double u_inf, double v_inf
 
     // upward: P2M and M2M at order PM = ND - 1 (biotsavart_fmm_2d.cpp:123-188;
     // the exact shift C(p, k), the reference's bico values to rounding)
+    // (the root's local row is not read: the tree's leaves are of level >= 1)
     k_p2m64<<<div_up(nl, kP2m64Waves * kP2mLeaves), kWave * kP2m64Waves, 0, s>>>(
-        leaf_idx, nl, PM, c_flags, c_begin, c_end, c_cx, c_cy, xs, ys, qs, as, ak);
-    for (int L = ti.max_level - 1; L >= 1; --L) {
-        const int j0 = (int)ti.lev_off[L], j1 = (int)ti.lev_off[L + 1];
-        if (j1 <= j0) continue;
-        k_m2m64<<<div_up((long long)(j1 - j0) * ND, 256), 256, 0, s>>>(
-            j0, j1, PM, (const double *)c.t1_m2m.p, c_flags, c_cx, c_cy, c_child, ak);
-    }
+        leaf_idx, nl, PM, c_flags, c_begin, c_end, c_cx, c_cy, xs, ys, qs, as, ak, bk, 1, NL);
+    m2m64_run(ti, PM, (const double *)c.t1_m2m.p, c_flags, c_cx, c_cy, c_child, ak, s);
     mk.mark(3, s);
     // M2L and P2L: every cell of level >= 1 (all of bk written)
     const int j1 = (int)ti.lev_off[1];
@@ -1392,12 +1432,19 @@ void fmm_t1_run(Ctx &c, int ND, double *u, double *v, double u_inf, double v_inf
             (const uint8_t *)c.n2.p, (const int *)c.l4.p, (const uint8_t *)c.n4.p, c_cx, c_cy,
             c_begin, c_end, xs, ys, qs, ak, bk);
     mk.mark(4, s);
-    for (int L = 3; L <= ti.max_level; ++L) {
-        const int j0 = (int)ti.lev_off[L], jz = (int)ti.lev_off[L + 1];
-        if (jz <= j0) continue;
-        k_l2l_t1<<<div_up((long long)(jz - j0) * NL, 256), 256, 0, s>>>(
-            j0, jz, ND, (const double *)c.t1_l2l_c.p, (const int *)c.t1_l2l_e.p, c_parent, c_cx,
-            c_cy, bk);
+    const double *coef = (const double *)c.t1_l2l_c.p;
+    const int *expo = (const int *)c.t1_l2l_e.p;
+    if (ND < kTrP1) {
+        for (int L = 2; L < ti.max_level; L += kSpan)
+            k_l2l64_span<kL2lT1><<<(int)(ti.lev_off[L + 1] - ti.lev_off[L]), kSpanBlock, 0, s>>>(
+                (int)ti.lev_off[L], std::min(kSpan, ti.max_level - L), ND, coef, expo, c_child,
+                c_cx, c_cy, bk);
+    } else {
+        for (int L = 3; L <= ti.max_level; ++L) {
+            const int j0 = (int)ti.lev_off[L], jz = (int)ti.lev_off[L + 1];
+            k_l2l_t1<<<div_up((long long)(jz - j0) * NL, 256), 256, 0, s>>>(j0, jz, ND, coef, expo,
+                                                                          c_parent, c_cx, c_cy, bk);
+        }
     }
     mk.mark(5, s);
     const Eval64Args ea = eval64_args(c, ND, true, u_inf, v_inf, 7, u, v);
