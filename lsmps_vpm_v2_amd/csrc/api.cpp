@@ -272,13 +272,9 @@ void ensure_tables(vpmfmm_handle *h) {
     VPM_HIP(hipMemcpyAsync(c.tab_m2m.get(nb), m2m.data(), nb, hipMemcpyHostToDevice, c.stream));
     VPM_HIP(hipMemcpyAsync(c.tab_l2l.get(nb), l2l.data(), nb, hipMemcpyHostToDevice, c.stream));
     // the list-2 M2L matrices for the matrix cores (orders up to 16)
-    std::vector<double> r64;
     c.tab_r64_p = -1;
     if (P >= 1 && P <= 16) {
-        fmm64_mfma_table(P, m2l.data(), r64);
-        const size_t nr = r64.size() * sizeof(double);
-        VPM_HIP(hipMemcpyAsync(c.tab_r64.get(nr), r64.data(), nr, hipMemcpyHostToDevice,
-                               c.stream));
+        fmm64_mfma_table(P, false, (const double *)c.tab_m2l.p, c.tab_r64, c.stream);
         c.tab_r64_p = P;
     }
     VPM_HIP(hipStreamSynchronize(c.stream));
@@ -789,6 +785,7 @@ void ensure_t1_tables(vpmfmm_handle *h, int nd, int mode) {
     };
     up(c.t1_m2m, m2m.data(), m2m.size() * sizeof(double));
     up(c.t1_m2l, tm2l.data(), tm2l.size() * sizeof(double));
+    if (nd <= 16) fmm64_mfma_table(nd, true, (const double *)c.t1_m2l.p, c.t1_r64, c.stream);
     up(c.t1_l2l_c, coef.data(), coef.size() * sizeof(double));
     up(c.t1_l2l_e, expo.data(), expo.size() * sizeof(int));
     VPM_HIP(hipStreamSynchronize(c.stream));

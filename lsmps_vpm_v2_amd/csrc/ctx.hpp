@@ -174,6 +174,7 @@ struct Ctx {
     // L2L coefficients and exponents (ndp + 1)^2, and the all-active flags
     // of a type-1 call
     DBuf t1_m2m, t1_m2l, t1_l2l_c, t1_l2l_e, t1_ones;
+    DBuf t1_r64;  // type-1 M2L matrices for the matrix cores (ndp <= 16)
 
     // mixed path: FP32 particle offsets and sources, tables, tiles
     DBuf oxy, qf;
@@ -247,10 +248,10 @@ void fmm64_run(Ctx &c, int p, int list4_mode, int stage_mask, double *out_a, dou
                bool velocity, double u_inf, double v_inf, const FmmMarks &mk,
                bool potential = false);
 
-// The FP64 path's list-2 M2L matrices for the matrix cores, order P <= 16,
-// from its M2L table tab ((P+1) x (P+1)): 40 offsets x 2P x 2(P+1) in
-// v_mfma_f64_16x16x4f64 A-operand lane order.
-void fmm64_mfma_table(int P, const double *tab, std::vector<double> &R);
+// The list-2 M2L matrices for the matrix cores, order P <= 16, from the FP64
+// path's M2L table tab ((P+1) x (P+1)) or, with type1, the type-1 one
+// ((P+1) x P), both on the device: 40 offsets in A-operand lane order.
+void fmm64_mfma_table(int P, bool type1, const double *tab, DBuf &R, hipStream_t s);
 
 // Type-1 FMM (fmm64.hip, biotsavart_fmm_2d.cpp:93-446) on a type-1 tree:
 // multipoles of orders 0..ndp-1 (P2M, M2M), locals of orders 0..ndp from

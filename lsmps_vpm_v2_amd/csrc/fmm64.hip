@@ -469,26 +469,58 @@ __global__ void __launch_bounds__(kWave *kM2lwWaves)
     }
 }
 
-// List-2 M2L of the FP64 path on the matrix cores (orders P <= 16, field and
-// velocity; the potential keeps k_m2l64w).  A workgroup takes a tile of 16
-// consecutive cells of one level; the tiles of levels 2.. follow each other
-// in the grid.  With len the level's cell side and delta = (zs - zt) / len
-// (|dx|, |dy| <= 3, not both <= 1: 40 offsets), the list-2 sum
+// M2L of the FP64 path on the matrix cores (orders P <= 16, field and velocity;
+// the potential keeps k_m2l64w) and of the type-1 path (T1, ND = P <= 16).
+// With len the level's cell side and delta = (zs - zt) / len (|dx|, |dy| <= 3,
+// not both <= 1: 40 offsets), the list-2 sum
 //   b_p = sum_k tab[p][k] a_k (zs - zt)^-(p+k)
 // is, in the scaled coefficients a^_k = a_k len^-k and b^_p = b_p len^p,
 //   b^ = sum over offsets of M_delta a^,  M_delta[p][k] = tab[p][k] delta^-(p+k),
-// a realified 2P x 2(P+1) matrix per offset (fmm64_mfma_table), the A operand
-// of v_mfma_f64_16x16x4f64; the B operand is a source cell's a^ along
-// K = 2(P+1).  Lane l: target column n = l % 16, k-quarter kq = l / 16;
-// wavefront w takes the offsets w, w + kM2l64Waves, ... that a target of the
-// tile uses, and the wavefronts' accumulators are summed through LDS.  The
-// output rows follow the f64 instruction's layout D[4v + l / 16][l % 16].
-// The offset is exact here, where the reference forms zs - zt from rounded
+// a realified 2P x 2(P+1) matrix per offset (fmm64_mfma_table), the A operand;
+// the B operand is a source cell's a^.  Type 1 has a_0..a_{P-1} and Cauchy
+// coefficients b_0..b_P: b_l = sum_k tab[l][k] a_k (zs - zt)^-(l+1+k), 2(P+1) x
+// 2P.  The offset is exact here, where the reference forms zs - zt from rounded
 // centres: the two agree to the rounding of the centres (about 1e-16 of the
-// root box over the cell side).  List 4 is added afterwards by k_m2l64w in
-// its list-4 mode.
-constexpr int kM2l64Waves = 4;
+// root box over the cell side).
+//
+// A workgroup takes 96 consecutive cells of one level and sorts them into the
+// four classes of a cell's place in its parent: list 2 lies within the
+// parent's neighbours, so a class has 27 of the 40 offsets, and 32 targets of
+// one class (16 above order 12) take an offset's matrix together.  Two
+// wavefronts share a class (every other offset each, summed through LDS).
+// What bound 16 unsorted targets at a time (120 us on the 780k flat plate, the
+// matrix cores busy a quarter of it) was the L1: 1 GB of matrices from L2, and
+// a lane's 8 or 16 bytes of a source row at a time, 64 accesses a load, up to 27
+// times per row.  The source rows of the workgroup, about 200, are found with a
+// hash table and staged in LDS once, scaled; a matrix is read once per 32
+// targets, the next one's loads under way while this one's products run, and a
+// half of the 32 without a source at the offset takes no products: 81 us, now
+// bound by the products (14 offsets a wavefront) and, a quarter, by the lists'
+// and rows' dependent loads.  Type 1 at 200k: one thread per order and cell 121
+// us, 34 us.  (96 cells and not 128: where some children are missing a class
+// would exceed its 32 targets and need a second round.)
+//
+// NQ = 1: a workgroup takes one of the four classes, all its wavefronts the
+// class's offsets.  A tree of a few workgroups' cells leaves the chip idle
+// while each of them runs its 14 offsets in turn (18 of 28 us): the 2000
+// particle solve takes 226 us with four classes per workgroup and 218 with one,
+// 54k vortices 371 and 364; the lists are read four times, which a larger tree
+// pays for: 780k 543 and 593, type 1 at 200k 422 and 435.
+//
+// Rows beyond a multiple of 16 go four at a time to v_mfma_f64_4x4x4f64 if they
+// are at most 8 (a quarter of the cycles each): its A operand holds row l % 4
+// and column l / 16 of a step, its B operand is laid out as the 16x16x4 one
+// (target l % 16, step row l / 16) and its result is row l / 16 of target
+// l % 16.  The 16x16x4 result is row 4 v + l / 16 of target l % 16.
+constexpr int kM2lCells = 96;   // cells per workgroup
+constexpr int kM2lWaves = 8;
+constexpr int kM2lBlock = kWave * kM2lWaves;
+constexpr int kM2lSlots = 36;   // 6 x 6 source places around the parent's neighbourhood
+constexpr int kM2lHash = 1024;  // hash table of the workgroup's sources
+constexpr int kM2lProbes = 16;
+constexpr int kM2lRowBytes = 56 * 1024;  // LDS of the staged rows
 typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ uint32_t compact1by1(uint32_t v) {
     v &= 0x55555555u;
@@ -499,131 +531,301 @@ __device__ __forceinline__ uint32_t compact1by1(uint32_t v) {
     return v;
 }
 
-// Eight resident wavefronts per SIMD (the register budget that allows them:
-// 64 per lane, accumulators included): the kernel waits on its gathers, and
-// 8 instead of 5 resident wavefronts cut it from 170 to 146 us at 780k (p 10).
-template <int P>
-__global__ void __launch_bounds__(kWave *kM2l64Waves) __attribute__((amdgpu_waves_per_eu(8, 8)))
-    k_m2l64_mfma(const DevHdr *hdr, int maxL, const uint32_t *c_key, const int *l2,
+// The workgroups of each level: level L (2 .. maxL) has blocks first[L] ..
+// first[L + 1] - 1 and cells cell0[L] .. cell0[L + 1] - 1.
+struct M2lLevels {
+    int first[kMaxDepth + 2], cell0[kMaxDepth + 2];
+    int maxL;
+};
+
+// Sizes of an order's matrices (host and device).
+template <int P, bool T1>
+struct M2lShape {
+    static constexpr int RW = T1 ? 2 * P + 2 : 2 * P;        // rows
+    static constexpr int K = T1 ? 2 * P : 2 * P + 2;         // columns
+    static constexpr int KP = (K + 7) / 8, KS = 2 * KP;      // steps of 4 columns, in pairs
+    static constexpr int R16 = RW / 16, REM = RW % 16;
+    static constexpr int T16 = REM > 8 ? R16 + 1 : R16;      // 16-row tiles
+    static constexpr int T4 = REM > 8 ? 0 : (REM + 3) / 4;   // 4-row tiles after them
+    static constexpr int NS = T16 + T4;
+    static constexpr int ACC = 4 * T16 + T4;                 // accumulators per lane and target set
+    // sets of 16 targets per wavefront: two while they fit 128 registers
+    static constexpr int U = P <= 12 ? 2 : 1;
+    static constexpr bool AHEAD = KS * NS <= 12;             // and the next matrix too
+};
+
+template <int P, bool T1, int NQ>
+__global__ void __launch_bounds__(kM2lBlock) __attribute__((amdgpu_waves_per_eu(4, 4)))
+    k_m2l64_mfma(const DevHdr *hdr, M2lLevels lv, const uint32_t *c_key, const int *l2,
                  const uint8_t *n2, const double *R, const double2 *ak, double2 *bk) {
-    constexpr int P1 = P + 1, K = 2 * P1, KS = (K + 3) / 4, MT = (2 * P + 15) / 16;
-    __shared__ int smap[16][49];
-    __shared__ double red[kM2l64Waves][MT * 4][kWave];
-    __shared__ double s_sc[P1];
-    __shared__ int s_tile[3];
-    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    if (threadIdx.x == 0) {
-        // this block's tile: level L, first cell, cells (up to 16)
-        int b = (int)blockIdx.x, L = 2, j0 = -1, cnt = 0;
-        for (; L <= maxL; ++L) {
-            const int c0 = (int)hdr->lev_off[L], cn = (int)hdr->lev_off[L + 1] - c0;
-            const int nt = (cn + 15) / 16;
-            if (b < nt) {
-                j0 = c0 + 16 * b;
-                cnt = min(16, cn - 16 * b);
-                break;
-            }
-            b -= nt;
+    using Sh = M2lShape<P, T1>;
+    constexpr int K = Sh::K, KP = Sh::KP, KS = Sh::KS, NS = Sh::NS, T16 = Sh::T16, T4 = Sh::T4;
+    constexpr int P1 = P + 1, U = Sh::U;
+    constexpr int kShare = kM2lWaves / NQ;          // wavefronts per class
+    constexpr int AS = T1 ? P : P1;                 // coefficients per cell of ak
+    constexpr int kRows = kM2lRowBytes / (16 * AS); // rows that fit
+    __shared__ union {
+        double2 row[kRows][AS];
+        double red[NQ][kShare - 1][U * Sh::ACC][kWave];
+    } s;
+    // source per target and place: a staged row, -1: none, below: cell -2 - v
+    __shared__ int src[kM2lCells][kM2lSlots];
+    __shared__ int ht[kM2lHash];            // source cells by hash, -1: free
+    __shared__ uint16_t hid[kM2lHash];      // their rows
+    __shared__ int rowcell[kRows];
+    __shared__ uint8_t memb[4][kM2lCells];  // the classes' members
+    __shared__ int n_memb[2][4], n_rows;
+    __shared__ double s_sc[P1 + 1];         // len^-k
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int lane = tid & (kWave - 1);
+    const int blk = (int)blockIdx.x / (4 / NQ), only = NQ == 1 ? (int)blockIdx.x % 4 : 0;
+    int L = 2;
+    while (L < lv.maxL && blk >= lv.first[L + 1]) ++L;
+    const int j0 = lv.cell0[L] + kM2lCells * (blk - lv.first[L]);
+    const int cnt = min(kM2lCells, lv.cell0[L + 1] - j0);
+    // list entries of the workgroup's cells, 27 places per cell
+    constexpr int kPer = (27 * kM2lCells + kM2lBlock - 1) / kM2lBlock;
+    int ent[kPer], slot[kPer];
+    uint32_t kt[kPer], ks[kPer];  // keys of the target and the source
+    {
+        // (every load of a round in flight together: clamped, then selected)
+        int len[kPer];
+#pragma unroll
+        for (int v = 0; v < kPer; ++v) {
+            const int e = min(tid + v * kM2lBlock, 27 * cnt - 1), c = e / 27;
+            len[v] = (int)n2[j0 + c];
+            kt[v] = c_key[j0 + c];
+            ent[v] = l2[27 * (size_t)j0 + e];
         }
-        s_tile[0] = L;
-        s_tile[1] = j0;
-        s_tile[2] = cnt;
+#pragma unroll
+        for (int v = 0; v < kPer; ++v) {
+            const int e = tid + v * kM2lBlock;
+            if (e >= 27 * cnt || e % 27 >= len[v] || (NQ == 1 && (int)(kt[v] & 3u) != only))
+                ent[v] = -1;
+        }
+#pragma unroll
+        for (int v = 0; v < kPer; ++v) ks[v] = c_key[max(ent[v], 0)];
     }
-    for (int t = threadIdx.x; t < 16 * 49; t += blockDim.x) smap[t / 49][t % 49] = -1;
-    __syncthreads();
-    const int L = s_tile[0], j0 = s_tile[1], cnt = s_tile[2];
-    if (j0 < 0) return;  // (uniform over the block)
-    if (threadIdx.x < P1) {
-        // len^-k, k = 0..P
+    if (tid <= P1) {
         const double inv = ldexp(1.0 / hdr->root_len, L);
         double sc = 1.0;
-        for (int k = 0; k < (int)threadIdx.x; ++k) sc *= inv;
-        s_sc[threadIdx.x] = sc;
+        for (int k = 0; k < tid; ++k) sc *= inv;
+        s_sc[tid] = sc;
     }
-    {
-        // source map of the tile: slot (dx+3) + 7 (dy+3) -> source cell or -1
-        const int tn = threadIdx.x % 16, tu = threadIdx.x / 16;
-        const int tj = j0 + tn;
-        if (tn < cnt) {
-            const uint32_t kj = c_key[tj];
-            const int jx = (int)compact1by1(kj), jy = (int)compact1by1(kj >> 1);
-            const int m2 = n2[tj];
-            for (int u = tu; u < m2; u += (int)blockDim.x / 16) {
-                const int sidx = l2[27 * tj + u];
-                const uint32_t ks = c_key[sidx];
-                const int dx = (int)compact1by1(ks) - jx, dy = (int)compact1by1(ks >> 1) - jy;
-                smap[tn][(dx + 3) + 7 * (dy + 3)] = sidx;
+    for (int t = tid; t < kM2lCells * kM2lSlots; t += kM2lBlock) (&src[0][0])[t] = -1;
+    for (int t = tid; t < kM2lHash; t += kM2lBlock) ht[t] = -1;
+    if (tid == 0) n_rows = 0;
+    // the classes' members, in cell order (two wavefronts hold a cell a lane)
+    const int cls = tid < cnt ? (int)(c_key[j0 + tid] & 3u) : -1;
+    uint64_t same = 0;
+    if (w < 2) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint64_t m = __ballot(cls == q);
+            if (cls == q) same = m;
+            if (lane == 0) n_memb[w][q] = __popcll(m);
+        }
+    }
+    __syncthreads();
+    if (cls >= 0) {
+        const int r = __popcll(same & (lane ? ~0ull >> (kWave - lane) : 0ull)) +
+                      (w == 1 ? n_memb[0][cls] : 0);
+        memb[cls][r] = (uint8_t)tid;
+    }
+    // the distinct sources: hash slot of every entry (none after kM2lProbes
+    // probes: read from global memory below), then a row per used slot
+#pragma unroll
+    for (int v = 0; v < kPer; ++v) {
+        slot[v] = -1;
+        if (ent[v] < 0) continue;
+        uint32_t h = ((uint32_t)ent[v] * 2654435761u) >> 22;
+#pragma unroll 1
+        for (int t = 0; t < kM2lProbes; ++t, h = (h + 1) & (kM2lHash - 1)) {
+            const int old = atomicCAS(&ht[h], -1, ent[v]);
+            if (old == -1 || old == ent[v]) {
+                slot[v] = (int)h;
+                break;
             }
         }
     }
     __syncthreads();
-    const int n = lane % 16, kq = lane / 16;
-    const double *a1 = reinterpret_cast<const double *>(ak);
-    // orders 9 and 10: rows 16.. (at most 4) on v_mfma_f64_4x4x4f64, whose
-    // A operand holds row 16 + l % 4, column l / 16 of a 4-step, whose B
-    // operand is laid out as the 16x16x4 one (target l % 16, step row l / 16)
-    // and whose result is row 16 + l / 16 of target l % 16
-    constexpr bool LEFT = 2 * P > 16 && 2 * P <= 20;
-    v4d acc[MT];
-    double acc4 = 0.0;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[mt] = v4d{0.0, 0.0, 0.0, 0.0};
-    int o = 0;
-    for (int slot = 0; slot < 49; ++slot) {
-        const int dx = slot % 7 - 3, dy = slot / 7 - 3;
-        if (dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1) continue;
-        const int oc = o++;
-        if (oc % kM2l64Waves != w) continue;
-        const int sidx = smap[n][slot];
-        if (__ballot(sidx >= 0) == 0) continue;  // no target of the tile uses this offset
-        double b[KS];
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const int col = ks * 4 + kq;  // 2k (Re a_k) or 2k + 1 (Im a_k)
-            b[ks] = (sidx >= 0 && col < K) ? a1[(size_t)sidx * K + col] * s_sc[col >> 1] : 0.0;
-        }
-        const double *Ro = R + (size_t)oc * KS * MT * kWave + lane;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-            for (int mt = 0; mt < (LEFT ? 1 : MT); ++mt)
-                acc[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(Ro[(ks * MT + mt) * kWave], b[ks],
-                                                               acc[mt], 0, 0, 0);
-            if (LEFT)
-                acc4 = __builtin_amdgcn_mfma_f64_4x4x4f64(Ro[(ks * MT + 1) * kWave], b[ks], acc4,
-                                                          0, 0, 0);
-        }
+    for (int t = tid; t < kM2lHash; t += kM2lBlock) {
+        const bool used = ht[t] >= 0;
+        const uint64_t m = __ballot(used);
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&n_rows, __popcll(m));
+        base = __builtin_amdgcn_readfirstlane(base);
+        const int id = base + __popcll(m & (lane ? ~0ull >> (kWave - lane) : 0ull));
+        hid[t] = (uint16_t)id;
+        if (used && id < kRows) rowcell[id] = ht[t];
     }
-#pragma unroll
-    for (int mt = 0; mt < (LEFT ? 1 : MT); ++mt)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) red[w][mt * 4 + v][lane] = acc[mt][v];
-    if (LEFT) red[w][4][lane] = acc4;
     __syncthreads();
-    if (w != 0) return;
-    if (lane < cnt) bk[(size_t)(j0 + lane) * P1] = make_double2(0.0, 0.0);  // b_0 is not formed
-    double *bo = reinterpret_cast<double *>(bk);
-    if (LEFT) {
-        double sum = 0.0;
 #pragma unroll
-        for (int u = 0; u < kM2l64Waves; ++u) sum += red[u][4][lane];
-        const int row = 16 + kq;
-        if (n < cnt && row < 2 * P) {
-            const int p = row / 2 + 1;
-            bo[((size_t)(j0 + n) * P1 + p) * 2 + (row & 1)] = sum * s_sc[p];
-        }
+    for (int v = 0; v < kPer; ++v) {
+        if (ent[v] < 0) continue;
+        const int c = (tid + v * kM2lBlock) / 27;
+        // place of a source: (dx + 2 + qx) + 6 (dy + 2 + qy), with (qx, qy) the
+        // target's place in its parent
+        const int jx = (int)compact1by1(kt[v]), jy = (int)compact1by1(kt[v] >> 1);
+        const int px = (int)compact1by1(ks[v]) - jx + 2 + (jx & 1);
+        const int py = (int)compact1by1(ks[v] >> 1) - jy + 2 + (jy & 1);
+        const int id = slot[v] >= 0 ? (int)hid[slot[v]] : kRows;
+        src[c][px + 6 * py] = id < kRows ? id : -2 - ent[v];
     }
+    const int nrow = min(n_rows, kRows);
+    const int q = NQ == 1 ? only : w & 3, part = w / NQ;  // class, share
+    const int qx = q & 1, qy = q >> 1;
+    const int nm = n_memb[0][q] + n_memb[1][q];
+    const int n = lane % 16, kq = lane / 16;
+    double *bo = reinterpret_cast<double *>(bk);
+    // (uniform over the workgroup: the classes' longest member list; more than
+    // one round only in ragged trees)
+    int most = 0;
+    for (int k = 0; k < 4; ++k)
+        if (NQ == 4 || k == only) most = max(most, n_memb[0][k] + n_memb[1][k]);
+    for (int rd = 0; 16 * U * rd < most; ++rd) {
+        __syncthreads();  // (the sums of the round before share the rows' space)
+        for (int e0 = tid; e0 < nrow * AS; e0 += 4 * kM2lBlock) {
+            v2d v[4];
 #pragma unroll
-    for (int mt = 0; mt < (LEFT ? 1 : MT); ++mt) {
+            for (int t = 0; t < 4; ++t) {
+                const int e = min(e0 + t * kM2lBlock, nrow * AS - 1), r = e / AS;
+                v[t] = reinterpret_cast<const v2d *>(ak)[(size_t)rowcell[r] * AS + (e - r * AS)];
+            }
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            double sum = 0.0;
+            for (int t = 0; t < 4; ++t) {
+                const int e = min(e0 + t * kM2lBlock, nrow * AS - 1), r = e / AS, k = e - r * AS;
+                s.row[r][k] = make_double2(v[t].x * s_sc[k], v[t].y * s_sc[k]);
+            }
+        }
+        __syncthreads();
+        v4d acc[U][T16 > 0 ? T16 : 1];
+        double acc4[U][T4 > 0 ? T4 : 1];
+        int mt[U], cs[U];  // the lane's targets, and their sources at the place
+        bool use[U];       // whether any lane has one
 #pragma unroll
-            for (int u = 0; u < kM2l64Waves; ++u) sum += red[u][mt * 4 + v][lane];
-            const int row = mt * 16 + 4 * v + kq;  // Re b^_1, Im b^_1, Re b^_2, ...
-            if (n < cnt && row < 2 * P) {
-                const int p = row / 2 + 1;
-                bo[((size_t)(j0 + n) * P1 + p) * 2 + (row & 1)] = sum * s_sc[p];
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int t = 0; t < T16; ++t) acc[u][t] = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int t = 0; t < T4; ++t) acc4[u][t] = 0.0;
+            const int r = 16 * (U * rd + u) + n;
+            mt[u] = r < nm ? memb[q][r] : -1;
+        }
+        // the next place of this wavefront that a target of the round uses
+        int place = -1, turn = 0;
+        auto next = [&]() {
+#pragma unroll 1
+            for (++place; place < kM2lSlots; ++place) {
+                const int dx = place % 6 - 2 - qx, dy = place / 6 - 2 - qy;
+                if (dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1) continue;
+                if (turn++ % kShare != part) continue;
+                bool any = false;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    cs[u] = mt[u] >= 0 ? src[mt[u]][place] : -1;
+                    use[u] = __ballot(cs[u] != -1) != 0;
+                    any |= use[u];
+                }
+                if (any) return;
+            }
+        };
+        // the matrix of the place (index of its offset among the 40, dy major)
+        auto matrix = [&](double (&A)[KS * NS]) {
+            const int dx = place % 6 - 2 - qx, dy = place / 6 - 2 - qy;
+            const int oc = (dx + 3) + 7 * (dy + 3) -
+                           (dy < -1 ? 0 : dy > 1 ? 9 : 3 * (dy + 1) + (dx > 1 ? 3 : 0));
+            const double *Ro = R + (size_t)oc * KS * NS * kWave + lane;
+#pragma unroll
+            for (int t = 0; t < KS * NS; ++t) A[t] = Ro[t * kWave];
+        };
+        double A[KS * NS], nA[Sh::AHEAD ? KS * NS : 1];
+        next();
+        if (Sh::AHEAD && place < kM2lSlots) matrix(A);
+        while (place < kM2lSlots) {
+            if (!Sh::AHEAD) matrix(A);
+            int cu[U];
+            bool on[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                cu[u] = cs[u];
+                on[u] = use[u];
+            }
+            next();
+            if constexpr (Sh::AHEAD)
+                if (place < kM2lSlots) matrix(nA);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (U > 1 && !on[u]) continue;
+                // the lane's columns 8 m + 2 kq and + 1 are a_k's parts, k = 4 m + kq
+                v2d b[KP];
+#pragma unroll
+                for (int m = 0; m < KP; ++m) {
+                    b[m] = v2d{0.0, 0.0};
+                    if (cu[u] >= 0 && 4 * m + kq < K / 2)
+                        b[m] = *reinterpret_cast<const v2d *>(&s.row[cu[u]][4 * m + kq]);
+                }
+                if (__ballot(cu[u] < -1))  // rows beyond the staged ones
+#pragma unroll
+                    for (int m = 0; m < KP; ++m)
+                        if (cu[u] < -1 && 4 * m + kq < K / 2) {
+                            const double2 v = ak[(size_t)(-2 - cu[u]) * AS + 4 * m + kq];
+                            b[m] = v2d{v.x * s_sc[4 * m + kq], v.y * s_sc[4 * m + kq]};
+                        }
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    const double x = b[ks / 2][ks & 1];
+#pragma unroll
+                    for (int t = 0; t < T16; ++t)
+                        acc[u][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[ks * NS + t], x,
+                                                                         acc[u][t], 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < T4; ++t)
+                        acc4[u][t] = __builtin_amdgcn_mfma_f64_4x4x4f64(A[ks * NS + T16 + t], x,
+                                                                        acc4[u][t], 0, 0, 0);
+                }
+            }
+            if constexpr (Sh::AHEAD)
+#pragma unroll
+                for (int t = 0; t < KS * NS; ++t) A[t] = nA[t];
+        }
+        // sum of the class's wavefronts, and the store by the first of them
+        __syncthreads();
+        if (part > 0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+#pragma unroll
+                for (int t = 0; t < T16; ++t)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        s.red[NQ == 1 ? 0 : q][part - 1][u * Sh::ACC + 4 * t + v][lane] = acc[u][t][v];
+#pragma unroll
+                for (int t = 0; t < T4; ++t)
+                    s.red[NQ == 1 ? 0 : q][part - 1][u * Sh::ACC + 4 * T16 + t][lane] = acc4[u][t];
+            }
+        }
+        __syncthreads();
+        if (part == 0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int mc = mt[u];
+                auto put = [&](int row, double v, int i) {
+#pragma unroll
+                    for (int o = 0; o < kShare - 1; ++o) v += s.red[NQ == 1 ? 0 : q][o][u * Sh::ACC + i][lane];
+                    if (mc < 0 || row >= Sh::RW) return;
+                    // row: the parts of b_1, b_2, ... (type 1: b_0, b_1, ...)
+                    const int p = row / 2 + (T1 ? 0 : 1);
+                    bo[((size_t)(j0 + mc) * P1 + p) * 2 + (row & 1)] = v * s_sc[row / 2 + 1];
+                };
+#pragma unroll
+                for (int t = 0; t < T16; ++t)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) put(16 * t + 4 * v + kq, acc[u][t][v], 4 * t + v);
+#pragma unroll
+                for (int t = 0; t < T4; ++t)
+                    put(16 * T16 + 4 * t + kq, acc4[u][t], 4 * T16 + t);
+                if (!T1 && kq == 0 && mc >= 0)  // b_0 is not formed
+                    bk[(size_t)(j0 + mc) * P1] = make_double2(0.0, 0.0);
             }
         }
     }
@@ -1204,6 +1406,41 @@ __global__ void __launch_bounds__(256)
     st(bk, (size_t)j * NL + l, acc);
 }
 
+// Type-1 P2L from list 4 (k_m2l_t1's second sum) added to the list-2 sum: one
+// wavefront per target cell, skipped by a cell without a list 4; lane l forms
+// order l % NL over the particles of its group, the groups added in order.
+constexpr int kP2lT1Waves = 4;
+
+__global__ void __launch_bounds__(kWave *kP2lT1Waves)
+    k_p2l_t1(int j0, int nc, int ND, const int *l4, const uint8_t *n4, const double *c_cx,
+             const double *c_cy, const uint32_t *c_begin, const uint32_t *c_end, const double *xs,
+             const double *ys, const double *qs, double2 *bk) {
+    __shared__ double2 red[kP2lT1Waves][kWave];
+    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    const int j = j0 + blockIdx.x * kP2lT1Waves + w;
+    if (j >= nc) return;
+    const int m4 = n4[j];
+    if (m4 == 0) return;  // uniform over the wavefront
+    const int NL = ND + 1, G = kWave / NL, g = lane / NL, l = lane % NL;
+    const double cx = c_cx[j], cy = c_cy[j];
+    cd acc = {0.0, 0.0};
+    if (g < G)
+        for (int u = 0; u < m4; ++u) {
+            const int sc = l4[8 * j + u];
+            for (uint32_t i = c_begin[sc] + g; i < c_end[sc]; i += G) {
+                const cd wv = cinv(cd{xs[i] - cx, ys[i] - cy});
+                acc = csub(acc, cscale(cpowi(wv, l + 1), qs[i]));
+            }
+        }
+    st(red[w], lane, acc);
+    wave_sync();
+    if (lane < NL) {
+        cd sum = ld(bk, (size_t)j * NL + lane);
+        for (int gg = 0; gg < G; ++gg) sum = cadd(sum, ld(red[w], gg * NL + lane));
+        st(bk, (size_t)j * NL + lane, sum);
+    }
+}
+
 // Type-1 L2L for the cells of one level (>= 3; level-1 locals are zero), thread
 // per (cell, l): orders ND above 15.
 __global__ void __launch_bounds__(256)
@@ -1290,6 +1527,46 @@ static Eval64Args eval64_args(const Ctx &c, int P, bool velocity, double u_inf, 
     return A;
 }
 
+// List-2 M2L of every cell of level >= 2 on the matrix cores, order P <= 16.
+template <bool T1>
+static void m2l64_run(const Ctx &c, int P, const double *R, const double2 *ak, double2 *bk,
+                      hipStream_t s) {
+    const TreeInfo &ti = c.info;
+    M2lLevels lv{};
+    lv.maxL = ti.max_level;
+    int blocks = 0;
+    for (int L = 2; L <= ti.max_level; ++L) {
+        lv.first[L] = blocks;
+        lv.cell0[L] = (int)ti.lev_off[L];
+        blocks += div_up((long long)(ti.lev_off[L + 1] - ti.lev_off[L]), kM2lCells);
+    }
+    if (blocks == 0) return;
+    lv.first[ti.max_level + 1] = blocks;
+    lv.cell0[ti.max_level + 1] = (int)ti.lev_off[ti.max_level + 1];
+    const uint32_t *c_key = (const uint32_t *)c.c_key.p;
+    const int *l2 = (const int *)c.l2.p;
+    const uint8_t *n2 = (const uint8_t *)c.n2.p;
+    // One class per workgroup while four times the workgroups still fit the
+    // chip's 256 CUs at once (k_m2l64_mfma's comment has both sides).
+    constexpr int split = 64;
+    switch (P) {
+#define M2L64_CASE(PP)                                                                          \
+    case PP:                                                                                    \
+        if (blocks <= split)                                                                    \
+            k_m2l64_mfma<PP, T1, 1><<<4 * blocks, kM2lBlock, 0, s>>>(c.hdr_d, lv, c_key, l2,    \
+                                                                    n2, R, ak, bk);         \
+        else                                                                                    \
+            k_m2l64_mfma<PP, T1, 4><<<blocks, kM2lBlock, 0, s>>>(c.hdr_d, lv, c_key, l2, n2, R, \
+                                                                 ak, bk);                   \
+        break;
+        M2L64_CASE(1) M2L64_CASE(2) M2L64_CASE(3) M2L64_CASE(4) M2L64_CASE(5) M2L64_CASE(6)
+        M2L64_CASE(7) M2L64_CASE(8) M2L64_CASE(9) M2L64_CASE(10) M2L64_CASE(11)
+        M2L64_CASE(12) M2L64_CASE(13) M2L64_CASE(14) M2L64_CASE(15) M2L64_CASE(16)
+#undef M2L64_CASE
+        default: break;
+    }
+}
+
 // M2M from the leaves' multipoles up to level 1.
 static void m2m64_run(const TreeInfo &ti, int P, const double *tab, const uint8_t *c_flags,
                       const double *c_cx, const double *c_cy, const int *c_child, double2 *ak,
@@ -1340,24 +1617,9 @@ void fmm64_run(Ctx &c, int P, int list4_mode, int stage_mask, double *out_a, dou
     const double *t_r64 = (const double *)c.tab_r64.p;
     if (nc > j2 && P >= 1 && P < kM2lwP1 && !potential && t_r64 && c.tab_r64_p == P) {
         // list 2 on the matrix cores, then list 4 added by the wavefront kernel
-        int ntiles = 0;
-        for (int L = 2; L <= ti.max_level; ++L)
-            ntiles += (int)div_up((long long)(ti.lev_off[L + 1] - ti.lev_off[L]), 16LL);
-        const uint32_t *c_key = (const uint32_t *)c.c_key.p;
         const int *l2 = (const int *)c.l2.p;
         const uint8_t *n2 = (const uint8_t *)c.n2.p;
-        switch (P) {
-#define M2L64_CASE(PP)                                                                          \
-    case PP:                                                                                    \
-        k_m2l64_mfma<PP><<<ntiles, kWave * kM2l64Waves, 0, s>>>(c.hdr_d, ti.max_level, c_key, l2, \
-                                                              n2, t_r64, ak, bk);               \
-        break;
-            M2L64_CASE(1) M2L64_CASE(2) M2L64_CASE(3) M2L64_CASE(4) M2L64_CASE(5) M2L64_CASE(6)
-            M2L64_CASE(7) M2L64_CASE(8) M2L64_CASE(9) M2L64_CASE(10) M2L64_CASE(11)
-            M2L64_CASE(12) M2L64_CASE(13) M2L64_CASE(14) M2L64_CASE(15) M2L64_CASE(16)
-#undef M2L64_CASE
-            default: break;
-        }
+        m2l64_run<false>(c, P, t_r64, ak, bk, s);
         k_m2l64w<false, true><<<div_up(nc - j2, kM2lwWaves), kWave * kM2lwWaves, 0, s>>>(
             j2, nc, P, list4_mode, t_m2l, l2, n2, (const int *)c.l4.p,
             (const uint8_t *)c.n4.p, c_cx, c_cy, c_begin, c_end, xs, ys, qs, as, ak, bk);
@@ -1419,18 +1681,27 @@ void fmm_t1_run(Ctx &c, int ND, double *u, double *v, double u_inf, double v_inf
 
     // upward: P2M and M2M at order PM = ND - 1 (biotsavart_fmm_2d.cpp:123-188;
     // the exact shift C(p, k), the reference's bico values to rounding)
-    // (the root's local row is not read: the tree's leaves are of level >= 1)
     k_p2m64<<<div_up(nl, kP2m64Waves * kP2mLeaves), kWave * kP2m64Waves, 0, s>>>(
-        leaf_idx, nl, PM, c_flags, c_begin, c_end, c_cx, c_cy, xs, ys, qs, as, ak, bk, 1, NL);
+        leaf_idx, nl, PM, c_flags, c_begin, c_end, c_cx, c_cy, xs, ys, qs, as, ak, bk,
+        (int)ti.lev_off[2], NL);
     m2m64_run(ti, PM, (const double *)c.t1_m2m.p, c_flags, c_cx, c_cy, c_child, ak, s);
     mk.mark(3, s);
-    // M2L and P2L: every cell of level >= 1 (all of bk written)
-    const int j1 = (int)ti.lev_off[1];
-    if (nc > j1)
+    // M2L and P2L: every cell of level >= 1 (all of bk written); up to order 16
+    // list 2 on the matrix cores, then P2L added, and level 1 cleared by P2M
+    const int j1 = (int)ti.lev_off[1], j2 = (int)ti.lev_off[2];
+    const double *t_m2l = (const double *)c.t1_m2l.p;
+    const int *l2 = (const int *)c.l2.p, *l4 = (const int *)c.l4.p;
+    const uint8_t *n2 = (const uint8_t *)c.n2.p, *n4 = (const uint8_t *)c.n4.p;
+    if (ND < kTrP1) {
+        m2l64_run<true>(c, ND, (const double *)c.t1_r64.p, ak, bk, s);
+        if (nc > j2)
+            k_p2l_t1<<<div_up(nc - j2, kP2lT1Waves), kWave * kP2lT1Waves, 0, s>>>(
+                j2, nc, ND, l4, n4, c_cx, c_cy, c_begin, c_end, xs, ys, qs, bk);
+    } else if (nc > j1) {
         k_m2l_t1<<<div_up((long long)(nc - j1) * NL, 256), 256, 0, s>>>(
-            j1, nc, ND, (const double *)c.t1_m2l.p, c_level, (const int *)c.l2.p,
-            (const uint8_t *)c.n2.p, (const int *)c.l4.p, (const uint8_t *)c.n4.p, c_cx, c_cy,
-            c_begin, c_end, xs, ys, qs, ak, bk);
+            j1, nc, ND, t_m2l, c_level, l2, n2, l4, n4, c_cx, c_cy, c_begin, c_end, xs, ys, qs, ak,
+            bk);
+    }
     mk.mark(4, s);
     const double *coef = (const double *)c.t1_l2l_c.p;
     const int *expo = (const int *)c.t1_l2l_e.p;
@@ -1526,57 +1797,60 @@ void direct64(int n, const double *x, const double *y, const double *q, const ui
     VPM_LAUNCH_CHECK();
 }
 
-// Realified list-2 M2L matrices of order P for k_m2l64_mfma, one per offset
-// delta = (dx, dy) (source minus target centre over the cell side; |dx|,
-// |dy| <= 3, not both <= 1; slot order, dy major): row 2(p-1) (Re b^_p) and
-// 2(p-1)+1 (Im), p = 1..P; column 2k (Re a^_k) and 2k+1 (Im), k = 0..P;
-// entry M[p][k] = tab[p][k] delta^-(p+k), tab being the path's M2L table
-// (tab[p][0] = -1/p, tab[p][k] = -C(p+k-1, k-1) (-1)^k / k with its
-// binomials).  Stored in the A-operand lane order of v_mfma_f64_16x16x4f64:
-// R[((o KS + ks) MT + mt) 64 + l] = M[16 mt + l % 16][4 ks + l / 16].
-void fmm64_mfma_table(int P, const double *tab, std::vector<double> &R) {
-    const int P1 = P + 1, K = 2 * P1, KS = (K + 3) / 4, MT = (2 * P + 15) / 16;
-    const bool left = 2 * P > 16 && 2 * P <= 20;  // rows 16.. for the 4x4x4 instruction
-    R.assign((size_t)40 * KS * MT * kWave, 0.0);
-    std::vector<double> pwr(2 * P + 2), pwi(2 * P + 2);
-    int o = 0;
-    for (int dy = -3; dy <= 3; ++dy) {
-        for (int dx = -3; dx <= 3; ++dx) {
-            if (std::abs(dx) <= 1 && std::abs(dy) <= 1) continue;
-            const double r2 = (double)(dx * dx + dy * dy);
-            const double wr = dx / r2, wi = -dy / r2;  // 1 / delta
-            pwr[0] = 1.0;
-            pwi[0] = 0.0;
-            for (int t = 1; t <= 2 * P + 1; ++t) {
-                pwr[t] = pwr[t - 1] * wr - pwi[t - 1] * wi;
-                pwi[t] = pwr[t - 1] * wi + pwi[t - 1] * wr;
-            }
-            for (int p = 1; p <= P; ++p) {
-                for (int k = 0; k <= P; ++k) {
-                    const double T = tab[(size_t)p * P1 + k];
-                    const double Mr = T * pwr[p + k], Mi = T * pwi[p + k];
-                    const int r0 = 2 * (p - 1), c0 = 2 * k;
-                    const double val[2][2] = {{Mr, -Mi}, {Mi, Mr}};
-                    for (int a = 0; a < 2; ++a) {
-                        for (int bq = 0; bq < 2; ++bq) {
-                            const int row = r0 + a, col = c0 + bq;
-                            const int mt = row / 16, ks = col / 4;
-                            const size_t base = (((size_t)o * KS + ks) * MT + mt) * kWave;
-                            if (left && row >= 16) {
-                                // v_mfma_f64_4x4x4f64 A operand: row 16 + l % 4,
-                                // step column l / 16, the same for the four blocks
-                                for (int q = 0; q < 4; ++q)
-                                    R[base + (row - 16) + 4 * q + 16 * (col % 4)] = val[a][bq];
-                            } else {
-                                const int lane = (row % 16) + 16 * (col % 4);
-                                R[base + lane] = val[a][bq];
-                            }
-                        }
-                    }
-                }
-            }
-            ++o;
-        }
+// An entry of the list-2 M2L matrices a thread (R in k_m2l64_mfma's order: 40
+// offsets, KS steps, NS tiles, lane): tab[p][k] delta^-(p+k) as a 2 x 2 real
+// block.  (On the host the matrices and their upload cost 0.1 ms of a handle's
+// first solve.)
+__global__ void __launch_bounds__(256)
+    k_mfma_table(bool T1, int TS, int RW, int K, int KS, int T16, int NS, const double *tab,
+                 double *R) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= 40 * KS * NS * kWave) return;
+    const int lane = e % kWave, t = e / kWave % NS, ks = e / (kWave * NS) % KS;
+    // the offsets in order, dy major: 14 of dy < -1, 4 each (dx = -3, -2, 2, 3) of
+    // dy = -1, 0, 1, 14 of dy > 1
+    const int o = e / (kWave * NS * KS), i = o - 14;
+    const bool mid = i >= 0 && i < 12;
+    const int dy = mid ? i / 4 - 1 : o < 14 ? o / 7 - 3 : (o - 26) / 7 + 2;
+    const int dx = mid ? (i % 4 < 2 ? i % 4 - 3 : i % 4) : o < 14 ? o % 7 - 3 : (o - 26) % 7 - 3;
+    const int col = 8 * (ks / 2) + 2 * (lane / 16) + (ks & 1);
+    const int row = t < T16 ? 16 * t + lane % 16 : 16 * T16 + 4 * (t - T16) + lane % 4;
+    double v = 0.0;
+    if (row < RW && col < K) {
+        const int l = row / 2, k = col / 2;
+        // output order l + 1 (type 1: order l, whose power is l + 1 too)
+        const double c = tab[(size_t)(T1 ? l : l + 1) * TS + k];
+        const double r2 = (double)(dx * dx + dy * dy);
+        const cd w = {dx / r2, -dy / r2};  // 1 / delta
+        cd pw = w;
+        for (int i = 1; i < l + 1 + k; ++i) pw = cmul(pw, w);
+        // ((Re, -Im), (Im, Re))
+        v = (row & 1) == (col & 1) ? c * pw.x : (row & 1) ? c * pw.y : -(c * pw.y);
+    }
+    R[e] = v;
+}
+
+template <int P, bool T1>
+static void mfma_table(const double *tab, DBuf &buf, hipStream_t s) {
+    using Sh = M2lShape<P, T1>;
+    constexpr int total = 40 * Sh::KS * Sh::NS * kWave;
+    double *R = (double *)buf.get(total * sizeof(double));
+    k_mfma_table<<<div_up(total, 256), 256, 0, s>>>(T1, T1 ? P : P + 1, Sh::RW, Sh::K, Sh::KS,
+                                                    Sh::T16, Sh::NS, tab, R);
+    VPM_LAUNCH_CHECK();
+}
+
+void fmm64_mfma_table(int P, bool type1, const double *tab, DBuf &R, hipStream_t s) {
+    switch (P) {
+#define M2L64_CASE(PP)                                                                      \
+    case PP:                                                                                \
+        type1 ? mfma_table<PP, true>(tab, R, s) : mfma_table<PP, false>(tab, R, s);         \
+        break;
+        M2L64_CASE(1) M2L64_CASE(2) M2L64_CASE(3) M2L64_CASE(4) M2L64_CASE(5) M2L64_CASE(6)
+        M2L64_CASE(7) M2L64_CASE(8) M2L64_CASE(9) M2L64_CASE(10) M2L64_CASE(11)
+        M2L64_CASE(12) M2L64_CASE(13) M2L64_CASE(14) M2L64_CASE(15) M2L64_CASE(16)
+#undef M2L64_CASE
+        default: break;
     }
 }
 
