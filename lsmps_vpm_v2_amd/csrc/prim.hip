@@ -190,10 +190,11 @@ __global__ void __launch_bounds__(kScanBlock)
         // the producer counted the zeros of a 0/1 input: none means out and
         // compact are the identity, which the caller then uses unwritten
         __shared__ int s_skip;
-        if (threadIdx.x == 0) {
+        if (threadIdx.x < kWave) {
             unsigned long long z = 0;
-            for (int k = 0; k < skip_n; ++k) z += skip[(size_t)k * skip_stride];
-            s_skip = z == 0;
+            for (int k = threadIdx.x; k < skip_n; k += kWave) z |= skip[(size_t)k * skip_stride];
+            const uint64_t any = __ballot(z != 0);
+            if (threadIdx.x == 0) s_skip = any == 0;
         }
         __syncthreads();
         if (s_skip) {

@@ -520,31 +520,50 @@ __global__ void __launch_bounds__(kSplitBlock)
 // ---------------------------------------------------------------------------
 // 5. cells
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_lv_scan(uint32_t *blk_lv, int nbs, uint32_t *lv_tot) {
-    // exclusive scan, in place, of one row of per-block counts: rows 0 ..
-    // kMaxDepth cells per level, the next kMaxDepth + 1 rows leaves per level
-    __shared__ uint32_t sw[256 / kWave];
+// Exclusive scan, in place, of one row of per-block counts a block: rows 0 ..
+// kMaxDepth cells per level, the next kMaxDepth + 1 rows leaves per level.  Only
+// 34 blocks: bound by their loads in turn, so a row is read 4096 counts at a time
+// with the next ones under way (256 threads each reading its own stretch of the
+// row, a count after the other: 64 us at 8M particles, 13 at 2M; 19, 6).
+constexpr int kLvBlock = 1024, kLvItems = 4;
+
+__global__ void __launch_bounds__(kLvBlock) k_lv_scan(uint32_t *blk_lv, int nbs, uint32_t *lv_tot) {
+    __shared__ uint32_t sw[2][kLvBlock / kWave];
     uint32_t *row = blk_lv + (size_t)blockIdx.x * nbs;
-    const int per = (nbs + 255) / 256;
-    const int b0 = threadIdx.x * per, b1 = min(b0 + per, nbs);
-    uint32_t sum = 0;
-    for (int b = b0; b < b1; ++b) sum += row[b];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    uint32_t inc = sum;
-    for (int o = 1; o < kWave; o <<= 1) {
-        const uint32_t y = __shfl_up(inc, o, kWave);
-        if (lane >= o) inc += y;
+    uint32_t next[kLvItems];
+    auto fetch = [&](int b) {
+#pragma unroll
+        for (int k = 0; k < kLvItems; ++k) next[k] = b + k < nbs ? row[b + k] : 0u;
+    };
+    uint32_t carry = 0;
+    fetch((int)threadIdx.x * kLvItems);
+    for (int t0 = 0, turn = 0; t0 < nbs; t0 += kLvBlock * kLvItems, turn ^= 1) {
+        const int b = t0 + (int)threadIdx.x * kLvItems;
+        uint32_t v[kLvItems], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kLvItems; ++k) sum += v[k] = next[k];
+        fetch(b + kLvBlock * kLvItems);
+        uint32_t inc = sum;
+        for (int o = 1; o < kWave; o <<= 1) {
+            const uint32_t y = __shfl_up(inc, o, kWave);
+            if (lane >= o) inc += y;
+        }
+        if (lane == kWave - 1) sw[turn][w] = inc;
+        __syncthreads();  // (two rows of sums: the next turn writes the other one)
+        uint32_t run = carry + inc - sum;
+#pragma unroll
+        for (int u = 0; u < kLvBlock / kWave; ++u) {
+            run += u < w ? sw[turn][u] : 0u;
+            carry += sw[turn][u];
+        }
+#pragma unroll
+        for (int k = 0; k < kLvItems; ++k) {
+            if (b + k < nbs) row[b + k] = run;
+            run += v[k];
+        }
     }
-    if (lane == kWave - 1) sw[w] = inc;
-    __syncthreads();
-    uint32_t run = inc - sum;
-    for (int u = 0; u < w; ++u) run += sw[u];
-    for (int b = b0; b < b1; ++b) {
-        const uint32_t v = row[b];
-        row[b] = run;
-        run += v;
-    }
-    if (threadIdx.x == 255) lv_tot[blockIdx.x] = run;
+    if (threadIdx.x == 0) lv_tot[blockIdx.x] = carry;
 }
 
 // Cells in level-major order, Morton order inside a level (the order the
@@ -565,28 +584,36 @@ __global__ void __launch_bounds__(kSplitBlock)
     __shared__ uint32_t s_base[kMaxDepth + 1], s_lbase[kMaxDepth + 1];
     __shared__ uint32_t s_w[kMaxDepth + 1][kW], s_lw[kMaxDepth + 1][kW];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
-    if (tid <= kMaxDepth) {
-        uint32_t off = 1, loff = 0;  // the root is cell 0
-        for (int l = 1; l < tid; ++l) {
-            off += lv_tot[l];
-            loff += lv_tot[kL + l];
-        }
-        s_base[tid] = off + blk_lv[(size_t)tid * nbs + blockIdx.x];
-        s_lbase[tid] = loff + blk_lv[(size_t)(kL + tid) * nbs + blockIdx.x];
-    }
-    if (blockIdx.x == 0 && tid == 0) {
-        lev_level[0] = 0;
-        lev_begin[0] = 0;
-        uint32_t tot = 0, ltot = 0;
-        for (int l = 1; l <= kMaxDepth; ++l) {
-            tot += lv_tot[l];
-            ltot += lv_tot[kL + l];
-        }
-        hdr_w->n_cells_pre = tot;
-        hdr_w->n_leaves = ltot;
-    }
     const int i = blockIdx.x * kSplitBlock + tid;
     const int di = i < n ? (int)d[i] : 0, lv = i < n ? (int)leaf_lvl[i] : 0;
+    static_assert(kMaxDepth < kWave / 2, "a level per lane");
+    if (tid < kWave) {
+        // a level per lane, all its loads at once, and a scan over the lanes (a
+        // lane adding the levels before it in turn waited for each of them)
+        const int l = min(tid, kMaxDepth);
+        const uint32_t base = blk_lv[(size_t)l * nbs + blockIdx.x];
+        const uint32_t lbase = blk_lv[(size_t)(kL + l) * nbs + blockIdx.x];
+        const uint32_t c = tid >= 1 && tid <= kMaxDepth ? lv_tot[l] : 0u;
+        const uint32_t cl = tid >= 1 && tid <= kMaxDepth ? lv_tot[kL + l] : 0u;
+        uint32_t inc = c, incl = cl;
+        for (int o = 1; o <= kMaxDepth; o <<= 1) {
+            const uint32_t y = __shfl_up(inc, o, kWave), z = __shfl_up(incl, o, kWave);
+            if (tid >= o) {
+                inc += y;
+                incl += z;
+            }
+        }
+        if (tid <= kMaxDepth) {
+            s_base[tid] = 1 + inc - c + base;  // the root is cell 0
+            s_lbase[tid] = incl - cl + lbase;
+        }
+        if (blockIdx.x == 0 && tid == kMaxDepth) {
+            lev_level[0] = 0;
+            lev_begin[0] = 0;
+            hdr_w->n_cells_pre = inc;
+            hdr_w->n_leaves = incl;
+        }
+    }
     const uint64_t below = lane ? (~0ull >> (kWave - lane)) : 0ull;
     // per-wave counts start at zero: a wave visits only the levels its own
     // particles start (a few of the 16)
@@ -1246,7 +1273,7 @@ void tree_build(Ctx &c, int n, const double *x, const double *y, const Sources &
     // decision and run while the host waits for the copy and decides.
     VPM_HIP(hipMemcpyAsync(c.hdr_h, c.hdr_d, sizeof(DevHdr), hipMemcpyDeviceToHost, s));
     stream_mark(c);
-    k_lv_scan<<<2 * (kMaxDepth + 1), 256, 0, s>>>(blk_lv, nbs, lv_tot);
+    k_lv_scan<<<2 * (kMaxDepth + 1), kLvBlock, 0, s>>>(blk_lv, nbs, lv_tot);
     // emission into buffers sized from the previous build (dropped beyond)
     const size_t cap = std::max(c.cell_cap, (size_t)n / 4 + 1024);
     uint32_t *lev_level = c.lev_level.as<uint32_t>(cap), *lev_begin = c.lev_begin.as<uint32_t>(cap);
