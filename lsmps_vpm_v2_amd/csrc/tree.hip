@@ -659,36 +659,38 @@ __global__ void __launch_bounds__(kSplitBlock)
 }
 
 // End of the particle range that starts at b and shares the key prefix pre
-// (key >> sh): the first index after b whose prefix differs, or n.  The 64
-// lanes of a wavefront search together, one load per lane per round: a
-// 64-way gallop from b (strides 1, 64, 4096, ...) brackets the end, then
-// 64-way refinement narrows the bracket to one index, about 2 log64 of the
-// range in dependent loads.  b, sh and pre are wavefront-uniform and every
-// lane of the wavefront is active.
-__device__ __forceinline__ uint32_t range_end_wave(const uint32_t *key, int n, uint32_t b, int sh,
-                                                   uint32_t pre, int lane) {
+// (key >> sh): the first index after b whose prefix differs, or n.  G lanes
+// search together, one load per lane per round: a G-way gallop from b (strides
+// 64 / G, 64, 64 G, ..., so that the first round covers 64 particles) brackets
+// the end, then G-way refinement narrows the bracket to one index.  b, sh and
+// pre are uniform over the G lanes (g: lane within them, at: their first lane)
+// and all of them are active.
+template <int G>
+__device__ __forceinline__ uint32_t range_end(const uint32_t *key, int n, uint32_t b, int sh,
+                                              uint32_t pre, int g, int at) {
+    constexpr uint64_t all = G == kWave ? ~0ull : (1ull << (G % kWave)) - 1;
     // invariant: key[lo] has the prefix; the first index without it is <= hi
-    long long lo = b, hi, stride = 1;
+    long long lo = b, hi, stride = kWave / G;
     for (;;) {
-        const long long pos = lo + stride * (lane + 1);
+        const long long pos = lo + stride * (g + 1);
         bool out = pos >= n;
         if (!out) out = (key[pos] >> sh) != pre;
-        const uint64_t m = __ballot(out);
+        const uint64_t m = (__ballot(out) >> at) & all;
         if (m) {
             const int f = __ffsll((unsigned long long)m) - 1;
             hi = min((long long)n, lo + stride * (f + 1));
             lo += stride * f;
             break;
         }
-        lo += stride * kWave;
-        stride *= kWave;
+        lo += stride * G;
+        stride *= G;
     }
     while (hi - lo > 1) {
-        const long long st = (hi - lo + kWave - 1) / kWave;  // lane 63 reaches hi
-        const long long pos = lo + st * (lane + 1);
+        const long long st = (hi - lo + G - 1) / G;  // the last lane reaches hi
+        const long long pos = lo + st * (g + 1);
         bool out = pos >= hi;
         if (!out) out = (key[pos] >> sh) != pre;
-        const uint64_t m = __ballot(out);
+        const uint64_t m = (__ballot(out) >> at) & all;
         const int f = __ffsll((unsigned long long)m) - 1;
         hi = min(hi, lo + st * (f + 1));
         lo += st * f;
@@ -725,15 +727,22 @@ __device__ __forceinline__ void cell_attrs(
 
 constexpr int kCells1Block = 256;
 
+// G lanes per cell.  Bound by the search's dependent loads: a wavefront per cell
+// needs the fewest in turn and serves as long as every cell's wavefront fits the
+// chip at once (kCellsWave); larger trees take 8 lanes per cell, eight cells'
+// chains a wavefront (8 M particles, 345k cells: 146 -> 32 us, with 16 lanes 50;
+// 780k, 19k cells: 27 -> 8).
+constexpr int kCellsWave = 8192;  // 32 wavefronts on each of 256 CUs
+
+template <int G>
 __global__ void __launch_bounds__(kCells1Block)
     k_cells1(const uint32_t *lev_level, const uint32_t *lev_begin, int nc, const uint32_t *key,
              const uint32_t *A, const uint8_t *leaf_lvl, int n, const DevHdr *hdr,
              uint8_t *c_level, uint8_t *c_flags, uint32_t *c_key, uint32_t *c_begin,
              uint32_t *c_end, uint32_t *c_src, double *c_cx, double *c_cy, int *c_child,
              SplitLevels sl, DevHdr *hdr_w) {
-    // one wavefront per cell (j is wavefront-uniform)
-    const int j = blockIdx.x * (kCells1Block / kWave) + (int)(threadIdx.x / kWave);
-    const int lane = (int)(threadIdx.x & (kWave - 1));
+    const int j = blockIdx.x * (kCells1Block / G) + (int)(threadIdx.x / G);
+    const int g = (int)(threadIdx.x % G);
     // level offsets / counts and the leaf-level range for the later kernels
     if (blockIdx.x == 0 && threadIdx.x < kMaxDepth + 2) {
         hdr_w->lev_off[threadIdx.x] = sl.lev_off[threadIdx.x];
@@ -750,9 +759,9 @@ __global__ void __launch_bounds__(kCells1Block)
     if (L > 0) {
         const int sh = 32 - 2 * L;
         pre = key[b] >> sh;
-        e = range_end_wave(key, n, b, sh, pre, lane);
+        e = range_end<G>(key, n, b, sh, pre, g, (int)(threadIdx.x % kWave) - g);
     }
-    if (lane == 0)
+    if (g == 0)
         cell_attrs(j, L, b, e, pre, A, leaf_lvl, n, hdr, c_level, c_flags, c_key, c_begin, c_end,
                    c_src, c_cx, c_cy, c_child);
 }
@@ -1366,9 +1375,11 @@ void tree_build(Ctx &c, int n, const double *x, const double *y, const Sources &
     uint32_t *c_end = c.c_end.as<uint32_t>(nc), *c_src = c.c_src.as<uint32_t>(nc);
     double *c_cx = c.c_cx.as<double>(nc), *c_cy = c.c_cy.as<double>(nc);
     int *c_parent = c.c_parent.as<int>(nc), *c_child = c.c_child.as<int>(4 * (size_t)nc);
-    k_cells1<<<div_up(nc, kCells1Block / kWave), kCells1Block, 0, s>>>(lev_level, lev_begin, nc, key, A, leaf_lvl, n,
-                                             c.hdr_d, c_level, c_flags, c_key, c_begin, c_end,
-                                             c_src, c_cx, c_cy, c_child, sl, c.hdr_d);
+    const int lanes = nc <= kCellsWave ? kWave : 8;
+    (lanes == 8 ? k_cells1<8> : k_cells1<kWave>)<<<div_up(nc, kCells1Block / lanes),
+                                                     kCells1Block, 0, s>>>(
+        lev_level, lev_begin, nc, key, A, leaf_lvl, n, c.hdr_d, c_level, c_flags, c_key, c_begin,
+        c_end, c_src, c_cx, c_cy, c_child, sl, c.hdr_d);
     k_cells2<<<div_up(nc, 256), 256, 0, s>>>(c_level, c_key, nc, c.hdr_d, c_parent, c_child);
     if (tp.type1)
         k_t1_bounds<<<div_up(nc, 256), 256, 0, s>>>(c_level, c_key, nc, c.hdr_d,
