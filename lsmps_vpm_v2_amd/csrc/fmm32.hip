@@ -1104,13 +1104,17 @@ int mixed_level_setup(Ctx &c, const uint8_t *orders, LevelTab *lt, int2 *tiles,
 
 // Split levels of the three-tier passes: K = first level with >= kSubRoots
 // cells (subtrees below), T = first level with >= kTopCells cells (one
-// workgroup above T).
+// workgroup above T).  Trees of more than kSubCells cells have no subtrees: a
+// subtree's few wavefronts take its cells in turn, which costs more there than a
+// launch per level (8 M particles, 345k cells: M2M and L2L 218 + 127 us in
+// subtrees, the solve 2665 us, 2613 without; 2 M, 43k cells: 896 and 902).
+constexpr int kSubCells = 1 << 16;
 static void tier_levels(const TreeInfo &ti, int &K, int &T) {
     const int maxL = ti.max_level;
     K = T = maxL;
     for (int L = maxL; L >= 1; --L) {
         const int cnt = (int)(ti.lev_off[L + 1] - ti.lev_off[L]);
-        if (cnt >= kSubRoots) K = L;
+        if (cnt >= kSubRoots && ti.n_cells <= kSubCells) K = L;
         if (cnt >= kTopCells) T = L;
     }
     T = std::min(T, K);
