@@ -308,8 +308,8 @@ def fmm3d_section(torch, steps, warmup, cpu, accuracy):
     velocity_fmm_3d_fast) on the 778,873-particle vortex ring
     (workloads.vortex_ring) with the reference's DIM 3 options: time per
     solve with inputs in HBM, stage times and the evaluation kernel's
-    roofline from a solver that records HIP events, lane use of the
-    wavefront walk, the error against the 3-D direct sum (2,000 seeded
+    roofline from a solver that records HIP events, lane use of its
+    wavefronts, the error against the 3-D direct sum (2,000 seeded
     targets, oracle), and the oracle on the host cores (the CPU baseline,
     whose velocities also check the GPU's to 1e-10)."""
     from lsmps_vpm_v2_amd import FmmSolver, workloads
