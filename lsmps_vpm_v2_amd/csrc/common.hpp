@@ -58,6 +58,15 @@ enum DevFlag : unsigned {
     kFlagListOverflow = 8u,
     kFlagRange = 16u,
     kFlagT1Lost = 32u,  // type-1 tree: a particle outside every box of its level
+    kFlagT1Beside = 64u,  // type-1 list 2: a source box beside its target (t1_beside)
 };
+
+// A type-1 list-2 source beside its target (or at a corner of it): where two
+// neighbouring boxes' rounded bounds part by more than the box tests'
+// tolerance, the tests call them well separated.  (dx, dy): the distance of the
+// centres; side: the boxes' side.
+__host__ __device__ inline bool t1_beside(double dx, double dy, double side) {
+    return fabs(dx) < 1.5 * side && fabs(dy) < 1.5 * side;
+}
 
 }  // namespace vpm

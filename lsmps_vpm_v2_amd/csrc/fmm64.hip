@@ -1373,6 +1373,15 @@ void eval64_launch(const Eval64Args &A, hipStream_t s) {
 //       - sum_{list 4} sum_i q_i w_i^(l+1),               w_i = 1 / (z_i - zt)
 // (the reference's list 4 is always P2L from the leaf's particles).  Cells of
 // level 1 have no lists (their locals are zero, as in the reference).
+// m2l_t1_sum: order l from one source's multipoles a, d = zs - zt.
+__device__ __forceinline__ cd m2l_t1_sum(int l, int ND, const double *row, const double2 *a,
+                                         cd d) {
+    const cd w = cinv(d);
+    cd sm = cscale(ld(a, ND - 1), row[ND - 1]);
+    for (int k = ND - 2; k >= 0; --k) sm = cadd(cmul(sm, w), cscale(ld(a, k), row[k]));
+    return cmul(sm, cpowi(w, l + 1));
+}
+
 __global__ void __launch_bounds__(256)
     k_m2l_t1(int j0, int nc, int ND, const double *tab, const uint8_t *c_level, const int *l2,
              const uint8_t *n2, const int *l4, const uint8_t *n4, const double *c_cx,
@@ -1389,11 +1398,8 @@ __global__ void __launch_bounds__(256)
         const int m2 = n2[j], m4 = n4[j];
         for (int u = 0; u < m2; ++u) {
             const int sidx = l2[27 * j + u];
-            const cd w = cinv(cd{c_cx[sidx] - cx, c_cy[sidx] - cy});
-            const size_t b = (size_t)sidx * ND;
-            cd sm = cscale(ld(ak, b + ND - 1), row[ND - 1]);
-            for (int k = ND - 2; k >= 0; --k) sm = cadd(cmul(sm, w), cscale(ld(ak, b + k), row[k]));
-            acc = cadd(acc, cmul(sm, cpowi(w, l + 1)));
+            acc = cadd(acc, m2l_t1_sum(l, ND, row, ak + (size_t)sidx * ND,
+                                       cd{c_cx[sidx] - cx, c_cy[sidx] - cy}));
         }
         for (int u = 0; u < m4; ++u) {
             const int sidx = l4[8 * j + u];
@@ -1406,24 +1412,43 @@ __global__ void __launch_bounds__(256)
     st(bk, (size_t)j * NL + l, acc);
 }
 
-// Type-1 P2L from list 4 (k_m2l_t1's second sum) added to the list-2 sum: one
-// wavefront per target cell, skipped by a cell without a list 4; lane l forms
-// order l % NL over the particles of its group, the groups added in order.
+// Type-1 P2L from list 4 (k_m2l_t1's second sum) added to the list-2 sum of the
+// matrix cores, and with it the list-2 sources beside their target (t1_beside),
+// which are not among the 40 offsets of k_m2l64_mfma: the list build flags a
+// tree that has any (their pairs are a whole row of boxes; without them the
+// velocity there is of no use).  One wavefront per target cell, skipped by a
+// cell without either; lane l forms order l % NL over the particles and sources
+// of its group, the groups added in order.
 constexpr int kP2lT1Waves = 4;
 
 __global__ void __launch_bounds__(kWave *kP2lT1Waves)
-    k_p2l_t1(int j0, int nc, int ND, const int *l4, const uint8_t *n4, const double *c_cx,
-             const double *c_cy, const uint32_t *c_begin, const uint32_t *c_end, const double *xs,
-             const double *ys, const double *qs, double2 *bk) {
+    k_p2l_t1(int j0, int nc, int ND, const DevHdr *hdr, const double *tab, const uint8_t *c_level,
+             const int *l2, const uint8_t *n2, const int *l4, const uint8_t *n4,
+             const double *c_cx, const double *c_cy, const uint32_t *c_begin,
+             const uint32_t *c_end, const double *xs, const double *ys, const double *qs,
+             const double2 *ak, double2 *bk) {
     __shared__ double2 red[kP2lT1Waves][kWave];
     const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
     const int j = j0 + blockIdx.x * kP2lT1Waves + w;
     if (j >= nc) return;
     const int m4 = n4[j];
-    if (m4 == 0) return;  // uniform over the wavefront
-    const int NL = ND + 1, G = kWave / NL, g = lane / NL, l = lane % NL;
     const double cx = c_cx[j], cy = c_cy[j];
+    int s2 = -1;
+    uint64_t beside = 0;
+    if (hdr->flags & kFlagT1Beside) {
+        if (lane < (int)n2[j]) s2 = l2[27 * (size_t)j + lane];
+        const double side = ldexp(hdr->root_len, -(int)c_level[j]);
+        beside = __ballot(s2 >= 0 && t1_beside(c_cx[max(s2, 0)] - cx, c_cy[max(s2, 0)] - cy, side));
+    }
+    if (m4 == 0 && beside == 0) return;  // uniform over the wavefront
+    const int NL = ND + 1, G = kWave / NL, g = lane / NL, l = lane % NL;
     cd acc = {0.0, 0.0};
+    for (int q = 0; beside; beside &= beside - 1, ++q) {
+        const int sc = __shfl(s2, __ffsll((unsigned long long)beside) - 1, kWave);
+        if (q % G == g)
+            acc = cadd(acc, m2l_t1_sum(l, ND, tab + (size_t)l * ND, ak + (size_t)sc * ND,
+                                       cd{c_cx[sc] - cx, c_cy[sc] - cy}));
+    }
     if (g < G)
         for (int u = 0; u < m4; ++u) {
             const int sc = l4[8 * j + u];
@@ -1696,7 +1721,8 @@ void fmm_t1_run(Ctx &c, int ND, double *u, double *v, double u_inf, double v_inf
         m2l64_run<true>(c, ND, (const double *)c.t1_r64.p, ak, bk, s);
         if (nc > j2)
             k_p2l_t1<<<div_up(nc - j2, kP2lT1Waves), kWave * kP2lT1Waves, 0, s>>>(
-                j2, nc, ND, l4, n4, c_cx, c_cy, c_begin, c_end, xs, ys, qs, bk);
+                j2, nc, ND, c.hdr_d, t_m2l, c_level, l2, n2, l4, n4, c_cx, c_cy, c_begin, c_end,
+                xs, ys, qs, ak, bk);
     } else if (nc > j1) {
         k_m2l_t1<<<div_up((long long)(nc - j1) * NL, 256), 256, 0, s>>>(
             j1, nc, ND, t_m2l, c_level, l2, n2, l4, n4, c_cx, c_cy, c_begin, c_end, xs, ys, qs, ak,

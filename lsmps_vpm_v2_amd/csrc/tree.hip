@@ -954,6 +954,8 @@ __global__ void __launch_bounds__(256)
                         if (ch[q] < 0 || !(c_flags[ch[q]] & kActive)) continue;
                         keep[q] = T1 ? t1_sep(bnd[ch[q]], bnd[j])
                                      : fabs(c_cx[ch[q]] - cx) > md2 || fabs(c_cy[ch[q]] - cy) > md2;
+                        if (T1 && keep[q] && t1_beside(c_cx[ch[q]] - cx, c_cy[ch[q]] - cy, s))
+                            atomicOr(&hdr_w->flags, kFlagT1Beside);
                     }
                 } else if (fa & kLeaf) {
                     cand = A;

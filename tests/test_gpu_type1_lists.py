@@ -1,0 +1,49 @@
+"""Type-1 list-2 sources beside their target.
+
+The type-1 box tests compare bounds that are rounded level by level, against an
+absolute tolerance of 1e-15.  Where two neighbouring boxes' bounds part by more
+than that, the reference calls the boxes well separated and forms their whole
+interaction by M2L, at a distance of one box side.  On the fields here this
+holds along a whole row of level-3 boxes (a box that straddles the origin rounds
+its upper bound away from its neighbour's), which the test asserts from the
+oracle's lists; the velocity is then the oracle's only if these sources are
+summed too."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-10
+
+
+def _field(w, lo, n, seed):
+    """n particles over [lo, lo + w] x [-w / 4, w / 4], the extremes included."""
+    g = np.random.default_rng(seed)
+    x, y = g.uniform(lo, lo + w, n), g.uniform(-w / 4, w / 4, n)
+    x[:2], y[2:4] = (lo, lo + w), (-w / 4, w / 4)
+    return x, y, np.full(n, 0.01 * w), g.normal(0, 1e-3, n)
+
+
+def _beside(oracle, x, y, o):
+    """List-2 entries whose box touches the target's."""
+    t = oracle.T1Tree(x, y, o)
+    b = t.boxes()
+    return sum(max(abs(b["ix"][e] - b["ix"][k]), abs(b["iy"][e] - b["iy"][k])) <= 1
+               for k in range(t.nboxes) if b["level"][k] >= 2 for e in t.list(k, 2))
+
+
+@pytest.mark.parametrize("w, lo", [(1053.080880327208, -23.790051421199692),
+                                   (128.6897492015798, -3.1167964408478293)])
+@pytest.mark.parametrize("ndp, icutoff, mode", [(1, 2, 0), (5, 0, 0), (10, 2, 1), (12, 3, 1),
+                                                (16, 2, 0), (17, 2, 0)])
+def test_type1_sources_beside_the_target(gpu, oracle, w, lo, ndp, icutoff, mode):
+    from lsmps_vpm_v2_amd import FmmSolver
+    x, y, sz, g = _field(w, lo, 2000, 7)
+    o = oracle.t1_opts(n_s=20, lmax=6, ndp=ndp, icutoff=icutoff, l2l_mode=mode)
+    assert _beside(oracle, x, y, o) == 20
+    ur, vr = oracle.t1_velocity(x, y, sz, g, o)
+    u, v = FmmSolver(u_inf=0.0, v_inf=0.0).velocity_type1(x, y, sz, g, n_s=20, lmax=6, ndp=ndp,
+                                                          icutoff=icutoff, l2l_mode=mode)
+    err = np.max(np.hypot(u - ur, v - vr)) / np.sqrt(np.mean(ur ** 2 + vr ** 2))
+    print(f"w {w:.0f} ndp {ndp} icutoff {icutoff} l2l {mode}: {err:.2e}")
+    assert err <= TOL
