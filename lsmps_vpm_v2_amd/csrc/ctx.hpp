@@ -142,6 +142,7 @@ struct Ctx {
     // reference's box tests to them
     bool t1 = false;
     DBuf c_bnd;
+    DBuf c_res;  // type-1: a cell's centre less the grid's, in cell sides (k_t1_bounds)
     // near-field kernel of this call (0 singular, 1..3 the regularized
     // kernels of regul_func_2d) and, when regularized, the sorted sizes
     int icut = 0;

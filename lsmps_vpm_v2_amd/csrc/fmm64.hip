@@ -16,6 +16,7 @@
 // global memory.  Thread mappings: one thread per (cell, order) for the
 // translations (Horner in the translation distance, no per-thread arrays),
 // one wavefront per leaf for the evaluation.
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <vector>
@@ -480,8 +481,13 @@ __global__ void __launch_bounds__(kWave *kM2lwWaves)
 // the B operand is a source cell's a^.  Type 1 has a_0..a_{P-1} and Cauchy
 // coefficients b_0..b_P: b_l = sum_k tab[l][k] a_k (zs - zt)^-(l+1+k), 2(P+1) x
 // 2P.  The offset is exact here, where the reference forms zs - zt from rounded
-// centres: the two agree to the rounding of the centres (about 1e-16 of the
-// root box over the cell side).
+// centres.  A stored centre is off its grid position by up to 2^-53 |coordinate|
+// per rounding, which over the cell side is eps, and b by about that much: 1e-12
+// for a field 100 of its own sizes from the origin, level 7.  Type 1, whose
+// other stages use the stored centres, moves the sources' expansions to the grid
+// and the targets' back to their own centres, to first order in eps: 1e-15 of the
+// oracle (without it 6e-13 at 50 sizes from the origin, 4e-10 at 5e4, 2e-12 at
+// level 16).  Trees with a larger eps (t1_on_grid) go to k_m2l_t1.
 //
 // A workgroup takes 96 consecutive cells of one level and sorts them into the
 // four classes of a cell's place in its parent: list 2 lies within the
@@ -531,6 +537,18 @@ __device__ __forceinline__ uint32_t compact1by1(uint32_t v) {
     return v;
 }
 
+// Type 1: what the k-th scaled coefficient of a source gains when its expansion
+// is moved from the cell's own centre to the grid's, residual eps sides away:
+// k eps a^_{k-1} (the next term is of order eps^2, below 1e-20 of a^).
+__device__ __forceinline__ cd on_grid(v2d eps, v2d prev, double sc, int k) {
+    return cscale(cmul(cd{eps.x, eps.y}, cd{prev.x * sc, prev.y * sc}), (double)k);
+}
+
+// Row 2 l, 2 l + 1 of a cell's scaled result: the parts of b + 2 l.
+__device__ __forceinline__ void store_row(double *b, int row, double v, const double *sc) {
+    b[row] = v * sc[row / 2 + 1];
+}
+
 // The workgroups of each level: level L (2 .. maxL) has blocks first[L] ..
 // first[L + 1] - 1 and cells cell0[L] .. cell0[L + 1] - 1.
 struct M2lLevels {
@@ -557,13 +575,15 @@ struct M2lShape {
 template <int P, bool T1, int NQ>
 __global__ void __launch_bounds__(kM2lBlock) __attribute__((amdgpu_waves_per_eu(4, 4)))
     k_m2l64_mfma(const DevHdr *hdr, M2lLevels lv, const uint32_t *c_key, const int *l2,
-                 const uint8_t *n2, const double *R, const double2 *ak, double2 *bk) {
+                 const uint8_t *n2, const double *R, const double2 *cres, const double2 *ak,
+                 double2 *bk) {
     using Sh = M2lShape<P, T1>;
     constexpr int K = Sh::K, KP = Sh::KP, KS = Sh::KS, NS = Sh::NS, T16 = Sh::T16, T4 = Sh::T4;
     constexpr int P1 = P + 1, U = Sh::U;
     constexpr int kShare = kM2lWaves / NQ;          // wavefronts per class
     constexpr int AS = T1 ? P : P1;                 // coefficients per cell of ak
-    constexpr int kRows = kM2lRowBytes / (16 * AS); // rows that fit
+    constexpr int kFit = kM2lRowBytes / (16 * AS);  // rows that fit (a row has a hash slot)
+    constexpr int kRows = kFit < kM2lHash ? kFit : kM2lHash;
     __shared__ union {
         double2 row[kRows][AS];
         double red[NQ][kShare - 1][U * Sh::ACC][kWave];
@@ -686,16 +706,23 @@ __global__ void __launch_bounds__(kM2lBlock) __attribute__((amdgpu_waves_per_eu(
     for (int rd = 0; 16 * U * rd < most; ++rd) {
         __syncthreads();  // (the sums of the round before share the rows' space)
         for (int e0 = tid; e0 < nrow * AS; e0 += 4 * kM2lBlock) {
-            v2d v[4];
+            v2d v[4], pv[T1 ? 4 : 1], eps[T1 ? 4 : 1];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const int e = min(e0 + t * kM2lBlock, nrow * AS - 1), r = e / AS;
-                v[t] = reinterpret_cast<const v2d *>(ak)[(size_t)rowcell[r] * AS + (e - r * AS)];
+                const int e = min(e0 + t * kM2lBlock, nrow * AS - 1), r = e / AS, k = e - r * AS;
+                const v2d *row = reinterpret_cast<const v2d *>(ak) + (size_t)rowcell[r] * AS;
+                v[t] = row[k];
+                if (T1) {
+                    pv[t] = row[max(k - 1, 0)];
+                    eps[t] = reinterpret_cast<const v2d *>(cres)[rowcell[r]];
+                }
             }
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const int e = min(e0 + t * kM2lBlock, nrow * AS - 1), r = e / AS, k = e - r * AS;
-                s.row[r][k] = make_double2(v[t].x * s_sc[k], v[t].y * s_sc[k]);
+                cd a = {v[t].x * s_sc[k], v[t].y * s_sc[k]};
+                if (T1 && k > 0) a = cadd(a, on_grid(eps[T1 ? t : 0], pv[T1 ? t : 0], s_sc[k - 1], k));
+                st(s.row[r], k, a);
             }
         }
         __syncthreads();
@@ -769,8 +796,13 @@ __global__ void __launch_bounds__(kM2lBlock) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
                     for (int m = 0; m < KP; ++m)
                         if (cu[u] < -1 && 4 * m + kq < K / 2) {
-                            const double2 v = ak[(size_t)(-2 - cu[u]) * AS + 4 * m + kq];
-                            b[m] = v2d{v.x * s_sc[4 * m + kq], v.y * s_sc[4 * m + kq]};
+                            const int k = 4 * m + kq, sc = -2 - cu[u];
+                            const v2d *row = reinterpret_cast<const v2d *>(ak) + (size_t)sc * AS;
+                            cd a = {row[k].x * s_sc[k], row[k].y * s_sc[k]};
+                            if (T1 && k > 0)
+                                a = cadd(a, on_grid(reinterpret_cast<const v2d *>(cres)[sc],
+                                                    row[k - 1], s_sc[k - 1], k));
+                            b[m] = v2d{a.x, a.y};
                         }
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
@@ -809,21 +841,39 @@ __global__ void __launch_bounds__(kM2lBlock) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int mc = mt[u];
-                auto put = [&](int row, double v, int i) {
+                double(*red)[kWave] = &s.red[NQ == 1 ? 0 : q][0][u * Sh::ACC];
+                // sum i, row 4 i + kq: stored, or (type 1) left in LDS
+                auto put = [&](double v, int i) {
 #pragma unroll
-                    for (int o = 0; o < kShare - 1; ++o) v += s.red[NQ == 1 ? 0 : q][o][u * Sh::ACC + i][lane];
-                    if (mc < 0 || row >= Sh::RW) return;
-                    // row: the parts of b_1, b_2, ... (type 1: b_0, b_1, ...)
-                    const int p = row / 2 + (T1 ? 0 : 1);
-                    bo[((size_t)(j0 + mc) * P1 + p) * 2 + (row & 1)] = v * s_sc[row / 2 + 1];
+                    for (int o = 0; o < kShare - 1; ++o)
+                        v += s.red[NQ == 1 ? 0 : q][o][u * Sh::ACC + i][lane];
+                    if constexpr (T1) red[i][lane] = v;
+                    else if (mc >= 0 && 4 * i + kq < Sh::RW)
+                        store_row(bo + (size_t)(j0 + mc) * P1 * 2 + 2, 4 * i + kq, v, s_sc);
                 };
 #pragma unroll
                 for (int t = 0; t < T16; ++t)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) put(16 * t + 4 * v + kq, acc[u][t][v], 4 * t + v);
+                    for (int v = 0; v < 4; ++v) put(acc[u][t][v], 4 * t + v);
 #pragma unroll
-                for (int t = 0; t < T4; ++t)
-                    put(16 * T16 + 4 * t + kq, acc4[u][t], 4 * T16 + t);
+                for (int t = 0; t < T4; ++t) put(acc4[u][t], 4 * T16 + t);
+                if constexpr (T1) {
+                    // from the grid's centre to the target's: b_l + (l + 1) eps
+                    // b_{l+1}, whose parts are two rows on
+                    wave_sync();
+                    const double2 e = mc >= 0 ? cres[j0 + mc] : make_double2(0.0, 0.0);
+#pragma unroll 1
+                    for (int i = 0; 4 * i < Sh::RW; ++i) {
+                        const int row = 4 * i + kq, nxt = row + 2;
+                        double v = red[i][lane];
+                        if (nxt < Sh::RW)
+                            v += (double)(row / 2 + 1) *
+                                 (e.x * red[nxt / 4][16 * (nxt & 3) + n] +
+                                  (row & 1 ? e.y : -e.y) * red[nxt / 4][16 * ((nxt & 3) ^ 1) + n]);
+                        if (mc >= 0 && row < Sh::RW)
+                            store_row(bo + (size_t)(j0 + mc) * P1 * 2, row, v, s_sc);
+                    }
+                }
                 if (!T1 && kq == 0 && mc >= 0)  // b_0 is not formed
                     bk[(size_t)(j0 + mc) * P1] = make_double2(0.0, 0.0);
             }
@@ -1571,6 +1621,7 @@ static void m2l64_run(const Ctx &c, int P, const double *R, const double2 *ak, d
     const uint32_t *c_key = (const uint32_t *)c.c_key.p;
     const int *l2 = (const int *)c.l2.p;
     const uint8_t *n2 = (const uint8_t *)c.n2.p;
+    const double2 *cres = (const double2 *)c.c_res.p;  // (type 1)
     // One class per workgroup while four times the workgroups still fit the
     // chip's 256 CUs at once (k_m2l64_mfma's comment has both sides).
     constexpr int split = 64;
@@ -1579,10 +1630,10 @@ static void m2l64_run(const Ctx &c, int P, const double *R, const double2 *ak, d
     case PP:                                                                                    \
         if (blocks <= split)                                                                    \
             k_m2l64_mfma<PP, T1, 1><<<4 * blocks, kM2lBlock, 0, s>>>(c.hdr_d, lv, c_key, l2,    \
-                                                                    n2, R, ak, bk);         \
+                                                                    n2, R, cres, ak, bk);   \
         else                                                                                    \
             k_m2l64_mfma<PP, T1, 4><<<blocks, kM2lBlock, 0, s>>>(c.hdr_d, lv, c_key, l2, n2, R, \
-                                                                 ak, bk);                   \
+                                                                 cres, ak, bk);             \
         break;
         M2L64_CASE(1) M2L64_CASE(2) M2L64_CASE(3) M2L64_CASE(4) M2L64_CASE(5) M2L64_CASE(6)
         M2L64_CASE(7) M2L64_CASE(8) M2L64_CASE(9) M2L64_CASE(10) M2L64_CASE(11)
@@ -1689,6 +1740,24 @@ void fmm64_run(Ctx &c, int P, int list4_mode, int stage_mask, double *out_a, dou
     VPM_LAUNCH_CHECK();
 }
 
+// Whether the list-2 M2L of a type-1 tree may use the grid's offsets: up to order
+// 16, and while eps, the stored centres' distance from the grid in cell sides, is
+// small enough (each of max_level + 1 roundings adds up to 2^-53 of the largest
+// coordinate).  The first-order correction (k_m2l64_mfma) leaves eps times the
+// truncation error, which falls by about 2.5 per order: a velocity difference from
+// the stored-centre form of 2e-13 at order 2 and eps 1e-11, 2e-14 at order 4,
+// rounding alone from order 8 on.  The limits keep it at 1e-14 of the velocity;
+// near the origin order 10 then takes trees of up to 12 or 13 levels.
+static bool t1_on_grid(const TreeInfo &ti, int ND) {
+    if (ND >= kTrP1) return false;
+    double far = 0.0;
+    for (int d = 0; d < 2; ++d)
+        far = std::max({far, std::fabs(ti.pivot[d]), std::fabs(ti.pivot[d] + ti.root_len)});
+    const double side = std::ldexp(ti.root_len, -ti.max_level);
+    const double limit = std::min(1e-11, 1e-14 * std::pow(2.5, ND));
+    return (ti.max_level + 1) * 0x1p-53 * far <= limit * side;
+}
+
 void fmm_t1_run(Ctx &c, int ND, double *u, double *v, double u_inf, double v_inf,
                 const FmmMarks &mk) {
     hipStream_t s = c.stream;
@@ -1711,13 +1780,13 @@ void fmm_t1_run(Ctx &c, int ND, double *u, double *v, double u_inf, double v_inf
         (int)ti.lev_off[2], NL);
     m2m64_run(ti, PM, (const double *)c.t1_m2m.p, c_flags, c_cx, c_cy, c_child, ak, s);
     mk.mark(3, s);
-    // M2L and P2L: every cell of level >= 1 (all of bk written); up to order 16
+    // M2L and P2L: every cell of level >= 1 (all of bk written); on the grid
     // list 2 on the matrix cores, then P2L added, and level 1 cleared by P2M
     const int j1 = (int)ti.lev_off[1], j2 = (int)ti.lev_off[2];
     const double *t_m2l = (const double *)c.t1_m2l.p;
     const int *l2 = (const int *)c.l2.p, *l4 = (const int *)c.l4.p;
     const uint8_t *n2 = (const uint8_t *)c.n2.p, *n4 = (const uint8_t *)c.n4.p;
-    if (ND < kTrP1) {
+    if (t1_on_grid(ti, ND)) {
         m2l64_run<true>(c, ND, (const double *)c.t1_r64.p, ak, bk, s);
         if (nc > j2)
             k_p2l_t1<<<div_up(nc - j2, kP2lT1Waves), kWave * kP2lT1Waves, 0, s>>>(

@@ -801,14 +801,17 @@ __global__ void __launch_bounds__(256)
 // 179-182, 229-240): from the root (pivot, side root_len = 2 db) down the
 // cell's path with the reference's additions, in the order the reference
 // forms them (t1_path); the centre (max + min) / 2 (:201-202, 258-259)
-// replaces the pivot-based centre of cell_attrs.
+// replaces the pivot-based centre of cell_attrs.  res: how far that centre lies
+// from the exact position pivot + (i + 1/2) side, in sides, formed with the
+// rounding errors of the product and the sum (to about 2^-53 of itself).
 __global__ void __launch_bounds__(256)
     k_t1_bounds(const uint8_t *c_level, const uint32_t *c_key, int nc, const DevHdr *hdr,
-                double4 *bnd, double *c_cx, double *c_cy) {
+                double4 *bnd, double2 *res, double *c_cx, double *c_cy) {
 #pragma clang fp contract(off)
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= nc) return;
     const int L = c_level[j];
+    double off[2] = {0.0, 0.0};
     const double db = hdr->root_len / 2.0;
     double lo[2] = {hdr->pivot[0], hdr->pivot[1]}, hi[2] = {lo[0] + 2.0 * db, lo[1] + 2.0 * db};
     if (L > 0) {
@@ -827,8 +830,13 @@ __global__ void __launch_bounds__(256)
             }
             lo[d] = l;
             hi[d] = h;
+            const double side = cell_len(hdr->root_len, L), f = (double)ix[d] + 0.5;
+            const double p = f * side, pe = fma(f, side, -p);
+            const double g = o + p, t = g - o, ge = (o - (g - t)) + (p - t);
+            off[d] = (((h + l) / 2.0 - g) - (ge + pe)) / side;
         }
     }
+    res[j] = make_double2(off[0], off[1]);
     bnd[j] = make_double4(lo[0], hi[0], lo[1], hi[1]);
     c_cx[j] = (hi[0] + lo[0]) / 2.0;
     c_cy[j] = (hi[1] + lo[1]) / 2.0;
@@ -1385,7 +1393,8 @@ void tree_build(Ctx &c, int n, const double *x, const double *y, const Sources &
     k_cells2<<<div_up(nc, 256), 256, 0, s>>>(c_level, c_key, nc, c.hdr_d, c_parent, c_child);
     if (tp.type1)
         k_t1_bounds<<<div_up(nc, 256), 256, 0, s>>>(c_level, c_key, nc, c.hdr_d,
-                                                    c.c_bnd.as<double4>(nc), c_cx, c_cy);
+                                                    c.c_bnd.as<double4>(nc),
+                                                    c.c_res.as<double2>(nc), c_cx, c_cy);
     VPM_LAUNCH_CHECK();
 }
 

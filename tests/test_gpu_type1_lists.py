@@ -1,13 +1,18 @@
-"""Type-1 list-2 sources beside their target.
+"""Type-1 list-2 M2L where the rounding of the box bounds shows.
 
-The type-1 box tests compare bounds that are rounded level by level, against an
+Sources beside their target: the type-1 box tests compare bounds that are rounded level by level, against an
 absolute tolerance of 1e-15.  Where two neighbouring boxes' bounds part by more
 than that, the reference calls the boxes well separated and forms their whole
 interaction by M2L, at a distance of one box side.  On the fields here this
 holds along a whole row of level-3 boxes (a box that straddles the origin rounds
 its upper bound away from its neighbour's), which the test asserts from the
 oracle's lists; the velocity is then the oracle's only if these sources are
-summed too."""
+summed too.
+
+Centres off the grid: the centres are rounded too, to 2^-53 of the coordinates,
+which deep in a tree or far from the origin is a good part of a box side.  P2M,
+M2M, L2L and L2P use the rounded centres, so the rounding cancels in the velocity
+if M2L uses them as well."""
 import numpy as np
 import pytest
 
@@ -47,3 +52,46 @@ def test_type1_sources_beside_the_target(gpu, oracle, w, lo, ndp, icutoff, mode)
     err = np.max(np.hypot(u - ur, v - vr)) / np.sqrt(np.mean(ur ** 2 + vr ** 2))
     print(f"w {w:.0f} ndp {ndp} icutoff {icutoff} l2l {mode}: {err:.2e}")
     assert err <= TOL
+
+
+# An M2L from grid offsets alone differs from the oracle by eps = 2^-53
+# |coordinate| / side: 6e-14 (rel-L2) at offset 1e3, 6e-11 at 1e6, 3e-13 at level
+# 16.  The stored-centre form differs by the rounding of sums of some hundred
+# terms, 3e-15 at most on these fields; 1e-14 is 45 units of the last place.
+REL = 1e-14
+
+
+def _rel(u, v, ur, vr):
+    return float(np.sqrt(np.mean((u - ur) ** 2 + (v - vr) ** 2) / np.mean(ur ** 2 + vr ** 2)))
+
+
+def _check(oracle, x, y, sz, g, n_s, lmax, ndp, icutoff):
+    from lsmps_vpm_v2_amd import FmmSolver
+    ur, vr = oracle.t1_velocity(x, y, sz, g, oracle.t1_opts(n_s=n_s, lmax=lmax, ndp=ndp,
+                                                            icutoff=icutoff, l2l_mode=0))
+    u, v = FmmSolver(u_inf=0.0, v_inf=0.0).velocity_type1(x, y, sz, g, n_s=n_s, lmax=lmax,
+                                                          ndp=ndp, icutoff=icutoff, l2l_mode=0)
+    err = _rel(u, v, ur, vr)
+    print(f"lmax {lmax} ndp {ndp}: {err:.2e}")
+    assert err <= REL
+
+
+@pytest.mark.parametrize("ndp", [2, 4, 6, 8, 10, 13, 16])
+@pytest.mark.parametrize("offset", [0.0, 60.0, 1e3, 1e4, 1e6])
+def test_type1_far_from_the_origin(gpu, oracle, offset, ndp):
+    from lsmps_vpm_v2_amd import workloads as W
+    c = W.random_clusters(7000, seed=51)
+    for lmax in (7, 10):
+        _check(oracle, c["x"] * 11 + offset, c["y"] * 11 - offset, np.full(7000, 0.04), c["q"],
+               8, lmax, ndp, 2)
+
+
+@pytest.mark.parametrize("ndp", [2, 4, 10, 16])
+@pytest.mark.parametrize("lmax", [12, 13, 14, 16])
+def test_type1_deep_trees(gpu, oracle, lmax, ndp):
+    """Particles crowding towards a point, down to the deepest level."""
+    g = np.random.default_rng(11)
+    n = 9000
+    r, th = 10.0 ** g.uniform(-6, 0, n), g.uniform(0, 2 * np.pi, n)
+    x, y = r * np.cos(th) + 0.3, r * np.sin(th) - 0.2
+    _check(oracle, x, y, np.full(n, 1e-4), g.normal(0, 1e-3, n), 10, lmax, ndp, 2)
