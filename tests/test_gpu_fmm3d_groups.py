@@ -56,3 +56,39 @@ def test_inactive_source_without_finite_strength(gpu):
     got, ref = _check(cols, act, type=2)
     assert 0 < np.isnan(ref).any(1).sum() < 2000
     assert np.array_equal(np.isnan(got), np.isnan(ref))
+
+
+@pytest.mark.parametrize("n", [5, 8192, 8193, 20001])
+def test_work_counts(gpu, n):
+    """Pairs and far-cell terms as a walk over the oracle's tree counts them, on
+    both sides of the 1024 records (of 8 targets) one workgroup adds up, and the
+    same again for a second call on the handle."""
+    from lsmps_vpm_v2_amd import FmmSolver
+    from oracle import oracle as O
+    cols, act = _field(n, n)
+    act[:] = 1
+    o = dict(crit_num=30, support=2.0)
+    t = O.O3Tree(*cols[:3], act, O.o3_opts(**o))
+    kids = {}
+    for c in range(len(t.level)):
+        kids.setdefault((int(t.level[c]) - 1, int(t.key[c]) >> 3), []).append(c)
+    p = np.stack(cols[:3], 1)
+    pairs = far = 0
+    walk = [(c, np.arange(n)) for c in range(len(t.level)) if t.level[c] == 1 and not t.leaf[c]]
+    while walk:
+        c, tgt = walk.pop()
+        for k in kids.get((int(t.level[c]), int(t.key[c])), []):
+            r2 = ((p[tgt] - t.centre[k]) ** 2).sum(1)
+            near = tgt[~(r2 > (o["support"] * t.size[k]) ** 2)]
+            far += len(tgt) - len(near)
+            if t.leaf[k]:
+                own = t.particles(k)
+                pairs += len(near) * len(own) - len(np.intersect1d(near, own))
+            else:
+                walk.append((k, near))
+    s = FmmSolver()
+    for _ in range(2):
+        s.velocity3d(*cols, act, **o)
+        st = s.fmm3d_stats()
+        print(f"work n={n}: {st['pairs']} pairs, {st['m2p']} far", flush=True)
+        assert (st["pairs"], st["m2p"]) == (pairs, far)
