@@ -898,7 +898,9 @@ struct Acc3 {
     double u[kGrp], v[kGrp], w[kGrp];
 };
 
-// The far cells fq[base .. base + cnt) (cnt <= 64).
+// The far cells fq[base .. base + cnt) (cnt <= 64).  A masked term is multiplied by
+// zero; with STRICT (near_terms) it is left out, whatever the cell's coefficients.
+template <bool STRICT>
 __device__ __forceinline__ void eval_far(EvalLds &l, int base, int cnt, int lane,
                                          const double *__restrict__ far, const double (&xt)[kGrp],
                                          const double (&yt)[kGrp], const double (&zt)[kGrp],
@@ -935,7 +937,15 @@ __device__ __forceinline__ void eval_far(EvalLds &l, int base, int cnt, int lane
     const double cx = fb[5].y, cy = fb[6].x, cz = fb[6].y;
 #pragma unroll
     for (int t = 0; t < kGrp; ++t) {
-        far_term(fc, xt[t] - cx, yt[t] - cy, zt[t] - cz, m, t, acc.u[t], acc.v[t], acc.w[t]);
+        if (STRICT) {
+            double u = 0.0, v = 0.0, w = 0.0;
+            far_term(fc, xt[t] - cx, yt[t] - cy, zt[t] - cz, m, t, u, v, w);
+            acc.u[t] += masked(u, m, t);
+            acc.v[t] += masked(v, m, t);
+            acc.w[t] += masked(w, m, t);
+        } else {
+            far_term(fc, xt[t] - cx, yt[t] - cy, zt[t] - cz, m, t, acc.u[t], acc.v[t], acc.w[t]);
+        }
         __builtin_amdgcn_sched_barrier(0);  // one target's temporaries at a time
     }
 }
@@ -1139,7 +1149,7 @@ __global__ void __launch_bounds__(kEvalWaves *kWave) __attribute__((amdgpu_waves
         if (nf >= kWave || (done && nf > 0)) {
             const int cnt = min(nf, kWave);
             nf -= cnt;
-            eval_far(l, nf, cnt, lane, far, xt, yt, zt, acc);
+            eval_far<STRICT>(l, nf, cnt, lane, far, xt, yt, zt, acc);
             wfar += kGrp;
         }
         done = done && nf == 0;

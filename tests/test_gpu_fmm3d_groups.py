@@ -58,6 +58,26 @@ def test_inactive_source_without_finite_strength(gpu):
     assert np.array_equal(np.isnan(got), np.isnan(ref))
 
 
+@pytest.mark.parametrize("type", [1, 2])
+def test_infinite_strength(gpu, type):
+    """An infinite x vorticity leaves u as it is; v and w become infinite where the
+    particle is summed directly and NaN or infinite where a cell's moments carry it,
+    target by target as in the oracle; the particle itself stays finite."""
+    cols, act = _field(4000, 5)
+    k = 3000
+    act[k] = 1
+    cols[4][k] = np.inf
+    got, ref = _check(cols, act, type=type)
+    sc = np.sqrt(np.mean((ref[:, 0] - 1.0) ** 2))
+    assert np.max(np.abs(got[:, 0] - ref[:, 0])) <= TOL * sc
+    assert np.max(np.abs(got[k] - ref[k])) <= TOL * sc
+    for c in (1, 2):
+        inf = np.isinf(ref[:, c])
+        assert inf.sum() > 50
+        assert np.array_equal(np.isnan(got[:, c]), np.isnan(ref[:, c]))
+        assert np.array_equal(got[inf, c], ref[inf, c])
+
+
 @pytest.mark.parametrize("n", [5, 8192, 8193, 20001])
 def test_work_counts(gpu, n):
     """Pairs and far-cell terms as a walk over the oracle's tree counts them, on
