@@ -1173,8 +1173,10 @@ __device__ __forceinline__ bool eval64_leaf(const Eval64Args &A, int t, int j, i
     const bool own = (A.c_flags[j] & kActive) != 0;  // the leaf is in its own list 1
     const double lcx = A.c_cx[j], lcy = A.c_cy[j];
     const uint32_t a1 = A.off1[t], z1 = A.off1[t + 1], a3 = A.off3[t], z3 = A.off3[t + 1];
-    // padding source: zero strength, outside the root box
+    // padding source: zero strength, outside the root box, of a size at which any
+    // target's factor is finite (a zero size would leave 0 NaN)
     const double padx = lcx + 4.0 * A.hdr->root_len;
+    const double pads2 = A.hdr->root_len * A.hdr->root_len;
     if (wi == 0)
         for (int k = lane; k < P1; k += kWave) l.b[k] = A.bk[(size_t)j * P1 + k];
     bool odd = false;
@@ -1206,9 +1208,9 @@ __device__ __forceinline__ bool eval64_leaf(const Eval64Args &A, int t, int j, i
                                        : make_double2(padx, lcy);
                     l.q[r] = r < fill ? A.qs[src] : 0.0;
                     if (kSized) {
-                        const double s2 = A.ss[src] * A.ss[src];
+                        const double s2 = r < fill ? A.ss[src] * A.ss[src] : pads2;
                         l.s2[r] = s2;
-                        odd_s |= wild(s2);
+                        odd_s |= r < fill && wild(s2);
                     }
                 }
                 const bool tame = tame_t && (!kSized || __ballot(odd_s) == 0);
@@ -1260,9 +1262,9 @@ __device__ __forceinline__ bool eval64_leaf(const Eval64Args &A, int t, int j, i
                                        : make_double2(padx, lcy);
                     l.q[r] = r < fill ? A.qs[src] : 0.0;
                     if (kSized) {
-                        const double s2 = A.ss[src] * A.ss[src];
+                        const double s2 = r < fill ? A.ss[src] * A.ss[src] : pads2;
                         l.s2[r] = s2;
-                        odd_s |= wild(s2);
+                        odd_s |= r < fill && wild(s2);
                     }
                 }
                 const bool tame = tame_t && (!kSized || __ballot(odd_s) == 0);

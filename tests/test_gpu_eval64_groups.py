@@ -59,3 +59,24 @@ def test_sizes_of_zero(gpu, oracle):
     u, v = FmmSolver(icutoff=2).velocity(*a)
     u0, v0 = oracle.velocity(*a, oracle.opts(icutoff=2), 1.0, 0.0)
     assert np.isfinite(u).all() and _rel(u, u0) <= TOL and _rel(v, v0) <= TOL
+
+
+@pytest.mark.parametrize("n,cap", [(5, 7), (700, 9), (60001, 8)])
+@pytest.mark.parametrize("icut", [1, 2, 3])
+def test_single_size_of_zero(gpu, oracle, icut, n, cap):
+    """A point particle among blobs, the last of its leaf (of a source round, whose
+    padding follows it): every velocity is finite."""
+    f = W.random_clusters(n, seed=cap, active_frac=1.0)
+    solver = FmmSolver(max_par=cap, max_src=cap, icutoff=icut)
+    a = [f["x"], f["y"], f["s"].copy(), f["omega"], f["active"]]
+    solver.velocity(*a)
+    _, poff, pidx = solver.tree_leaves(n)
+    last = pidx[poff[1:] - 1]
+    for k in last[:: max(1, len(last) // 3)]:
+        print(f"point particle {k} of {n}, icutoff={icut}", flush=True)
+        a[2] = f["s"].copy()
+        a[2][k] = 0.0
+        u, v = solver.velocity(*a)
+        u0, v0 = oracle.velocity(*a, oracle.opts(icutoff=icut, max_par=cap, max_src=cap), 1.0, 0.0)
+        assert bool(np.isfinite(u0).all()) and bool(np.isfinite(u).all())
+        assert _rel(u, u0) <= TOL and _rel(v, v0) <= TOL
