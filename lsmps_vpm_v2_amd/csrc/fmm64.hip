@@ -1758,13 +1758,18 @@ void fmm64_run(Ctx &c, int P, int list4_mode, int stage_mask, double *out_a, dou
 // truncation error, which falls by about 2.5 per order: a velocity difference from
 // the stored-centre form of 2e-13 at order 2 and eps 1e-11, 2e-14 at order 4,
 // rounding alone from order 8 on.  The limits keep it at 1e-14 of the velocity;
-// near the origin order 10 then takes trees of up to 12 or 13 levels.
+// near the origin order 10 then takes trees of up to 12 or 13 levels.  (A box of side
+// 1e-30 has no list 2 under the box tests' tolerance, and k_m2l_t1 forms no power.)
 static bool t1_on_grid(const TreeInfo &ti, int ND) {
     if (ND >= kTrP1) return false;
     double far = 0.0;
     for (int d = 0; d < 2; ++d)
         far = std::max({far, std::fabs(ti.pivot[d]), std::fabs(ti.pivot[d] + ti.root_len)});
     const double side = std::ldexp(ti.root_len, -ti.max_level);
+    // the scaled coefficients' powers of a side of any level stay inside the range
+    const double range = 290.0 / (ND + 1);
+    if (!(std::fabs(std::log10(side)) < range && std::fabs(std::log10(ti.root_len)) < range))
+        return false;
     const double limit = std::min(1e-11, 1e-14 * std::pow(2.5, ND));
     return (ti.max_level + 1) * 0x1p-53 * far <= limit * side;
 }

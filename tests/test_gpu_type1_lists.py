@@ -95,3 +95,26 @@ def test_type1_deep_trees(gpu, oracle, lmax, ndp):
     r, th = 10.0 ** g.uniform(-6, 0, n), g.uniform(0, 2 * np.pi, n)
     x, y = r * np.cos(th) + 0.3, r * np.sin(th) - 0.2
     _check(oracle, x, y, np.full(n, 1e-4), g.normal(0, 1e-3, n), 10, lmax, ndp, 2)
+
+
+@pytest.mark.parametrize("ndp", [4, 10, 16])
+@pytest.mark.parametrize("scale", [1e-100, 1e-30, 1e6, 1e12])
+def test_type1_scales(gpu, oracle, scale, ndp):
+    """Fields of any size.  Below the box tests' tolerance no boxes are well
+    separated (the oracle refuses such a field): only near pairs are summed, the
+    same at every order."""
+    from lsmps_vpm_v2_amd import FmmSolver
+    g = np.random.default_rng(3)
+    x, y, gz = scale * g.random(3000), scale * g.random(3000), scale * g.standard_normal(3000)
+    sz = np.full(3000, 0.01 * scale)
+    s = FmmSolver(u_inf=0.0, v_inf=0.0)
+    kw = dict(n_s=20, lmax=8, icutoff=2, l2l_mode=0)
+    u, v = s.velocity_type1(x, y, sz, gz, ndp=ndp, **kw)
+    if scale < 1e-20:
+        ur, vr = s.velocity_type1(x, y, sz, gz, ndp=20, **kw)
+        assert np.isfinite(ur).all()
+    else:
+        ur, vr = oracle.t1_velocity(x, y, sz, gz, oracle.t1_opts(ndp=ndp, **kw))
+    err = _rel(u, v, ur, vr)
+    print(f"scale {scale:g} ndp {ndp}: {err:.2e}")
+    assert err <= TOL
