@@ -98,7 +98,7 @@ def test_type1_deep_trees(gpu, oracle, lmax, ndp):
 
 
 @pytest.mark.parametrize("ndp", [4, 10, 16])
-@pytest.mark.parametrize("scale", [1e-100, 1e-30, 1e6, 1e12])
+@pytest.mark.parametrize("scale", [1e-100, 1e-30, 1e6, 1e9])
 def test_type1_scales(gpu, oracle, scale, ndp):
     """Fields of any size.  Below the box tests' tolerance no boxes are well
     separated (the oracle refuses such a field): only near pairs are summed, the
