@@ -52,7 +52,10 @@ namespace {
 
 constexpr int kHalf = kFmm3Depth / 2;  // levels per key word
 constexpr unsigned kF3NonFinite = 1u, kF3Deeper = 2u, kF3Depth = 4u, kF3Degenerate = 8u,
-                   kF3OddStrength = 16u;  // a strength that is not finite
+                   kF3OddStrength = 16u;  // a strength beyond kF3MaxStrength, or not finite
+// Up to here a strength times a distance is finite, whatever the target: a pair or
+// term of it can be masked by a factor of zero.
+constexpr double kF3MaxStrength = 1e150;
 constexpr int kMomStride = 32;
 
 struct __align__(16) Par3 {
@@ -319,7 +322,8 @@ __global__ void __launch_bounds__(256)
     }
     r.act = a ? 1.0 : 0.0;
     r.pad = 0.0;
-    const uint64_t odd = __ballot(!(isfinite(r.ax) && isfinite(r.ay) && isfinite(r.az)));
+    auto tame = [](double a) { return fabs(a) <= kF3MaxStrength; };
+    const uint64_t odd = __ballot(!(tame(r.ax) && tame(r.ay) && tame(r.az)));
     if (odd && (threadIdx.x & (kWave - 1)) == (uint32_t)(__ffsll((unsigned long long)odd) - 1))
         atomicOr(&h->flags, kF3OddStrength);
     P[j] = r;
@@ -951,8 +955,7 @@ __device__ __forceinline__ void eval_far(EvalLds &l, int base, int cnt, int lane
 }
 
 // The pairs of the lane's source q with the targets of m.  A masked pair is
-// multiplied by zero; with STRICT its strength is masked too, for fields with
-// a strength that is not finite.
+// multiplied by zero; with STRICT its strength is masked too (k3_eval).
 template <bool STRICT>
 __device__ __forceinline__ void near_terms(const Src3 &q, uint32_t m, const double (&xt)[kGrp],
                                            const double (&yt)[kGrp], const double (&zt)[kGrp],
@@ -1045,9 +1048,9 @@ __device__ __forceinline__ void eval_leaves(EvalLds &l, int base, int cnt, int l
     } while (more);
 }
 
-// STRICT for fields with a strength that is not finite: such a source may reach
-// only the targets that take it (inactive particles of type 2 are summed by
-// near targets alone).
+// STRICT for fields with a strength that is not finite, or whose product with a
+// distance may not be: such a source may reach only the targets that take it
+// (inactive particles of type 2 are summed by near targets alone).
 template <bool STRICT>
 __global__ void __launch_bounds__(kEvalWaves *kWave) __attribute__((amdgpu_waves_per_eu(3, 3)))
     k3_eval(const Cell3 *__restrict__ cells, int ncell, const int *__restrict__ kids,

@@ -112,3 +112,26 @@ def test_work_counts(gpu, n):
         st = s.fmm3d_stats()
         print(f"work n={n}: {st['pairs']} pairs, {st['m2p']} far", flush=True)
         assert (st["pairs"], st["m2p"]) == (pairs, far)
+
+
+def test_strength_near_the_range(gpu):
+    """A strength whose product with the distance of a target overflows, where only
+    nearer targets sum it directly and the farther ones by its cell's moments:
+    everything stays finite."""
+    from lsmps_vpm_v2_amd import FmmSolver
+    from oracle import oracle as O
+    g = np.random.default_rng(2)
+    n = 400
+    p = g.uniform(-8.0, 8.0, (3, n))
+    a = 1e290 * g.standard_normal((3, n))
+    k = np.argmax(p.sum(0))
+    a[:, k] = 0.0
+    a[0, k] = 1.6e307
+    act = np.ones(n, np.uint8)
+    ref = np.stack(O.o3_velocity_alpha(*p, *a, act, O.o3_opts()), 1)
+    assert np.isfinite(ref).all()
+    got = np.stack(FmmSolver(u_inf=0.0, v_inf=0.0).velocity3d_alpha(*p, *a, act), 1)
+    assert np.isfinite(got).all()
+    # (scaled: the squares overflow)
+    err = np.linalg.norm(got / 1e300 - ref / 1e300, axis=1)
+    assert np.max(err) <= TOL * np.sqrt(np.mean(((ref / 1e300) ** 2).sum(1)))
