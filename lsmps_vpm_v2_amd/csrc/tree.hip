@@ -1135,7 +1135,10 @@ __global__ void __launch_bounds__(256)
                 stk[sp++][me] = A;
                 while (sp > 0) {
                     const int B = stk[--sp][me];
-                    const double adj = ((s + (cell_len(R, c_level[B]) / 2.0)) / 2.0) + kListEps;
+                    // (type 1: a quarter of a child's side apart at most, whatever the
+                    // coordinates' rounding; the box tests decide)
+                    const double cl = cell_len(R, c_level[B]) / 2.0;
+                    const double adj = ((s + cl) / 2.0) + (T1 ? fmax(0.25 * cl, kListEps) : kListEps);
                     const bool tb = !T1 || t1_touch(bnd[B], bj);
                     int chq[4];
 #pragma unroll
