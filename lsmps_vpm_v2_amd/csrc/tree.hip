@@ -1460,7 +1460,10 @@ void tree_lists_end(Ctx &c) {
     // direction) and the finer adjacent leaves; each finer leaf is adjacent to
     // at most 8 coarser leaves, so sum |list 1| <= 17 nl.  A cell is in the
     // list 3 of leaves coarser than it and adjacent to its parent: at most 8,
-    // so sum |list 3| <= 8 nc.  The fill pass checks both anyway.
+    // so sum |list 3| <= 8 nc.  That holds while the cells are larger than the
+    // tolerance kListEps; where they are not, a leaf is adjacent to everything below
+    // its neighbours.  So the fill pass checks both, the readers stop at the
+    // capacities (their results are then dropped), and tree_lists_absorb refuses.
     ti.cap1 = 17 * (size_t)nl + 1;
     ti.cap3 = 8 * (size_t)nc + 1;
     int *l1 = c.l1.as<int>(ti.cap1), *l3 = c.l3.as<int>(ti.cap3);
@@ -1474,6 +1477,8 @@ void tree_lists_end(Ctx &c) {
 void tree_lists_absorb(Ctx &c) {
     const DevHdr &hh = *c.hdr_h;
     TreeInfo &ti = c.info;
+    if ((hh.flags & kFlagListOverflow) || (size_t)hh.tot1 >= ti.cap1 || (size_t)hh.tot3 >= ti.cap3)
+        ti.n_cells = 0;  // no lists to inspect
     check_flags(hh);
     if ((int)hh.n_leaves != ti.n_leaves || (int)hh.n_cells_pre + 1 != ti.n_cells)
         throw Error(kInternal, "cell or leaf count of the cell build disagrees with the leaf split");
