@@ -67,8 +67,8 @@ __device__ __forceinline__ void wave_sync() {
 // P2M (fmm2D.cpp:237-284, with the sign and 1/p folded into the translation
 // tables): four leaves per wavefront, 16 lanes each.  A leaf's lanes take 16
 // of its particles at a time, and lane i stages q z^b (b = 0..3) and z^(4a)
-// (a = 0..3) of its particle, z from the leaf's centre, zero strength for
-// inactive particles and leaves; lane r then adds its own order p = 4a + b as
+// (a = 0..3) of its particle, z from the leaf's centre (zero for a particle without
+// strength or inactive, whatever its powers would be); lane r then adds its own order p = 4a + b as
 // one complex product per particle, four FMAs from two LDS reads, with no
 // cross-lane reduction.  Orders beyond 15 take further chunks of 16.  (Forming
 // z^p afresh per particle and order took about 40 operations: 37 -> 13 us at
@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(kWave *kP2m64Waves)
             const uint32_t i = in ? b + base + (uint32_t)r : 0u;
             const uint8_t ai = as[i];  // (the four loads in one round)
             const double xi = xs[i], yi = ys[i], qi = qs[i];
-            const bool src = in && ai != 0;
+            const bool src = in && ai != 0 && qi != 0.0;
             const cd z = {src ? xi - cx : 0.0, src ? yi - cy : 0.0};
             const double q = src ? qi : 0.0;
             const cd z2 = cmul(z, z), z4 = cmul(z2, z2), z8 = cmul(z4, z4);

@@ -169,3 +169,24 @@ def test_one_level_tree_after_a_large_solve_on_one_handle(gpu, oracle, precision
         ex0, ey0 = oracle.direct_field(x, y, q)
         tol = 1e-10 if precision == "fp64" else 5e-6 + 2 * _fp32_floor(oracle, x, y, q, a)
         _check(ex, ey, ex0, ey0, tol)
+
+
+@pytest.mark.parametrize("p", [3, 10, 16, 20])
+@pytest.mark.parametrize("scale", [1.0, 1e100])
+def test_no_strength_at_all(gpu, scale, p):
+    """A field without strength has no velocity of its own and no potential, also
+    where the powers of its coordinates overflow."""
+    from lsmps_vpm_v2_amd import FmmSolver
+    g = np.random.default_rng(4)
+    n = 2000
+    x, y, s = scale * g.random(n), scale * g.random(n), np.full(n, 0.01 * scale)
+    z, a = np.zeros(n), np.ones(n, np.uint8)
+    # (two levels: deeper, the lists' absolute tolerance is lost in such coordinates)
+    kw = dict(p=p, max_par=9, max_src=9, max_level=2, u_inf=0.5, v_inf=-0.25)
+    for icut in (0, 2):
+        u, v = FmmSolver(icutoff=icut, **kw).velocity(x, y, s, z, a)
+        assert np.all(u == 0.5) and np.all(v == -0.25)
+    solver = FmmSolver(**kw)
+    assert np.all(solver.potential(x, y, z, a) == 0.0)
+    u, v = solver.velocity_type1(x, y, s, z, n_s=9, lmax=2, ndp=p)
+    assert np.all(u == 0.5) and np.all(v == -0.25)
