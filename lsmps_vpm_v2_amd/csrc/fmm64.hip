@@ -13,9 +13,11 @@
 //
 // The per-order coefficient tables (M2L including the reference's int32
 // binomials in parity mode) are built on the host (api.cpp) and read from
-// global memory.  Thread mappings: one thread per (cell, order) for the
-// translations (Horner in the translation distance, no per-thread arrays),
-// one wavefront per leaf for the evaluation.
+// global memory.  Thread mappings, orders up to 16: 16 lanes per leaf (P2M), a
+// workgroup per subtree of three levels (M2M, L2L), the matrix cores (list-2 M2L;
+// the potential and list 4 a wavefront per cell), one or four wavefronts per leaf
+// (evaluation, any order).  Above order 16 the translations take one thread per
+// (cell, order): Horner in the translation distance, no per-thread arrays.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -304,10 +306,8 @@ __device__ __forceinline__ cd clog(cd z) { return {log(hypot(z.x, z.y)), atan2(z
 // w = 1/(zs - zt), so b_p = w^p sum_k tab[p][k] a_k w^k (Horner in w).  With
 // POT the order-0 row of the potential is formed too (fmm2D.cpp:463-467,
 // 504-508): b_0 = a_0 log(z_t - z_s) - sum_{k>=1} a_k (-1)^k / k w^k, and by
-// P2L b_0 += q log(z_t - z_i) (:540).  With PT > 0 (orders P <= PT) a
-// source's coefficients are loaded into registers at once before the Horner
-// sweep, rather than one dependent load per step.
-template <bool POT, int PT>
+// P2L b_0 += q log(z_t - z_i) (:540).  Orders above 16.
+template <bool POT>
 __global__ void __launch_bounds__(256)
     k_m2l64(int j0, int nc, int P, int list4_mode, const double *tab, const int *l2,
             const uint8_t *n2, const int *l4, const uint8_t *n4, const double *c_cx,
@@ -332,19 +332,8 @@ __global__ void __launch_bounds__(256)
             acc = cadd(acc, cadd(sw, cmul(ld(ak, b), clog(cd{cx - c_cx[sidx], cy - c_cy[sidx]}))));
             continue;
         }
-        cd s;
-        if constexpr (PT > 0) {
-            cd a[PT + 1];
-#pragma unroll
-            for (int k = 0; k <= PT; ++k) a[k] = k <= P ? ld(ak, b + k) : cd{0.0, 0.0};
-            s = cscale(a[PT], PT <= P ? row[PT] : 0.0);
-#pragma unroll
-            for (int k = PT - 1; k >= 0; --k)
-                if (k <= P) s = cadd(cmul(s, w), cscale(a[k], row[k]));
-        } else {
-            s = cscale(ld(ak, b + P), row[P]);
-            for (int k = P - 1; k >= 0; --k) s = cadd(cmul(s, w), cscale(ld(ak, b + k), row[k]));
-        }
+        cd s = cscale(ld(ak, b + P), row[P]);
+        for (int k = P - 1; k >= 0; --k) s = cadd(cmul(s, w), cscale(ld(ak, b + k), row[k]));
         acc = cadd(acc, cmul(s, cpowi(w, p)));
     }
     if (list4_mode == 2) {
@@ -368,21 +357,20 @@ __global__ void __launch_bounds__(256)
 
 // M2L by one wavefront per target cell, for orders P <= 16 (the same sums as
 // k_m2l64).  The wave stages its M2L sources' coefficients a_k and
-// w = 1/(zs - zt) in LDS once (the list-2 entries, then the list-4 ones
-// with list4_mode 1); lane l = g NP + i (NP = P orders, P + 1 for the
-// potential) forms order p = i (+1 without the potential) over the sources
-// u = g, g + G, ... (G = 64 / NP groups), and the groups' partial sums are
-// added in group order.  Every lane works, and a source's coefficients are
-// read from HBM / L2 once per target instead of once per (target, order).
-// P2L (list4_mode 2) splits the list-4 particles over the groups the same way.
-// With L4ONLY the wave takes list 4 alone (M2L or P2L by list4_mode), skips a
-// cell without one and adds its sum to b_p, which the matrix-core list-2
-// kernel has written.
+// w = 1/(zs - zt) in LDS once; lane l = g NP + i (NP orders per cell) forms order
+// p = i (+1 for the field) over the sources u = g, g + G, ... (G = 64 / NP
+// groups), and the groups' partial sums are added in group order.  Every lane
+// works, and a source's coefficients are read from HBM / L2 once per target
+// instead of once per (target, order).
+// POT, the potential: lists 2 and 4 (orders 0 .. P).  The field (orders 1 .. P)
+// takes list 4 alone, skips a cell without one and adds its sum to b_p, which the
+// matrix-core list-2 kernel has written.  List 4 by M2L (list4_mode 1) or P2L (2),
+// whose particles the groups split the same way.
 constexpr int kM2lwWaves = 4;
 constexpr int kM2lwSrc = 27 + 8;  // list 2 <= 27, list 4 <= 8
-constexpr int kM2lwP1 = 17;       // orders up to 16
+constexpr int kM2lwP1 = kTrP1;    // orders up to 16
 
-template <bool POT, bool L4ONLY>
+template <bool POT>
 __global__ void __launch_bounds__(kWave *kM2lwWaves)
     k_m2l64w(int j0, int nc, int P, int list4_mode, const double *tab, const int *l2,
              const uint8_t *n2, const int *l4, const uint8_t *n4, const double *c_cx,
@@ -391,7 +379,7 @@ __global__ void __launch_bounds__(kWave *kM2lwWaves)
              const double2 *ak, double2 *bk) {
     // sources staged per wavefront: lists 2 and 4, or list 4 alone (a
     // smaller LDS footprint, so more wavefronts reside)
-    constexpr int NS = L4ONLY ? 8 : kM2lwSrc;
+    constexpr int NS = POT ? kM2lwSrc : 8;
     __shared__ double2 sak[kM2lwWaves][NS * kM2lwP1];
     __shared__ double2 sw[kM2lwWaves][NS], slg[kM2lwWaves][NS];
     __shared__ double2 red[kM2lwWaves][kWave];
@@ -401,8 +389,8 @@ __global__ void __launch_bounds__(kWave *kM2lwWaves)
     const int P1 = P + 1, NP = POT ? P1 : P, G = kWave / NP;
     const int g = lane / NP, i = lane % NP, p = (POT ? 0 : 1) + i;
     const double cx = c_cx[j], cy = c_cy[j];
-    const int m2 = L4ONLY ? 0 : n2[j], m4 = n4[j];
-    if (L4ONLY && m4 == 0) return;  // uniform over the wavefront
+    const int m2 = POT ? n2[j] : 0, m4 = n4[j];
+    if (!POT && m4 == 0) return;  // uniform over the wavefront
     const int ns = m2 + (list4_mode == 1 ? m4 : 0);
     // staging: w and (potential) log(z_t - z_s) per source, then the a_k rows
     if (lane < ns) {
@@ -466,7 +454,7 @@ __global__ void __launch_bounds__(kWave *kM2lwWaves)
         cd sum = {0.0, 0.0};
         for (int gg = 0; gg < G; ++gg) sum = cadd(sum, ld(red[w], gg * NP + lane));
         const size_t o = (size_t)j * P1 + (POT ? 0 : 1) + lane;
-        st(bk, o, L4ONLY ? cadd(ld(bk, o), sum) : sum);
+        st(bk, o, POT ? sum : cadd(ld(bk, o), sum));
     }
 }
 
@@ -1531,7 +1519,7 @@ __global__ void __launch_bounds__(kWave *kP2lT1Waves)
 }
 
 // Type-1 L2L for the cells of one level (>= 3; level-1 locals are zero), thread
-// per (cell, l): orders ND above 15.
+// per (cell, l): orders ND above 16.
 __global__ void __launch_bounds__(256)
     k_l2l_t1(int j0, int j1, int ND, const double *coef, const int *expo, const int *c_parent,
              const double *c_cx, const double *c_cy, double2 *bk) {
@@ -1706,23 +1694,21 @@ void fmm64_run(Ctx &c, int P, int list4_mode, int stage_mask, double *out_a, dou
     // M2L: every cell of level >= 2
     const int j2 = (int)ti.lev_off[2];
     const int NP = potential ? P1 : P;  // orders formed per cell
-    const double *t_r64 = (const double *)c.tab_r64.p;
-    if (nc > j2 && P >= 1 && P < kM2lwP1 && !potential && t_r64 && c.tab_r64_p == P) {
-        // list 2 on the matrix cores, then list 4 added by the wavefront kernel
-        const int *l2 = (const int *)c.l2.p;
-        const uint8_t *n2 = (const uint8_t *)c.n2.p;
-        m2l64_run<false>(c, P, t_r64, ak, bk, s);
-        k_m2l64w<false, true><<<div_up(nc - j2, kM2lwWaves), kWave * kM2lwWaves, 0, s>>>(
-            j2, nc, P, list4_mode, t_m2l, l2, n2, (const int *)c.l4.p,
-            (const uint8_t *)c.n4.p, c_cx, c_cy, c_begin, c_end, xs, ys, qs, as, ak, bk);
-    } else if (nc > j2 && P < kM2lwP1)
-        (potential ? k_m2l64w<true, false> : k_m2l64w<false, false>)<<<
-            div_up(nc - j2, kM2lwWaves), kWave * kM2lwWaves, 0, s>>>(
-            j2, nc, P, list4_mode, t_m2l, (const int *)c.l2.p, (const uint8_t *)c.n2.p,
-            (const int *)c.l4.p, (const uint8_t *)c.n4.p, c_cx, c_cy, c_begin, c_end, xs, ys, qs,
+    if (nc > j2 && P < kTrP1) {
+        const int *l2 = (const int *)c.l2.p, *l4 = (const int *)c.l4.p;
+        const uint8_t *n2 = (const uint8_t *)c.n2.p, *n4 = (const uint8_t *)c.n4.p;
+        if (!potential) {
+            // list 2 on the matrix cores, then list 4 added by the wavefront kernel
+            if (c.tab_r64_p != P) throw Error(kInternal, "M2L matrices of another order");
+            m2l64_run<false>(c, P, (const double *)c.tab_r64.p, ak, bk, s);
+        }
+        (potential ? k_m2l64w<true> : k_m2l64w<false>)<<<div_up(nc - j2, kM2lwWaves),
+                                                         kWave * kM2lwWaves, 0, s>>>(
+            j2, nc, P, list4_mode, t_m2l, l2, n2, l4, n4, c_cx, c_cy, c_begin, c_end, xs, ys, qs,
             as, ak, bk);
-    else if (nc > j2)
-        (potential ? k_m2l64<true, 0> : k_m2l64<false, 0>)<<<
+    }
+    if (nc > j2 && P >= kTrP1)
+        (potential ? k_m2l64<true> : k_m2l64<false>)<<<
             div_up((long long)(nc - j2) * NP, 256), 256, 0, s>>>(
             j2, nc, P, list4_mode, t_m2l, (const int *)c.l2.p, (const uint8_t *)c.n2.p,
             (const int *)c.l4.p, (const uint8_t *)c.n4.p, c_cx, c_cy, c_begin, c_end, xs, ys, qs,
