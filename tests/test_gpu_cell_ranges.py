@@ -10,15 +10,17 @@ from lsmps_vpm_v2_amd import FmmSolver, workloads as W
 pytestmark = pytest.mark.gpu
 
 
-# 8192 cells lie between the first and the second of each pair
-@pytest.mark.parametrize("n,cap", [(2000, 1), (60000, 6), (30000, 15), (300000, 15), (60000, 17),
-                                   (250000, 63), (900000, 64), (1200000, 129), (2, 1)])
-def test_ranges_add_up(gpu, n, cap):
+@pytest.mark.parametrize("n,cap,many", [
+    (2, 1, False), (2000, 1, False), (30000, 15, False), (150000, 63, False), (150000, 64, False),
+    (300000, 129, False), (60000, 6, True), (60000, 17, True), (300000, 15, True),
+    (250000, 63, True), (900000, 64, True), (1200000, 129, True)])
+def test_ranges_add_up(gpu, n, cap, many):
     f = W.random_clusters(n, seed=cap, active_frac=0.9)
     s = FmmSolver(max_par=cap, max_src=cap)
     print(f"ranges n={n} max_par={cap}", flush=True)
     s.field(f["x"], f["y"], f["q"], f["active"])
     c = s.tree_cells()
+    assert (len(c["id"]) > 8192) == many
     lid, poff, pidx = s.tree_leaves(n)
     assert np.array_equal(np.sort(pidx), np.arange(n))
     leaf = c["is_leaf"] != 0

@@ -6,7 +6,7 @@ parity tests (the same FP64 sums in another order; measured under 1e-14)."""
 import numpy as np
 import pytest
 
-from lsmps_vpm_v2_amd import FmmSolver, workloads as W
+from lsmps_vpm_v2_amd import FmmSolver, VpmFmmError, workloads as W
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-10
@@ -16,6 +16,7 @@ def _rel(a, b):
     return float(np.linalg.norm(np.asarray(a) - np.asarray(b)) / np.linalg.norm(b))
 
 
+MANY = 8192  # leaves up to which four wavefronts share one
 CASES = [(7, 4), (700, 7), (700, 8), (700, 9), (900, 16), (900, 17), (1500, 32), (1500, 33),
          (3000, 64), (3000, 65), (3000, 130), (4000, 300), (60001, 8)]
 
@@ -27,7 +28,9 @@ def test_groups_match_oracle(gpu, oracle, n, cap):
     kw = dict(max_par=cap, max_src=cap)
     a = [f[k] for k in ("x", "y", "s", "omega", "active")]
     for icut in (0, 1, 2, 3):
-        u, v = FmmSolver(icutoff=icut, u_inf=0.0, **kw).velocity(*a)
+        solver = FmmSolver(icutoff=icut, u_inf=0.0, **kw)
+        u, v = solver.velocity(*a)
+        assert (solver.stats()["n_leaves"] > MANY) == (n > 60000)
         u0, v0 = oracle.velocity(*a, oracle.opts(icutoff=icut, **kw), 0.0, 0.0)
         assert _rel(np.hypot(u - u0, v - v0) + np.hypot(u0, v0), np.hypot(u0, v0)) <= TOL
     b = [f[k] for k in ("x", "y", "q", "active")]
@@ -42,12 +45,35 @@ def test_strength_that_is_not_finite_is_no_duplicate(gpu, n):
     f = W.random_clusters(n, seed=3)
     w = f["omega"].copy()
     w[n // 3] = np.nan
-    # one tree level, so that everything is near field
+    # one tree level, so that everything is near field, or many small leaves
+    cap = 4096 if n < 4096 else 8
     for icut in (0, 2):
-        s = FmmSolver(max_par=4096, max_src=4096, icutoff=icut) if n < 4096 else FmmSolver(icutoff=icut)
+        s = FmmSolver(max_par=cap, max_src=cap, icutoff=icut)
         u, v = s.velocity(f["x"], f["y"], f["s"], w, f["active"])
+        assert (s.stats()["n_leaves"] > MANY) == (n > 60000)
         bad = np.isnan(u)
         assert bad.any() and not bad[n // 3]
+
+
+@pytest.mark.parametrize("n", [3000, 60001])
+@pytest.mark.parametrize("strengths", ["both", "one", "none", "opposite"])
+def test_duplicates_are_found(gpu, n, strengths):
+    """Two particles at one point, whatever their strengths: the error and not a
+    NaN, from the field and the potential; apart, neither."""
+    f = W.random_clusters(n, seed=3)
+    x, y, q = f["x"].copy(), f["y"].copy(), f["q"].copy()
+    i, k = n // 3, n // 2
+    x[k], y[k] = x[i], y[i]
+    q[i], q[k] = dict(both=(1.0, 2.0), one=(0.0, 1.0), none=(0.0, 0.0),
+                      opposite=(1.0, -1.0))[strengths]
+    s = FmmSolver(max_par=8, max_src=8)
+    print(f"duplicates n={n} {strengths}", flush=True)
+    for call in (s.field, s.potential):
+        with pytest.raises(VpmFmmError) as e:
+            call(x, y, q, f["active"])
+        assert e.value.status == "DUPLICATE_POINTS"
+        assert np.isfinite(call(f["x"], f["y"], q, f["active"])).all()
+        assert (s.stats()["n_leaves"] > MANY) == (n > 60000)
 
 
 def test_sizes_of_zero(gpu, oracle):

@@ -28,9 +28,17 @@ def _field(kind, n):
     return x, y, np.full(n, 1e-4), rng.standard_normal(n), np.ones(n, np.uint8)
 
 
-def _check(oracle, f, **kw):
+def _workgroups(solver):
+    """96 cells of a level each; from 65 on a workgroup takes all four classes."""
+    level = solver.tree_cells()["level"]
+    return sum(-(-int(np.sum(level == k)) // 96) for k in range(2, 17))
+
+
+def _check(oracle, f, many, **kw):
     print(f"classes n={len(f[0])} {kw}", flush=True)
-    u, v = FmmSolver(**kw).velocity(*f)
+    solver = FmmSolver(**kw)
+    u, v = solver.velocity(*f)
+    assert (_workgroups(solver) > 64) == many
     u0, v0 = oracle.velocity(*f, oracle.opts(**kw), 1.0, 0.0)
     assert _rel(u, u0) <= TOL and _rel(v, v0) <= TOL
 
@@ -38,13 +46,13 @@ def _check(oracle, f, **kw):
 @pytest.mark.parametrize("kind", ["grid", "line", "diagonal"])
 @pytest.mark.parametrize("p", range(1, 17))
 def test_orders_match_oracle(gpu, oracle, kind, p):
-    _check(oracle, _field(kind, 3000), p=p, max_par=2, max_src=2, max_level=12)
+    _check(oracle, _field(kind, 3000), False, p=p, max_par=2, max_src=2, max_level=12)
 
 
 @pytest.mark.parametrize("kind", ["grid", "line", "diagonal"])
 @pytest.mark.parametrize("p", [3, 10, 12, 13, 16])
 def test_larger_trees_match_oracle(gpu, oracle, kind, p):
-    _check(oracle, _field(kind, 12000), p=p, max_par=2, max_src=2, max_level=14)
+    _check(oracle, _field(kind, 12000), True, p=p, max_par=2, max_src=2, max_level=14)
 
 
 @pytest.mark.parametrize("kind,n", [("grid", 3000), ("line", 3000), ("grid", 12000)])
@@ -53,6 +61,8 @@ def test_type1_orders_match_oracle(gpu, oracle, kind, n, ndp):
     x, y, s, g, _ = _field(kind, n)
     kw = dict(n_s=2, lmax=10, ndp=ndp, icutoff=2, l2l_mode=0)
     print(f"classes type 1 {kind} n={n} {kw}", flush=True)
-    u, v = FmmSolver(u_inf=0.0, v_inf=0.0).velocity_type1(x, y, s, g, **kw)
+    solver = FmmSolver(u_inf=0.0, v_inf=0.0)
+    u, v = solver.velocity_type1(x, y, s, g, **kw)
+    assert (_workgroups(solver) > 64) == (n > 3000)
     u0, v0 = oracle.t1_velocity(x, y, s, g, oracle.t1_opts(**kw))
     assert _rel(u, u0) <= TOL and _rel(v, v0) <= TOL
