@@ -787,7 +787,6 @@ struct EvalArgs {
     const int *l1;
     const uint32_t *off3;
     const int *l3;
-    uint32_t cap1, cap3;  // entries of l1 and l3
     const float2 *oxy;
     const float *qf;
     const double *ss;  // sorted sizes (regularized near field only)
@@ -812,9 +811,7 @@ __device__ __forceinline__ void eval_leaf(const EvalArgs &A, int t, int lane, fl
     const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)A.c_end[j]);
     const double tcx = A.c_cx[j], tcy = A.c_cy[j];
     const bool own_src = (A.c_flags[j] & kActive) != 0;  // the leaf is in its own list 1
-    // (within the capacities: tree_lists_end)
-    const uint32_t a1 = min(A.off1[t], A.cap1), z1 = min(A.off1[t + 1], A.cap1);
-    const uint32_t a3 = min(A.off3[t], A.cap3), z3 = min(A.off3[t + 1], A.cap3);
+    const uint32_t a1 = A.off1[t], z1 = A.off1[t + 1], a3 = A.off3[t], z3 = A.off3[t + 1];
     const int L = A.c_level[j];
     const int p = A.lt->p[L];
     const float inv_s = A.lt->inv_s[L];
@@ -1234,7 +1231,7 @@ void fmm32_rest(Ctx &c, const Mixed32 &mx, int list4_mode, int stage_mask, doubl
     mk.mark(5, s);
     EvalArgs ea{leaf_idx, c_level, c_flags, c_begin, c_end, c_cx, c_cy,
                 (const uint32_t *)c.off1.p, (const int *)c.l1.p, (const uint32_t *)c.off3.p,
-                (const int *)c.l3.p, (uint32_t)ti.cap1, (uint32_t)ti.cap3, oxy, qf, (const double *)c.ss.p, c.perm_sorted, mx.lt,
+                (const int *)c.l3.p, oxy, qf, (const double *)c.ss.p, c.perm_sorted, mx.lt,
                 ahat, bhat, kst, stage_mask, velocity ? 1 : 0, u_inf, v_inf, out_a, out_b,
                 &c.hdr_d->flags};
     const int nb = div_up(nl, kEvalWaves), nth = kWave * kEvalWaves;

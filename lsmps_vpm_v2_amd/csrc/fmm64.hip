@@ -1055,7 +1055,6 @@ struct Eval64Args {
     const int *l1;
     const uint32_t *off3;
     const int *l3;
-    uint32_t cap1, cap3;  // entries of l1 and l3
     const double *xs, *ys, *qs, *ss;
     const uint32_t *perm;
     const double2 *ak, *bk;
@@ -1161,9 +1160,7 @@ __device__ __forceinline__ bool eval64_leaf(const Eval64Args &A, int t, int j, i
     const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)A.c_end[j]);
     const bool own = (A.c_flags[j] & kActive) != 0;  // the leaf is in its own list 1
     const double lcx = A.c_cx[j], lcy = A.c_cy[j];
-    // (within the capacities: tree_lists_end)
-    const uint32_t a1 = min(A.off1[t], A.cap1), z1 = min(A.off1[t + 1], A.cap1);
-    const uint32_t a3 = min(A.off3[t], A.cap3), z3 = min(A.off3[t + 1], A.cap3);
+    const uint32_t a1 = A.off1[t], z1 = A.off1[t + 1], a3 = A.off3[t], z3 = A.off3[t + 1];
     // padding source: zero strength, outside the root box, of a size at which any
     // target's factor is finite (a zero size would leave 0 NaN)
     const double padx = lcx + 4.0 * A.hdr->root_len;
@@ -1391,7 +1388,7 @@ __global__ void __launch_bounds__(kWave *kEvalWaves)
             bool dup = false;
             const uint32_t b = A.c_begin[j], e = A.c_end[j];
             for (uint32_t i = b + lane; i < e; i += kWave)
-                for (uint32_t u = A.off1[t], z = min(A.off1[t + 1], A.cap1); u < z; ++u) {
+                for (uint32_t u = A.off1[t]; u < A.off1[t + 1]; ++u) {
                     const int c = A.l1[u];
                     for (uint32_t r = A.c_begin[c]; r < A.c_end[c]; ++r) {
                         const double dx = A.xs[i] - A.xs[r], dy = A.ys[i] - A.ys[r];
@@ -1586,8 +1583,6 @@ static Eval64Args eval64_args(const Ctx &c, int P, bool velocity, double u_inf, 
     A.l1 = (const int *)c.l1.p;
     A.off3 = (const uint32_t *)c.off3.p;
     A.l3 = (const int *)c.l3.p;
-    A.cap1 = (uint32_t)c.info.cap1;
-    A.cap3 = (uint32_t)c.info.cap3;
     A.xs = (const double *)c.xs.p;
     A.ys = (const double *)c.ys.p;
     A.qs = (const double *)c.qs.p;

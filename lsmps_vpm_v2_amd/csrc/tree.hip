@@ -1050,7 +1050,7 @@ __global__ void __launch_bounds__(256)
                  const double *c_cx, const double *c_cy, const int *c_child, const int *nbr,
                  const double4 *bnd, const DevHdr *hdr, const uint8_t *orders, uint32_t *cnt1,
                  uint32_t *cnt3,
-                 uint2 *cntk, const uint32_t *off1, const uint32_t *off3, int *l1, int *l3,
+                 uint2 *cntk, uint32_t *off1, uint32_t *off3, int *l1, int *l3,
                  uint32_t cap1, uint32_t cap3, uint32_t *bs1, uint32_t *bs3,
                  const uint32_t *c_begin, const uint32_t *c_end, DevHdr *hdr_w) {
 #pragma clang fp contract(off)
@@ -1191,6 +1191,14 @@ __global__ void __launch_bounds__(256)
         my_m2p = (unsigned long long)n3 * nt;
         my_m2p_terms = m2p_w * nt;
         if (k == 4) my_l2p_terms = (unsigned long long)orders[L] * nt;
+    }
+    if (FILL && leaf_live && k == 0) {  // (o1, o3: the leaf's own offsets)
+        if (o1 > cap1) off1[t] = cap1;
+        if (o3 > cap3) off3[t] = cap3;
+        if (t == nl - 1) {
+            off1[nl] = min(off1[nl], cap1);
+            off3[nl] = min(off3[nl], cap3);
+        }
     }
     if (overflow) atomicOr(&hdr_w->flags, kFlagListOverflow);
     if (FILL) {
@@ -1462,8 +1470,8 @@ void tree_lists_end(Ctx &c) {
     // list 3 of leaves coarser than it and adjacent to its parent: at most 8,
     // so sum |list 3| <= 8 nc.  That holds while the cells are larger than the
     // tolerance kListEps; where they are not, a leaf is adjacent to everything below
-    // its neighbours.  So the fill pass checks both, the readers stop at the
-    // capacities (their results are then dropped), and tree_lists_absorb refuses.
+    // its neighbours.  So the fill pass stops at both, and cuts the offsets there for
+    // the kernels that read the lists before tree_lists_absorb refuses the call.
     ti.cap1 = 17 * (size_t)nl + 1;
     ti.cap3 = 8 * (size_t)nc + 1;
     int *l1 = c.l1.as<int>(ti.cap1), *l3 = c.l3.as<int>(ti.cap3);
