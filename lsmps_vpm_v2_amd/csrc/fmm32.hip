@@ -1104,19 +1104,24 @@ int mixed_level_setup(Ctx &c, const uint8_t *orders, LevelTab *lt, int2 *tiles,
 
 // Split levels of the three-tier passes: K = first level with >= kSubRoots
 // cells (subtrees below), T = first level with >= kTopCells cells (one
-// workgroup above T).  Trees of more than kSubCells cells have no subtrees: a
-// subtree's few wavefronts take its cells in turn, which costs more there than a
-// launch per level (8 M particles, 345k cells: M2M and L2L 218 + 127 us in
-// subtrees, the solve 2665 us, 2613 without; 2 M, 43k cells: 896 and 902).
-constexpr int kSubCells = 1 << 16;
+// workgroup above T).  Trees deeper than kSubDepth levels below K have no subtrees:
+// a subtree's few wavefronts take its cells in turn, the pass waits for the
+// largest, and it holds up to 85 cells at three levels but 341 at four, 1300 where a
+// field crowds around a body, whatever the mean.  (Solves at leaf threshold 48, with
+// subtrees and with a launch per level: three levels, 500k and 1.5M vortices 313 and
+// 335, 499 and 525 us, 780k plate 498 and 528; four, clusters of 250k 397 and 397,
+// of 500k 501 and 472; five, of 1M 785 and 687; seven, the wake of 500k 691 and 470,
+// of 4M 1921 and 1809.)
+constexpr int kSubDepth = 3;
 static void tier_levels(const TreeInfo &ti, int &K, int &T) {
     const int maxL = ti.max_level;
     K = T = maxL;
     for (int L = maxL; L >= 1; --L) {
         const int cnt = (int)(ti.lev_off[L + 1] - ti.lev_off[L]);
-        if (cnt >= kSubRoots && ti.n_cells <= kSubCells) K = L;
+        if (cnt >= kSubRoots) K = L;
         if (cnt >= kTopCells) T = L;
     }
+    if (maxL - K > kSubDepth) K = maxL;
     T = std::min(T, K);
 }
 

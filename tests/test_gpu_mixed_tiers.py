@@ -1,5 +1,5 @@
-"""The mixed upward and downward passes on both sides of the cell count up to
-which subtrees are walked by a workgroup, against the FP64 path (held to the
+"""The mixed upward and downward passes on both sides of the depth (three levels
+below the first one of 1024 cells) up to which subtrees are walked by a workgroup, against the FP64 path (held to the
 oracle by its own tests) on a jittered lattice, even or graded towards its middle
 (subtrees of very different size): FP32 rounding of the pairs, kept 0.4 spacings
 apart, and expansions, rel-L2 <= 5e-6 as the other mixed tests."""
@@ -11,10 +11,11 @@ from lsmps_vpm_v2_amd import FmmSolver
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,many", [(200, False), (500, True)])
+@pytest.mark.parametrize("m,graded,deep", [(200, False, False), (300, False, False),
+                                           (500, False, True), (200, True, True),
+                                           (500, True, True)])
 @pytest.mark.parametrize("p", [3, 8, 16])
-@pytest.mark.parametrize("graded", [False, True])
-def test_tiers_match_fp64(gpu, m, many, p, graded):
+def test_tiers_match_fp64(gpu, m, graded, deep, p):
     rng = np.random.default_rng(m)
     g = (np.stack(np.divmod(np.arange(m * m), m)) + 0.5 + 0.6 * (rng.random((2, m * m)) - 0.5)) / m
     if graded:
@@ -24,7 +25,8 @@ def test_tiers_match_fp64(gpu, m, many, p, graded):
     print(f"tiers m={m} p={p} graded={graded}", flush=True)
     s = FmmSolver(precision="mixed", **kw)
     ex, ey = s.field(g[0], g[1], q, act)
-    assert (s.stats()["n_cells"] > 65536) == many
+    cells = np.bincount(s.tree_cells()["level"])
+    assert (len(cells) - 1 - np.argmax(cells >= 1024) > 3) == deep
     ex0, ey0 = FmmSolver(**kw).field(g[0], g[1], q, act)
     err = np.sqrt(np.sum((ex - ex0) ** 2 + (ey - ey0) ** 2) / np.sum(ex0 ** 2 + ey0 ** 2))
     print(f"  {err:.2e}")
