@@ -859,7 +859,7 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
 // lane out), and every wavefront step is 64 terms, of which the mask keeps
 // those whose target takes this cell.
 //
-// The kernel is bound by vector-ALU issue in FP64 (0.7 of the cycles), so what
+// The kernel is bound by vector-ALU issue in FP64 (0.83 of the cycles), so what
 // counts is the share of a step's 64 lane slots that hold a wanted term.  One
 // lane per target, one cell or source at a time for 64 targets, used 0.53
 // (far) and 0.30 (near) of them: the far cells and near leaves of 64

@@ -489,10 +489,11 @@ __global__ void __launch_bounds__(kWave *kM2lwWaves)
 // hash table and staged in LDS once, scaled; a matrix is read once per 32
 // targets, the next one's loads under way while this one's products run, and a
 // half of the 32 without a source at the offset takes no products: 81 us, now
-// bound by the products (14 offsets a wavefront) and, a quarter, by the lists'
-// and rows' dependent loads.  Type 1 at 200k: one thread per order and cell 121
-// us, 34 us.  (96 cells and not 128: where some children are missing a class
-// would exceed its 32 targets and need a second round.)
+// bound by the products (14 offsets a wavefront; the matrix cores are busy on 0.33
+// of the cycles) and, a quarter, by the lists' and rows' dependent loads.  Type 1
+// at 200k: one thread per order and cell 121 us, 37 us.  (96 cells and not 128:
+// where some children are missing a class would exceed its 32 targets and need a
+// second round.)
 //
 // NQ = 1: a workgroup takes one of the four classes, all its wavefronts the
 // class's offsets.  A tree of a few workgroups' cells leaves the chip idle
@@ -555,7 +556,10 @@ struct M2lShape {
     static constexpr int T4 = REM > 8 ? 0 : (REM + 3) / 4;   // 4-row tiles after them
     static constexpr int NS = T16 + T4;
     static constexpr int ACC = 4 * T16 + T4;                 // accumulators per lane and target set
-    // sets of 16 targets per wavefront: two while they fit 128 registers
+    // sets of 16 targets per wavefront: two up to order 12, where they need the 128
+    // registers and up to 72 bytes of scratch beside them (orders 8 to 12); a solve
+    // of a 200k plate takes 322, 335 and 350 us at orders 8, 10 and 12 and, with one
+    // set, 361 and 434 at 13 and 16
     static constexpr int U = P <= 12 ? 2 : 1;
     static constexpr bool AHEAD = KS * NS <= 12;             // and the next matrix too
 };
@@ -1019,7 +1023,7 @@ __device__ __forceinline__ double regul64(double rho2) {
 // targets, a group all of the leaf's (G by leaf size), and the groups and
 // wavefronts split the sources and list-3 cells and are reduced at the end.
 //
-// The kernel is bound by vector-ALU issue where leaves abound (0.74 of the
+// The kernel is bound by vector-ALU issue where leaves abound (0.76 of the
 // cycles on the 780k flat plate, half of them outside the pair loop, whose
 // leaves hold 16 targets) and by the latency of one leaf's chain where they
 // do not.  Two targets per lane halve the LDS reads per pair (24 B a source,
@@ -1622,7 +1626,8 @@ static void m2l64_run(const Ctx &c, int P, const double *R, const double2 *ak, d
     const uint8_t *n2 = (const uint8_t *)c.n2.p;
     const double2 *cres = (const double2 *)c.c_res.p;  // (type 1)
     // One class per workgroup while four times the workgroups still fit the
-    // chip's 256 CUs at once (k_m2l64_mfma's comment has both sides).
+    // chip's 256 CUs at once (k_m2l64_mfma's comment has both sides).  From there
+    // to 255 workgroups some CUs have none: 177 of 256 at 780k.
     constexpr int split = 64;
     switch (P) {
 #define M2L64_CASE(PP)                                                                          \
